@@ -222,8 +222,8 @@ int lard_attn_kl_backward(const lard_tensor4* qs, const lard_tensor4* ks, const 
  */
 /* Workspace needed by lard_attn_kl_forward_rowgrad (bytes): the forward's,
  * plus both sides' keys as float16 ([B, kv_heads, T, D] student,
- * [B, kv_heads_t, T, D] teacher; bfloat16 inputs are converted) and four
- * scalars. */
+ * [B, kv_heads_t, T, D] teacher; bfloat16 inputs are converted), the scratch
+ * of their maxima and their scales. */
 size_t lard_attn_kl_forward_rowgrad_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads,
                                                     int64_t kv_heads_t, int64_t seq_len, int64_t head_dim);
 

@@ -247,13 +247,18 @@ class Carver {
 struct LossWs {
   float* rows;
   double* partial;
+  unsigned* counter;  // ticket of the reduction
 };
+
+constexpr int kLossPartials = 512;
 
 LossWs loss_layout(void* base, int64_t n, size_t* bytes) {
   Carver c(base);
   LossWs w;
   w.rows = c.take<float>(n);
-  w.partial = c.take<double>(lard::kReduceBlocks);
+  w.partial = c.take<double>(kLossPartials);
+  static_assert(lard::kReduceBlocks < kLossPartials, "the last partial's slot holds the ticket counter");
+  w.counter = reinterpret_cast<unsigned*>(w.partial + (kLossPartials - 1));
   if (bytes != nullptr) *bytes = c.bytes();
   return w;
 }
@@ -284,14 +289,14 @@ FwdWs fwd_layout(void* base, int64_t B, int64_t H, int64_t T, size_t* bytes) {
 // scaled by.
 struct KeysF16 {
   lard::u16* k16;
-  unsigned* maxbits;
+  unsigned* maxima;
   float* scale;
 };
 
 KeysF16 take_keys(Carver& c, int64_t B, int64_t Hkv, int64_t T, int64_t D) {
   KeysF16 k;
   k.k16 = c.take<lard::u16>(B * Hkv * T * D);
-  k.maxbits = c.take<unsigned>(1);
+  k.maxima = c.take<unsigned>(lard::kKeyMaxima);
   k.scale = c.take<float>(1);
   return k;
 }
@@ -314,8 +319,9 @@ RowgradWs rowgrad_layout(void* base, int64_t B, int64_t Hq, int64_t Hkv_s, int64
 }
 
 // Both sides' float16 keys for the fused row-gradient forward: scaled copies
-// for bfloat16 inputs, the tensors themselves for float16 ones.
-hipError_t keys_f16(lard::HotArgs& f, bool bf, const KeysF16& ks, const KeysF16& kt, hipStream_t st) {
+// for bfloat16 inputs (appended to `sides`, for the launch that makes them),
+// the tensors themselves for float16 ones.
+void keys_f16(lard::HotArgs& f, bool bf, const KeysF16& ks, const KeysF16& kt, lard::KeySide* sides, int* n) {
   if (!bf) {
     f.k16 = f.r.s.k;
     f.k16_sb = f.r.s.k_sb;
@@ -327,7 +333,7 @@ hipError_t keys_f16(lard::HotArgs& f, bool bf, const KeysF16& ks, const KeysF16&
     f.k16t_sh = f.r.t.k_sh;
     f.k16t_st = f.r.t.k_st;
     f.k16t_scale = nullptr;
-    return hipSuccess;
+    return;
   }
   const int64_t D = f.r.s.dim, T = f.r.T;
   f.k16 = ks.k16;
@@ -340,9 +346,17 @@ hipError_t keys_f16(lard::HotArgs& f, bool bf, const KeysF16& ks, const KeysF16&
   f.k16t_sh = T * D;
   f.k16t_sb = (int64_t)f.r.t.hkv * T * D;
   f.k16t_scale = kt.scale;
-  hipError_t e = lard::launch_keys_f16(f.r.s, f.r.B, f.r.Hq, f.r.T, ks.maxbits, ks.scale, ks.k16, st);
-  if (e != hipSuccess) return e;
-  return lard::launch_keys_f16(f.r.t, f.r.B, f.r.Hq, f.r.T, kt.maxbits, kt.scale, kt.k16, st);
+  sides[(*n)++] = lard::key_side(f.r.s, f.r.B, f.r.Hq, ks.maxima, ks.scale, ks.k16);
+  sides[(*n)++] = lard::key_side(f.r.t, f.r.B, f.r.Hq, kt.maxima, kt.scale, kt.k16);
+}
+
+// The pre-passes of a fused forward: the token pass (tok != null) and the
+// float16 keys of n sides.
+int launch_forward_prep(const lard::TokenPrep* tok, const lard::KeySide* sides, int n, int B, int T, int D,
+                        hipStream_t st) {
+  if (n > 0) return hip_status(lard::launch_keys_f16(sides, n, tok, B, T, D, st), "forward_rowgrad prep launch");
+  if (tok != nullptr) return hip_status(lard::launch_token_prep(*tok, B, st), "forward_rowgrad token prep launch");
+  return LARD_OK;
 }
 
 // Backward of the autograd path: token validity, the first two valid tokens
@@ -494,6 +508,12 @@ lard::HotArgs relation_args(const lard_relation& R, const lard_mask* mask, int c
   f.tok_ok = tok_ok;
   f.first2 = first2;
   return f;
+}
+
+
+// The row normalisers' pre-pass of one relation of a batched backward.
+lard::RowPrep row_prep(const lard::HotArgs& f) {
+  return {f.r.lse_s_in, f.r.lse_t_in, const_cast<float*>(f.nl_s), const_cast<float*>(f.nl_t), f.r.Hq};
 }
 
 
@@ -667,12 +687,13 @@ int lard_kl_forward(const lard_tensor4* qs, const lard_tensor4* ks, const float*
     a.lse_t_in = lse_t;
     const LossWs w = loss_layout(workspace, n, nullptr);
     a.row_out = w.rows;
+    a.counter = w.counter;
     if ((rc = hip_status(lard::launch_row_kl(a, padded_dim(qs->size[3]), padded_dim(qt->size[3]), st),
                          "kl_forward launch")) != LARD_OK)
       return rc;
-    return hip_status(lard::launch_reduce_sum(w.rows, n, w.partial, loss_out, st), "kl_forward reduce launch");
+    return hip_status(lard::launch_reduce_sum(w.rows, n, w.partial, w.counter, loss_out, st), "kl_forward reduce launch");
   }
-  return hip_status(lard::launch_reduce_sum(nullptr, 0, nullptr, loss_out, st), "kl_forward reduce launch");
+  return hip_status(lard::launch_reduce_sum(nullptr, 0, nullptr, nullptr, loss_out, st), "kl_forward reduce launch");
 }
 
 int lard_kl_backward(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s, const lard_tensor4* qt,
@@ -759,14 +780,16 @@ int attn_kl_forward_impl(const lard_tensor4* qs, const lard_tensor4* ks, const l
         f.Tp = (int)padded_len(T);
         f.tok_ok = w.tok_ok;
         f.first2 = w.first2;
-        if ((rc = hip_status(lard::launch_token_prep(f.r, f.Tp, w.tok_ok, w.first2, st),
-                             "attn_kl_forward token prep launch")) != LARD_OK)
+        if ((rc = hip_status(
+                 lard::launch_token_prep(lard::token_prep(f.r, f.Tp, w.tok_ok, w.first2, w.loss.counter), (int)B, st),
+                 "attn_kl_forward token prep launch")) != LARD_OK)
           return rc;
         rc = hip_status(timed(LARD_KERNEL_FORWARD, st, [&] { return lard::launch_hot_fwd(f, padded_dim(ds), bf, st); }),
                         "attn_kl_forward launch");
       } else {
         lard::FusedArgs g{};
         g.r = f.r;
+        g.r.counter = w.loss.counter;
         g.lse_s_out = lse_s_out;
         g.lse_t_out = lse_t_out;
         g.row_out = f.row_out;
@@ -783,6 +806,7 @@ int attn_kl_forward_impl(const lard_tensor4* qs, const lard_tensor4* ks, const l
       g.lse_s_out = lse_s_out;
       g.lse_t_out = lse_t_out;
       g.row_out = w.loss.rows;
+      g.r.counter = w.loss.counter;
       if ((rc = hip_status(timed(LARD_KERNEL_FORWARD, st, [&] { return lard::launch_fused_fwd_f32(g, st); }),
                            "attn_kl_forward float32 launch")) != LARD_OK)
         return rc;
@@ -797,14 +821,15 @@ int attn_kl_forward_impl(const lard_tensor4* qs, const lard_tensor4* ks, const l
       a.lse_s_in = lse_s_out;
       a.lse_t_in = lse_t_out;
       a.row_out = w.loss.rows;
+      a.counter = w.loss.counter;
       if ((rc = hip_status(lard::launch_row_kl(a, padded_dim(ds), padded_dim(dt), st), "attn_kl_forward kl launch")) !=
           LARD_OK)
         return rc;
     }
-    return hip_status(lard::launch_reduce_sum(w.loss.rows, n, w.loss.partial, loss_out, st),
+    return hip_status(lard::launch_reduce_sum(w.loss.rows, n, w.loss.partial, w.loss.counter, loss_out, st),
                       "attn_kl_forward reduce launch");
   }
-  return hip_status(lard::launch_reduce_sum(nullptr, 0, nullptr, loss_out, st), "attn_kl_forward reduce launch");
+  return hip_status(lard::launch_reduce_sum(nullptr, 0, nullptr, nullptr, loss_out, st), "attn_kl_forward reduce launch");
 }
 
 // ---- the library's own forward workspace (lard_attn_kl_forward_noalloc) ----
@@ -932,11 +957,12 @@ int lard_attn_kl_backward(const lard_tensor4* qs, const lard_tensor4* ks, const 
     if ((rc = check_blocks(B, Hq, T)) != LARD_OK) return rc;
     const int Tp = (int)padded_len(T);
     const BwdWs w = bwd_layout(workspace, B, Hq, T, nullptr);
-    if ((rc = hip_status(lard::launch_token_prep(a, Tp, w.tok_ok, w.first2, st),
+    if ((rc = hip_status(lard::launch_token_prep(lard::token_prep(a, Tp, w.tok_ok, w.first2, nullptr), (int)B, st),
                          "attn_kl_backward token prep launch")) != LARD_OK)
       return rc;
-    if ((rc = hip_status(lard::launch_row_prep(a, Tp, w.tok_ok, w.first2, w.nl_s, w.nl_t, st),
-                         "attn_kl_backward row prep launch")) != LARD_OK)
+    lard::RowPrepBatch rp = lard::row_prep_batch(a, Tp);
+    rp.rel[rp.n++] = {lse_s, lse_t, w.nl_s, w.nl_t, (int)Hq};
+    if ((rc = hip_status(lard::launch_row_prep(rp, (int)B, st), "attn_kl_backward row prep launch")) != LARD_OK)
       return rc;
     lard::HotArgs f{};
     f.r = a;
@@ -1013,7 +1039,7 @@ int lard_attn_kl_forward_rowgrad(const lard_tensor4* qs, const lard_tensor4* ks,
   const int64_t n = B * Hq * T;
   const hipStream_t st = static_cast<hipStream_t>(stream);
   if (n == 0)
-    return hip_status(lard::launch_reduce_sum(nullptr, 0, nullptr, loss_out, st), "attn_kl_forward reduce launch");
+    return hip_status(lard::launch_reduce_sum(nullptr, 0, nullptr, nullptr, loss_out, st), "attn_kl_forward reduce launch");
   if (lse_s_out == nullptr || lse_t_out == nullptr || dq_row_out == nullptr)
     return fail(LARD_ERR_INVALID_ARGUMENT, "lse and dq_row outputs must not be NULL");
   if (reinterpret_cast<uintptr_t>(dq_row_out) % 16 != 0)
@@ -1037,18 +1063,17 @@ int lard_attn_kl_forward_rowgrad(const lard_tensor4* qs, const lard_tensor4* ks,
   f.Tp = (int)padded_len(T);
   f.tok_ok = w.tok_ok;
   f.first2 = w.first2;
-  if ((rc = hip_status(lard::launch_token_prep(f.r, f.Tp, w.tok_ok, w.first2, st),
-                       "attn_kl_forward_rowgrad token prep launch")) != LARD_OK)
-    return rc;
   const bool bf = qs->dtype == LARD_DTYPE_BF16;
-  if ((rc = hip_status(keys_f16(f, bf, rw.s, rw.t, st),
-                       "attn_kl_forward_rowgrad float16 keys launch")) != LARD_OK)
-    return rc;
+  lard::KeySide sides[2];
+  int nsides = 0;
+  keys_f16(f, bf, rw.s, rw.t, sides, &nsides);
+  const lard::TokenPrep tok = lard::token_prep(f.r, f.Tp, w.tok_ok, w.first2, w.loss.counter);
+  if ((rc = launch_forward_prep(&tok, sides, nsides, (int)B, (int)T, (int)D, st)) != LARD_OK) return rc;
   if ((rc = hip_status(timed(LARD_KERNEL_FORWARD_ROWGRAD, st,
                              [&] { return lard::launch_hot_fwdq(f, padded_dim(qs->size[3]), bf, st); }),
                        "attn_kl_forward_rowgrad launch")) != LARD_OK)
     return rc;
-  return hip_status(lard::launch_reduce_sum(w.loss.rows, n, w.loss.partial, loss_out, st),
+  return hip_status(lard::launch_reduce_sum(w.loss.rows, n, w.loss.partial, w.loss.counter, loss_out, st),
                     "attn_kl_forward_rowgrad reduce launch");
 }
 
@@ -1085,11 +1110,9 @@ int lard_attn_kl_backward_colgrad(const lard_tensor4* qs, const lard_tensor4* ks
   fill_common(f.r, B, Hq, T, mask, causal);
   f.r.lse_s_in = lse_s;
   f.r.lse_t_in = lse_t;
-  if ((rc = hip_status(lard::launch_token_prep(f.r, Tp, w.tok_ok, w.first2, st),
-                       "attn_kl_backward_colgrad token prep launch")) != LARD_OK)
-    return rc;
-  if ((rc = hip_status(lard::launch_row_prep(f.r, Tp, w.tok_ok, w.first2, w.nl_s, w.nl_t, st),
-                       "attn_kl_backward_colgrad row prep launch")) != LARD_OK)
+  lard::RowPrepBatch rp = lard::row_prep_batch(f.r, Tp);
+  rp.rel[rp.n++] = {lse_s, lse_t, w.nl_s, w.nl_t, (int)Hq};
+  if ((rc = hip_status(lard::launch_row_prep(rp, (int)B, st), "attn_kl_backward_colgrad row prep launch")) != LARD_OK)
     return rc;
   f.Tp = Tp;
   f.tok_ok = w.tok_ok;
@@ -1164,7 +1187,7 @@ int lard_attn_kl_batched_forward(const lard_relation* rels, int nrel, const lard
   }
   const hipStream_t st = static_cast<hipStream_t>(stream);
   if (rows == 0)
-    return hip_status(lard::launch_reduce_sum(nullptr, 0, nullptr, loss_out, st), "batched forward reduce launch");
+    return hip_status(lard::launch_reduce_sum(nullptr, 0, nullptr, nullptr, loss_out, st), "batched forward reduce launch");
   const size_t need = lard_attn_kl_batched_workspace_bytes(rels, nrel);
   if (workspace == nullptr || workspace_bytes < need)
     return fail(LARD_ERR_INVALID_ARGUMENT, "workspace too small: need %zu bytes", need);
@@ -1174,9 +1197,9 @@ int lard_attn_kl_batched_forward(const lard_relation* rels, int nrel, const lard
   const bool bf = rels[0].xs.dtype == LARD_DTYPE_BF16;
   {
     const lard::HotArgs f0 = relation_args(rels[0], mask, causal, sm_scale_s, sm_scale_t, Tp, w.tok_ok, w.first2);
-    if ((rc = hip_status(lard::launch_token_prep(f0.r, Tp, w.tok_ok, w.first2, st),
-                         "batched forward token prep launch")) !=
-        LARD_OK)
+    if ((rc = hip_status(
+             lard::launch_token_prep(lard::token_prep(f0.r, Tp, w.tok_ok, w.first2, w.loss.counter), f0.r.B, st),
+             "batched forward token prep launch")) != LARD_OK)
       return rc;
   }
   int64_t row_off = 0;
@@ -1197,7 +1220,7 @@ int lard_attn_kl_batched_forward(const lard_relation* rels, int nrel, const lard
                          "batched forward launch")) != LARD_OK)
       return rc;
   }
-  return hip_status(lard::launch_reduce_sum(w.loss.rows, rows, w.loss.partial, loss_out, st),
+  return hip_status(lard::launch_reduce_sum(w.loss.rows, rows, w.loss.partial, w.loss.counter, loss_out, st),
                     "batched forward reduce launch");
 }
 
@@ -1233,21 +1256,19 @@ int lard_attn_kl_batched_backward(const lard_relation* rels, int nrel, const lar
     f.nl_s = nl_s;
     f.nl_t = nl_t;
     nl_off += rels[r].xs.size[0] * rels[r].xs.size[1] * (int64_t)Tp;
-    if (r == 0 && (rc = hip_status(lard::launch_token_prep(f.r, Tp, w.tok_ok, w.first2, st),
+    if (r == 0 && (rc = hip_status(lard::launch_token_prep(lard::token_prep(f.r, Tp, w.tok_ok, w.first2, nullptr), f.r.B, st),
                                    "batched backward token prep launch")) != LARD_OK)
-      return rc;
-    if (rel_rows(rels[r]) > 0 &&
-        (rc = hip_status(lard::launch_row_prep(f.r, Tp, w.tok_ok, w.first2, nl_s, nl_t, st),
-                                                  "batched backward row prep launch")) != LARD_OK)
       return rc;
   }
   for (int g = 0; g < nrel; g += lard::kMaxRelations) {
     // row side first (into dxs), then the column side, which adds it in place
     // and applies dloss * weight once
     lard::HotBatch mq{}, mk{};
+    lard::RowPrepBatch rp = lard::row_prep_batch(fs[0].r, Tp);
     for (int r = g; r < nrel && r < g + lard::kMaxRelations; ++r) {
       if (rel_rows(rels[r]) == 0) continue;
       lard::HotArgs f = fs[(size_t)r];
+      rp.rel[rp.n++] = row_prep(f);
       f.dq_out = rels[r].dxs;
       mq.rel[mq.n++] = f;
       f.r.dk_out = rels[r].dxs;
@@ -1257,6 +1278,7 @@ int lard_attn_kl_batched_backward(const lard_relation* rels, int nrel, const lar
       mk.rel[mk.n++] = f;
     }
     if (mq.n == 0) continue;
+    if ((rc = hip_status(lard::launch_row_prep(rp, fs[0].r.B, st), "batched backward row prep launch")) != LARD_OK) return rc;
     if ((rc = hip_status(timed(LARD_KERNEL_ROW_GRAD, st, [&] { return lard::launch_hot_dq_batch(mq, dp, bf, st); }),
                          "batched backward dq launch")) != LARD_OK)
       return rc;
@@ -1283,7 +1305,7 @@ int lard_attn_kl_batched_forward_rowgrad(const lard_relation* rels, int nrel, co
   }
   const hipStream_t st = static_cast<hipStream_t>(stream);
   if (rows == 0)
-    return hip_status(lard::launch_reduce_sum(nullptr, 0, nullptr, loss_out, st), "batched forward reduce launch");
+    return hip_status(lard::launch_reduce_sum(nullptr, 0, nullptr, nullptr, loss_out, st), "batched forward reduce launch");
   const size_t need = lard_attn_kl_batched_rowgrad_workspace_bytes(rels, nrel);
   if (workspace == nullptr || workspace_bytes < need)
     return fail(LARD_ERR_INVALID_ARGUMENT, "workspace too small: need %zu bytes", need);
@@ -1292,15 +1314,15 @@ int lard_attn_kl_batched_forward_rowgrad(const lard_relation* rels, int nrel, co
   const int Tp = (int)padded_len(rels[0].xs.size[2]);
   const int dp = padded_dim(rels[0].xs.size[3]);
   const bool bf = rels[0].xs.dtype == LARD_DTYPE_BF16;
-  {
-    const lard::HotArgs f0 = relation_args(rels[0], mask, causal, sm_scale_s, sm_scale_t, Tp, w.tok_ok, w.first2);
-    if ((rc = hip_status(lard::launch_token_prep(f0.r, Tp, w.tok_ok, w.first2, st),
-                         "batched forward_rowgrad token prep launch")) != LARD_OK)
-      return rc;
-  }
+  // the token pass rides the first group's pre-pass
+  const lard::HotArgs f0 = relation_args(rels[0], mask, causal, sm_scale_s, sm_scale_t, Tp, w.tok_ok, w.first2);
+  const lard::TokenPrep tok = lard::token_prep(f0.r, Tp, w.tok_ok, w.first2, w.loss.counter);
   int64_t row_off = 0;
+  bool tokens_done = false;
   for (int g = 0; g < nrel; g += lard::kMaxRelations) {
     lard::HotBatch m{};
+    lard::KeySide sides[2 * lard::kMaxRelations];
+    int nsides = 0;
     for (int r = g; r < nrel && r < g + lard::kMaxRelations; ++r) {
       if (rel_rows(rels[r]) == 0) continue;
       lard::HotArgs f = relation_args(rels[r], mask, causal, sm_scale_s, sm_scale_t, Tp, w.tok_ok, w.first2);
@@ -1309,19 +1331,21 @@ int lard_attn_kl_batched_forward_rowgrad(const lard_relation* rels, int nrel, co
       f.row_out = w.loss.rows + row_off;
       f.dq_out = rels[r].dxs;
       f.r.weight = weights != nullptr ? weights + r : nullptr;
-      if ((rc = hip_status(keys_f16(f, bf, rw.s[(size_t)r], rw.t[(size_t)r], st),
-                           "batched forward_rowgrad float16 keys launch")) != LARD_OK)
-        return rc;
+      keys_f16(f, bf, rw.s[(size_t)r], rw.t[(size_t)r], sides, &nsides);
       row_off += rel_rows(rels[r]);
       m.rel[m.n++] = f;
     }
     if (m.n == 0) continue;
+    if ((rc = launch_forward_prep(tokens_done ? nullptr : &tok, sides, nsides, f0.r.B, f0.r.T, f0.r.s.dim, st)) !=
+        LARD_OK)
+      return rc;
+    tokens_done = true;
     if ((rc = hip_status(timed(LARD_KERNEL_FORWARD_ROWGRAD, st,
                                [&] { return lard::launch_hot_fwdq_batch(m, dp, bf, st); }),
                          "batched forward_rowgrad launch")) != LARD_OK)
       return rc;
   }
-  return hip_status(lard::launch_reduce_sum(w.loss.rows, rows, w.loss.partial, loss_out, st),
+  return hip_status(lard::launch_reduce_sum(w.loss.rows, rows, w.loss.partial, w.loss.counter, loss_out, st),
                     "batched forward_rowgrad reduce launch");
 }
 
@@ -1357,21 +1381,16 @@ int lard_attn_kl_batched_backward_colgrad(const lard_relation* rels, int nrel, c
     f.nl_s = nl_s;
     f.nl_t = nl_t;
     nl_off += rels[r].xs.size[0] * rels[r].xs.size[1] * (int64_t)Tp;
-    if (r == 0 && (rc = hip_status(lard::launch_token_prep(f.r, Tp, w.tok_ok, w.first2, st),
-                                   "batched backward_colgrad token prep launch")) != LARD_OK)
-      return rc;
-    if (rel_rows(rels[r]) > 0 &&
-        (rc = hip_status(lard::launch_row_prep(f.r, Tp, w.tok_ok, w.first2, nl_s, nl_t, st),
-                         "batched backward_colgrad row prep launch")) != LARD_OK)
-      return rc;
   }
   for (int g = 0; g < nrel; g += lard::kMaxRelations) {
     // the column side adds itself to the row side in place and applies
     // dloss * weight once
     lard::HotBatch mk{};
+    lard::RowPrepBatch rp = lard::row_prep_batch(fs[0].r, Tp);
     for (int r = g; r < nrel && r < g + lard::kMaxRelations; ++r) {
       if (rel_rows(rels[r]) == 0) continue;
       lard::HotArgs f = fs[(size_t)r];
+      rp.rel[rp.n++] = row_prep(f);
       f.r.dk_out = rels[r].dxs;
       f.r.dk_add = rels[r].dxs;
       f.r.dscale = dloss;
@@ -1379,6 +1398,8 @@ int lard_attn_kl_batched_backward_colgrad(const lard_relation* rels, int nrel, c
       mk.rel[mk.n++] = f;
     }
     if (mk.n == 0) continue;
+    if ((rc = hip_status(lard::launch_row_prep(rp, fs[0].r.B, st), "batched backward_colgrad row prep launch")) != LARD_OK)
+      return rc;
     if ((rc = hip_status(timed(LARD_KERNEL_COL_GRAD, st, [&] { return lard::launch_hot_bwd_batch(mk, dp, bf, st); }),
                          "batched backward_colgrad dk launch")) != LARD_OK)
       return rc;

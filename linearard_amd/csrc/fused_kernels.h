@@ -47,6 +47,7 @@ __global__ __launch_bounds__(kStageThreads) void fused_fwd_kernel(const FusedArg
   const int my_i = i0w + l32;
   const bool in_range = my_i < T;
   const bool row_valid = in_range && mask_at(a.mask, a.mask_kind, (int64_t)b * a.mask_sb + my_i);
+  clear_counter(a);
   u16x8 fq_s[KS];
   u16x8 fq_t[KT];
   {

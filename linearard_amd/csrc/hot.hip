@@ -3,50 +3,41 @@
 
 namespace lard {
 
-// One workgroup per sequence b: tok_ok[b][j] = (j < T && mask[b][j] != 0)
-// for j < Tp (four tokens per thread and store), and first2[b] = the first
-// and second valid token of the sequence (T where there is none).
-constexpr int kPrepThreads = 1024;
+__global__ __launch_bounds__(kPrepThreads) void token_prep_kernel(const TokenPrep p) { token_prep_block(p, blockIdx.x); }
 
-__device__ __forceinline__ void two_smallest(int& f0, int& f1, int g0, int g1) {  // merge two sorted pairs
-  const int lo = min(f0, g0);
-  f1 = min(max(f0, g0), min(f1, g1));
-  f0 = lo;
-}
+// First two valid tokens of sequence b, as far as one_key needs them: scanned
+// by the whole workgroup from the start of the sequence, 4 tokens per thread
+// and step, until they are found (the first step, unless the sequence starts
+// with padding).
+constexpr int kRowPrepThreads = 256;
+constexpr int kRowPrepRows = 1024;  // rows per workgroup
 
-__global__ __launch_bounds__(kPrepThreads) void token_prep_kernel(const RelArgs a, int Tp,
-                                                                  unsigned char* __restrict__ tok_ok,
-                                                                  int* __restrict__ first2) {
-  const int b = blockIdx.x;
-  const int tid = threadIdx.x;
-  int f0 = a.T, f1 = a.T;  // this thread's two smallest valid tokens (it visits them in order)
-  for (int j0 = 4 * tid; j0 < Tp; j0 += 4 * kPrepThreads) {
-    unsigned word = 0;
+__device__ __forceinline__ void first_valid(const RowPrepBatch& p, int b, int& f0, int& f1) {
+  __shared__ int part[2][kRowPrepThreads / 64];
+  f0 = f1 = p.T;
+  for (int j0 = 0; j0 < p.T; j0 += 4 * kRowPrepThreads) {
+    int g0 = p.T, g1 = p.T;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int j = j0 + e;
-      if (j < a.T && mask_at(a.mask, a.mask_kind, (int64_t)b * a.mask_sb + j)) {
-        word |= 1u << (8 * e);
-        if (f0 == a.T)
-          f0 = j;
-        else if (f1 == a.T)
-          f1 = j;
+      const int j = j0 + 4 * (int)threadIdx.x + e;
+      if (j < p.T && mask_at(p.mask, p.mask_kind, (int64_t)b * p.mask_sb + j)) {
+        if (g0 == p.T)
+          g0 = j;
+        else if (g1 == p.T)
+          g1 = j;
       }
     }
-    *reinterpret_cast<unsigned*>(tok_ok + (int64_t)b * Tp + j0) = word;  // Tp is a multiple of 64
-  }
 #pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) two_smallest(f0, f1, __shfl_xor(f0, o, 64), __shfl_xor(f1, o, 64));
-  __shared__ int part[2][kPrepThreads / 64];
-  if ((tid & 63) == 0) {
-    part[0][tid >> 6] = f0;
-    part[1][tid >> 6] = f1;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    for (int w = 1; w < kPrepThreads / 64; ++w) two_smallest(f0, f1, part[0][w], part[1][w]);
-    first2[2 * b] = f0;
-    first2[2 * b + 1] = f1;
+    for (int o = 32; o >= 1; o >>= 1) two_smallest(g0, g1, __shfl_xor(g0, o, 64), __shfl_xor(g1, o, 64));
+    if ((threadIdx.x & 63) == 0) {
+      part[0][threadIdx.x >> 6] = g0;
+      part[1][threadIdx.x >> 6] = g1;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kRowPrepThreads / 64; ++w) two_smallest(f0, f1, part[0][w], part[1][w]);
+    __syncthreads();
+    if (f1 < p.T || (p.causal && f0 < p.T)) return;
   }
 }
 
@@ -55,36 +46,54 @@ __global__ __launch_bounds__(kPrepThreads) void token_prep_kernel(const RelArgs 
 // A row with exactly one valid key also gets -inf: there P_s = P_t = 1, so
 // its D is exactly 0 (kernel_C.py:224-233 with lse == S), which the
 // normalisers then give without any rounding of S * c2 - lse * log2(e).
-__global__ __launch_bounds__(256) void row_prep_kernel(const RelArgs a, int Tp, const unsigned char* __restrict__ tok_ok,
-                                                       const int* __restrict__ first2, float* __restrict__ nl_s,
-                                                       float* __restrict__ nl_t) {
-  const int i = blockIdx.x * 256 + (int)threadIdx.x;
-  const int64_t bh = blockIdx.y;
-  if (i >= Tp) return;
-  const int b = (int)(bh / a.Hq);
-  bool ok = false;
-  float ls = 0.f, lt = 0.f;
-  if (i < a.T) {
-    ls = a.lse_s_in[bh * a.T + i];
-    lt = a.lse_t_in[bh * a.T + i];
-    const bool one_key = a.causal ? i == first2[2 * b] : first2[2 * b + 1] >= a.T;
-    ok = tok_ok[(int64_t)b * Tp + i] != 0 && ls != kNegInf && lt != kNegInf && !one_key;
+// One launch for all relations of a call; it reads the mask itself, so the
+// backward of the autograd pair has no token pass before it (that pass and
+// one launch per relation were 9 of 17 launches of an 8-relation backward).
+__global__ __launch_bounds__(kRowPrepThreads) void row_prep_kernel(const RowPrepBatch p) {
+  int r = 0;
+  while (r + 1 < p.n && (int)blockIdx.x >= p.first[r + 1]) ++r;
+  const RowPrep& q = p.rel[r];
+  const int item = (int)blockIdx.x - p.first[r];
+  const int64_t bh = item / p.blocks;
+  const int row0 = (item - (int)bh * p.blocks) * kRowPrepRows;
+  const int b = (int)(bh / q.Hq);
+  int f0 = 0, f1 = 1;
+  if (p.mask != nullptr) first_valid(p, b, f0, f1);
+#pragma unroll
+  for (int e = 0; e < kRowPrepRows / kRowPrepThreads; ++e) {
+    const int i = row0 + e * kRowPrepThreads + (int)threadIdx.x;
+    if (i >= p.Tp) break;
+    bool ok = false;
+    float ls = 0.f, lt = 0.f;
+    if (i < p.T) {
+      ls = q.lse_s[bh * p.T + i];
+      lt = q.lse_t[bh * p.T + i];
+      const bool one_key = p.causal ? i == f0 : f1 >= p.T;
+      ok = mask_at(p.mask, p.mask_kind, (int64_t)b * p.mask_sb + i) && ls != kNegInf && lt != kNegInf && !one_key;
+    }
+    q.nl_s[bh * p.Tp + i] = ok ? -ls * kLog2e : kNegInf;
+    q.nl_t[bh * p.Tp + i] = ok ? -lt * kLog2e : kNegInf;
   }
-  nl_s[bh * Tp + i] = ok ? -ls * kLog2e : kNegInf;
-  nl_t[bh * Tp + i] = ok ? -lt * kLog2e : kNegInf;
 }
 
 bool hot_supported(int ds, int dt, bool same_dtype) { return same_dtype && ds == dt && ds <= 128; }
 
-hipError_t launch_token_prep(const RelArgs& a, int Tp, unsigned char* tok_ok, int* first2, hipStream_t stream) {
-  hipLaunchKernelGGL(token_prep_kernel, dim3(a.B), dim3(kPrepThreads), 0, stream, a, Tp, tok_ok, first2);
+hipError_t launch_token_prep(const TokenPrep& p, int B, hipStream_t stream) {
+  hipLaunchKernelGGL(token_prep_kernel, dim3(B), dim3(kPrepThreads), 0, stream, p);
   return hipGetLastError();
 }
 
-hipError_t launch_row_prep(const RelArgs& a, int Tp, const unsigned char* tok_ok, const int* first2, float* nl_s,
-                           float* nl_t, hipStream_t stream) {
-  hipLaunchKernelGGL(row_prep_kernel, dim3((Tp + 255) / 256, a.B * a.Hq), dim3(256), 0, stream, a, Tp, tok_ok, first2,
-                     nl_s, nl_t);
+hipError_t launch_row_prep(RowPrepBatch& p, int B, hipStream_t stream) {
+  if (p.n < 1 || p.n > kMaxRelations) return hipErrorInvalidValue;
+  p.blocks = (p.Tp + kRowPrepRows - 1) / kRowPrepRows;
+  int64_t items = 0;
+  for (int r = 0; r < p.n; ++r) {
+    p.first[r] = (int)items;
+    items += (int64_t)B * p.rel[r].Hq * p.blocks;
+    if (items > INT32_MAX) return hipErrorInvalidValue;
+  }
+  p.first[p.n] = (int)items;
+  hipLaunchKernelGGL(row_prep_kernel, dim3((unsigned)items), dim3(kRowPrepThreads), 0, stream, p);
   return hipGetLastError();
 }
 

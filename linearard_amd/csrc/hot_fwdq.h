@@ -739,11 +739,25 @@ __global__ __launch_bounds__(kWavesQ * 64) void hot_fwdq_batch_kernel(const HotB
 }
 
 hipError_t launch_hot_fwdq(const HotArgs& f, int dp, bool bf16, hipStream_t stream);
-// bfloat16 inputs, one side: k16 = float16(k * scale) as a contiguous
-// [B, Hkv, T, D] tensor, *scale = the power of two 2^-e chosen against
-// max |q|, |k| (device; maxbits is scratch).
-hipError_t launch_keys_f16(const SideArgs& s, int B, int Hq, int T, unsigned* maxbits, float* scale, u16* k16,
-                           hipStream_t stream);
+// bfloat16 inputs, one side of one relation: k16 = float16(k * scale) as a
+// contiguous [B, Hkv, T, D] tensor, *scale = the power of two 2^-e chosen
+// against max |q|, |k| (device; maxima is scratch, kKeyMaxima values).
+constexpr int kKeyMaxima = 512;
+struct KeySide {
+  const u16* k;
+  const u16* q;  // null: q is k
+  int64_t k_sb, k_sh, k_st, q_sb, q_sh, q_st;
+  int hkv, hq;
+  int k_heads;   // B * hkv
+  int units;     // filled by the launcher
+  unsigned* maxima;
+  float* scale;
+  u16* k16;
+};
+KeySide key_side(const SideArgs& s, int B, int Hq, unsigned* maxima, float* scale, u16* k16);
+// n <= 2 * kMaxRelations sides sharing B, T and D, and the call's token pass
+// when tok is not null.
+hipError_t launch_keys_f16(const KeySide* sides, int n, const TokenPrep* tok, int B, int T, int D, hipStream_t stream);
 hipError_t launch_hot_fwdq_batch(HotBatch& m, int dp, bool bf16, hipStream_t stream);
 
 }  // namespace lard

@@ -40,31 +40,37 @@ hipError_t fwdq_batch_dispatch(const HotBatch& m, int dp, hipStream_t stream) {
 // bfloat16 value below 2^15 is exactly a float16 value, down to 2^-17 in
 // magnitude), e <= kMaxScaleExp (values of 2^55 and more are beyond this
 // path: they would overflow float16 even scaled).
-// Three launches, all plain kernels (no memset, valid under graph capture):
-//   clear_u32_kernel       the maximum := 0;
+// Two launches for both sides of up to kMaxRelations relations:
 //   keys_f16_kernel        converts k with s = 1 (the scale of every input
-//                          below 2^15) and folds max |x| of k, and of q when
-//                          it is another tensor, into the maximum;
-//   keys_f16_fixup_kernel  writes s; when s < 1 (rare) converts k again.
-// Grid: x = one (b, head) of k, then (q != k) one (b, head) of q; y = blocks
-// of kKeyRows rows of that head (strided by gridDim.y beyond 65535 blocks).
-constexpr int kPrepBlock = 256;
-constexpr int kKeyRows = 64;
+//                          below 2^15) and leaves max |x| of k, and of q when
+//                          it is another tensor, as one value per workgroup;
+//                          its first workgroups do the call's token pass;
+//   keys_f16_fixup_kernel  reduces those maxima, writes s and, when s < 1
+//                          (rare), converts k again.
+// (With a clear, a conversion and a fixup launch per side and the token pass
+// apart, a batch of 8 relations took 49 launches: 640 of 2920 us at B=2,
+// n=2048, 48 heads; now 2.)
+// A workgroup of a side takes units of kUnitChunks 16-byte chunks (a row
+// block of one head), one chunk per thread, strided by the side's
+// workgroups; at most kKeyBlocks of them, so that one workgroup of the fixup
+// reduces a side's maxima in one read per thread.
+constexpr int kUnitChunks = kPrepThreads;
+constexpr int kKeyBlocks = kKeyMaxima;
+constexpr int kFixupBlocks = 64;
 constexpr int kMaxScaleExp = 40;
+static_assert(kKeyBlocks <= kPrepThreads, "one maximum per thread in the fixup");
 
-__global__ __launch_bounds__(64) void clear_u32_kernel(unsigned* p) {
-  if (threadIdx.x == 0) *p = 0u;
-}
-
-struct KeyPrep {
-  const u16* k;
-  const u16* q;        // null: q is k
-  int64_t k_sb, k_sh, k_st, q_sb, q_sh, q_st;
-  int hkv, hq, T, D;   // D % 8 == 0
-  unsigned* maxbits;
-  float* scale;
-  u16* k16;            // [B, hkv, T, D] contiguous
+struct KeyBatch {
+  TokenPrep tok;
+  int tok_blocks;                     // workgroups of the token pass (0: none)
+  int T, D;
+  int rows;                           // rows per unit
+  int tblocks;                        // units per head
+  int n;                              // sides
+  int first[2 * kMaxRelations + 1];   // workgroups before side i (after the token pass)
+  KeySide side[2 * kMaxRelations];
 };
+static_assert(sizeof(KeyBatch) <= 4096, "KeyBatch exceeds the 4 KiB kernel-argument limit");
 
 __device__ __forceinline__ float side_scale(unsigned maxbits) {
   if (maxbits >= 0x7f80u) return 1.f;  // inf / NaN: nothing to scale against
@@ -75,93 +81,103 @@ __device__ __forceinline__ float side_scale(unsigned maxbits) {
   return ldexpf(1.f, -e);
 }
 
-// The rows of this block: (b, head) and the first row, for k (or q) heads.
-struct KeyRows {
-  const u16* base;
-  int64_t st;
-  int head;
-  bool is_q;
-  int64_t b;
-};
-
-__device__ __forceinline__ KeyRows key_rows(const KeyPrep& p, int nbk) {
-  KeyRows r;
-  const int x = (int)blockIdx.x;
-  r.is_q = x >= nbk;
-  const int bh = r.is_q ? x - nbk : x;
-  const int H = r.is_q ? p.hq : p.hkv;
-  r.b = bh / H;
-  r.head = bh - (int)r.b * H;
-  r.base = r.is_q ? p.q + r.b * p.q_sb + (int64_t)r.head * p.q_sh : p.k + r.b * p.k_sb + (int64_t)r.head * p.k_sh;
-  r.st = r.is_q ? p.q_st : p.k_st;
-  return r;
+// Converts the key rows of unit u (q units are only read) with scale s;
+// returns the maximum magnitude bits of this thread's chunk.
+__device__ __forceinline__ unsigned key_unit(const KeyBatch& p, const KeySide& k, int u, float s) {
+  const int bh0 = u / p.tblocks;
+  const bool is_q = bh0 >= k.k_heads;
+  const int bh = is_q ? bh0 - k.k_heads : bh0;
+  const int H = is_q ? k.hq : k.hkv;
+  const int b = bh / H, h = bh - b * H;
+  const u16* base = is_q ? k.q + b * k.q_sb + h * k.q_sh : k.k + b * k.k_sb + h * k.k_sh;
+  const int64_t st = is_q ? k.q_st : k.k_st;
+  const int cpr = p.D / 8;
+  const int r = (int)threadIdx.x / cpr, d0 = ((int)threadIdx.x - r * cpr) * 8;
+  const int t = (u - bh0 * p.tblocks) * p.rows + r;
+  if (r >= p.rows || t >= p.T) return 0;
+  const u16x8 v = *reinterpret_cast<const u16x8*>(base + t * st + d0);
+  unsigned m = 0;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) m = max(m, (unsigned)(v[e] & 0x7fffu));
+  if (!is_q) *reinterpret_cast<u16x8*>(k.k16 + ((int64_t)bh * p.T + t) * p.D + d0) = bf16_to_f16_scaled(v, s);
+  return m;
 }
 
-__global__ __launch_bounds__(kPrepBlock) void keys_f16_kernel(const KeyPrep p, int nbk) {
-  const KeyRows r = key_rows(p, nbk);
-  const int cpr = p.D / 8;
-  u16* out = p.k16 + ((r.b * p.hkv + r.head) * (int64_t)p.T) * p.D;
-  unsigned m = 0;
-  for (int t0 = (int)blockIdx.y * kKeyRows; t0 < p.T; t0 += (int)gridDim.y * kKeyRows) {
-    const int n = min(kKeyRows, p.T - t0) * cpr;
-    for (int c = (int)threadIdx.x; c < n; c += kPrepBlock) {
-      const int t = t0 + c / cpr;
-      const int d0 = (c - (t - t0) * cpr) * 8;
-      const u16x8 v = *reinterpret_cast<const u16x8*>(r.base + t * r.st + d0);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) m = max(m, (unsigned)(v[e] & 0x7fffu));
-      if (!r.is_q) *reinterpret_cast<u16x8*>(out + (int64_t)t * p.D + d0) = bf16_to_f16_scaled(v, 1.f);
-    }
-  }
+// Maximum over the workgroup, in every thread.
+__device__ __forceinline__ unsigned block_max(unsigned m) {
+  __shared__ unsigned red[kPrepThreads / 64];
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o, 64));
-  __shared__ unsigned red[kPrepBlock / 64];
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
-  if (threadIdx.x == 0) {
 #pragma unroll
-    for (int w = 1; w < kPrepBlock / 64; ++w) m = max(m, red[w]);
-    // the maximum only grows: a block below what is already there skips the
-    // atomic (a stale read only costs an atomic that changes nothing)
-    if (m > __hip_atomic_load(p.maxbits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(p.maxbits, m);
-  }
+  for (int w = 0; w < kPrepThreads / 64; ++w) m = max(m, red[w]);
+  return m;
 }
 
-__global__ __launch_bounds__(kPrepBlock) void keys_f16_fixup_kernel(const KeyPrep p, int nbk) {
-  const float s = side_scale(*p.maxbits);
-  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *p.scale = s;
-  if (s == 1.f || (int)blockIdx.x >= nbk) return;  // the first pass converted with s = 1
-  const KeyRows r = key_rows(p, nbk);
-  const int cpr = p.D / 8;
-  u16* out = p.k16 + ((r.b * p.hkv + r.head) * (int64_t)p.T) * p.D;
-  for (int t0 = (int)blockIdx.y * kKeyRows; t0 < p.T; t0 += (int)gridDim.y * kKeyRows) {
-    const int n = min(kKeyRows, p.T - t0) * cpr;
-    for (int c = (int)threadIdx.x; c < n; c += kPrepBlock) {
-      const int t = t0 + c / cpr;
-      const int d0 = (c - (t - t0) * cpr) * 8;
-      const u16x8 v = *reinterpret_cast<const u16x8*>(r.base + t * r.st + d0);
-      *reinterpret_cast<u16x8*>(out + (int64_t)t * p.D + d0) = bf16_to_f16_scaled(v, s);
-    }
+__global__ __launch_bounds__(kPrepThreads) void keys_f16_kernel(const KeyBatch p) {
+  if ((int)blockIdx.x < p.tok_blocks) {
+    token_prep_block(p.tok, blockIdx.x);
+    return;
   }
+  const int item = (int)blockIdx.x - p.tok_blocks;
+  int i = 0;
+  while (i + 1 < p.n && item >= p.first[i + 1]) ++i;
+  const KeySide& k = p.side[i];
+  const int blocks = p.first[i + 1] - p.first[i];
+  unsigned m = 0;
+  for (int u = item - p.first[i]; u < k.units; u += blocks) m = max(m, key_unit(p, k, u, 1.f));
+  m = block_max(m);
+  if (threadIdx.x == 0) k.maxima[item - p.first[i]] = m;
 }
 
-hipError_t launch_keys_f16(const SideArgs& s, int B, int Hq, int T, unsigned* maxbits, float* scale, u16* k16,
-                           hipStream_t stream) {
-  KeyPrep p{};
-  p.k = s.k;
-  p.q = s.q != s.k ? s.q : nullptr;
-  p.k_sb = s.k_sb, p.k_sh = s.k_sh, p.k_st = s.k_st;
-  p.q_sb = s.q_sb, p.q_sh = s.q_sh, p.q_st = s.q_st;
-  p.hkv = s.hkv, p.hq = Hq, p.T = T, p.D = s.dim;
-  p.maxbits = maxbits, p.scale = scale, p.k16 = k16;
-  const int64_t nbk = (int64_t)B * s.hkv;
-  const int64_t nbx = nbk + (p.q != nullptr ? (int64_t)B * Hq : 0);
-  const int64_t nby = std::min<int64_t>((T + kKeyRows - 1) / kKeyRows, 65535);
-  if (nbx > INT32_MAX) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)nbx, (unsigned)nby), block(kPrepBlock);
-  hipLaunchKernelGGL(clear_u32_kernel, dim3(1), dim3(64), 0, stream, maxbits);
-  hipLaunchKernelGGL(keys_f16_kernel, grid, block, 0, stream, p, (int)nbk);
-  hipLaunchKernelGGL(keys_f16_fixup_kernel, grid, block, 0, stream, p, (int)nbk);
+__global__ __launch_bounds__(kPrepThreads) void keys_f16_fixup_kernel(const KeyBatch p) {
+  const KeySide& k = p.side[blockIdx.y];
+  const int blocks = p.first[blockIdx.y + 1] - p.first[blockIdx.y];
+  const float s = side_scale(block_max((int)threadIdx.x < blocks ? k.maxima[threadIdx.x] : 0u));
+  if (blockIdx.x == 0 && threadIdx.x == 0) *k.scale = s;
+  if (s == 1.f) return;  // the first pass converted with s = 1
+  const int key_units = k.k_heads * p.tblocks;
+  for (int u = blockIdx.x; u < key_units; u += (int)gridDim.x) (void)key_unit(p, k, u, s);
+}
+
+KeySide key_side(const SideArgs& s, int B, int Hq, unsigned* maxima, float* scale, u16* k16) {
+  KeySide k{};
+  k.k = s.k;
+  k.q = s.q != s.k ? s.q : nullptr;
+  k.k_sb = s.k_sb, k.k_sh = s.k_sh, k.k_st = s.k_st;
+  k.q_sb = s.q_sb, k.q_sh = s.q_sh, k.q_st = s.q_st;
+  k.hkv = s.hkv, k.hq = Hq, k.k_heads = B * s.hkv;
+  k.maxima = maxima, k.scale = scale, k.k16 = k16;
+  return k;
+}
+
+hipError_t launch_keys_f16(const KeySide* sides, int n, const TokenPrep* tok, int B, int T, int D, hipStream_t stream) {
+  if (n < 1 || n > 2 * kMaxRelations || D < 8 || D > 8 * kUnitChunks) return hipErrorInvalidValue;
+  KeyBatch p{};
+  p.T = T, p.D = D, p.n = n;
+  p.rows = kUnitChunks / (D / 8);
+  p.tblocks = (T + p.rows - 1) / p.rows;
+  if (tok != nullptr) {
+    p.tok = *tok;
+    p.tok_blocks = B;
+  }
+  int64_t total = p.tok_blocks;
+  int fix = 1;
+  for (int i = 0; i < n; ++i) {
+    KeySide& k = p.side[i] = sides[i];
+    const int64_t heads = (int64_t)k.k_heads + (k.q != nullptr ? (int64_t)B * k.hq : 0);
+    const int64_t units = heads * p.tblocks;
+    if (units > INT32_MAX) return hipErrorInvalidValue;
+    k.units = (int)units;
+    p.first[i] = (int)(total - p.tok_blocks);
+    total += units < kKeyBlocks ? units : kKeyBlocks;
+    fix = std::max(fix, (int)std::min<int64_t>((int64_t)k.k_heads * p.tblocks, kFixupBlocks));
+  }
+  p.first[n] = (int)(total - p.tok_blocks);
+  if (total > INT32_MAX) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(keys_f16_kernel, dim3((unsigned)total), dim3(kPrepThreads), 0, stream, p);
+  hipLaunchKernelGGL(keys_f16_fixup_kernel, dim3((unsigned)fix, (unsigned)n), dim3(kPrepThreads), 0, stream, p);
   return hipGetLastError();
 }
 

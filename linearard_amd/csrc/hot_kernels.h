@@ -1,10 +1,13 @@
 // Throughput kernels of the autograd path for Ds == Dt <= 128 and one dtype
 // (every shape train.py produces: Llama/Mistral heads are d=128 bf16).
 //
-//   token_prep_kernel      per token: valid (j < T and mask != 0), one byte.
+//   token_prep_kernel      per token: valid (j < T and mask != 0), one byte,
+//                          and each sequence's first two valid tokens (part
+//                          of keys_f16_kernel's launch for bfloat16 inputs).
 //   row_prep_kernel        per query row of the backward: -lse * log2(e) for
 //                          student and teacher, -inf outside the valid set
-//                          (kernel_C.py:155-161), so exp2(x * c + nl) is P.
+//                          (kernel_C.py:155-161), so exp2(x * c + nl) is P;
+//                          one launch for every relation of a call.
 //   hot_fwd_kernel         forward of AttnKLAlignFn (integration.py:8-45):
 //                          per query row both online softmaxes (stage A for
 //                          student and teacher) and the KL (stage B), one pass.
@@ -1206,10 +1209,98 @@ __global__ __launch_bounds__(kWaves * 64) void hot_bwd_batch_kernel(const HotBat
   hot_bwd_body<DP, BF>(m.rel[r], g - m.first[r]);
 }
 
+// ----------------------------------------------------------------------------
+// pre-passes
+// ----------------------------------------------------------------------------
+// Token validity of every sequence (tok_ok[b][j] = (j < T && mask[b][j] != 0)
+// for j < Tp), its first two valid tokens (first2[b], T where there is none)
+// and the loss reduction's ticket counter := 0 (when not null).
+struct TokenPrep {
+  const void* mask;
+  int mask_kind;
+  int64_t mask_sb;
+  int T, Tp;
+  unsigned char* tok_ok;
+  int* first2;
+  unsigned* counter;
+};
+
+inline TokenPrep token_prep(const RelArgs& a, int Tp, unsigned char* tok_ok, int* first2, unsigned* counter) {
+  return {a.mask, a.mask_kind, a.mask_sb, a.T, Tp, tok_ok, first2, counter};
+}
+
+constexpr int kPrepThreads = 1024;
+
+__device__ __forceinline__ void two_smallest(int& f0, int& f1, int g0, int g1) {  // merge two sorted pairs
+  const int lo = min(f0, g0);
+  f1 = min(max(f0, g0), min(f1, g1));
+  f0 = lo;
+}
+
+// Sequence b, by one workgroup of kPrepThreads (four tokens per thread and store).
+__device__ __forceinline__ void token_prep_block(const TokenPrep& p, int b) {
+  const int tid = threadIdx.x;
+  if (b == 0 && tid == 0 && p.counter != nullptr) *p.counter = 0u;
+  int f0 = p.T, f1 = p.T;  // this thread's two smallest valid tokens (it visits them in order)
+  for (int j0 = 4 * tid; j0 < p.Tp; j0 += 4 * kPrepThreads) {
+    unsigned word = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int j = j0 + e;
+      if (j < p.T && mask_at(p.mask, p.mask_kind, (int64_t)b * p.mask_sb + j)) {
+        word |= 1u << (8 * e);
+        if (f0 == p.T)
+          f0 = j;
+        else if (f1 == p.T)
+          f1 = j;
+      }
+    }
+    *reinterpret_cast<unsigned*>(p.tok_ok + (int64_t)b * p.Tp + j0) = word;  // Tp is a multiple of 64
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) two_smallest(f0, f1, __shfl_xor(f0, o, 64), __shfl_xor(f1, o, 64));
+  __shared__ int part[2][kPrepThreads / 64];
+  if ((tid & 63) == 0) {
+    part[0][tid >> 6] = f0;
+    part[1][tid >> 6] = f1;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < kPrepThreads / 64; ++w) two_smallest(f0, f1, part[0][w], part[1][w]);
+    p.first2[2 * b] = f0;
+    p.first2[2 * b + 1] = f1;
+  }
+}
+
+// Row normalisers of up to kMaxRelations relations sharing B, T and the mask.
+struct RowPrep {
+  const float* lse_s;  // [B, Hq, T]
+  const float* lse_t;
+  float* nl_s;         // [B, Hq][Tp]
+  float* nl_t;
+  int Hq;
+};
+struct RowPrepBatch {
+  const void* mask;
+  int mask_kind;
+  int64_t mask_sb;
+  int T, Tp, causal;
+  int n;
+  int blocks;                    // workgroups per head (filled by the launcher)
+  int first[kMaxRelations + 1];  // workgroups before relation r (filled by the launcher)
+  RowPrep rel[kMaxRelations];
+};
+
+inline RowPrepBatch row_prep_batch(const RelArgs& a, int Tp) {
+  RowPrepBatch p{};
+  p.mask = a.mask, p.mask_kind = a.mask_kind, p.mask_sb = a.mask_sb;
+  p.T = a.T, p.Tp = Tp, p.causal = a.causal;
+  return p;
+}
+
 bool hot_supported(int ds, int dt, bool same_dtype);
-hipError_t launch_token_prep(const RelArgs& a, int Tp, unsigned char* tok_ok, int* first2, hipStream_t stream);
-hipError_t launch_row_prep(const RelArgs& a, int Tp, const unsigned char* tok_ok, const int* first2, float* nl_s,
-                           float* nl_t, hipStream_t stream);
+hipError_t launch_token_prep(const TokenPrep& p, int B, hipStream_t stream);
+hipError_t launch_row_prep(RowPrepBatch& p, int B, hipStream_t stream);
 hipError_t launch_hot_fwd(const HotArgs& f, int dp, bool bf16, hipStream_t stream);
 hipError_t launch_hot_dq(const HotArgs& f, int dp, bool bf16, hipStream_t stream);
 hipError_t launch_hot_bwd(const HotArgs& f, int dp, bool bf16, hipStream_t stream);

@@ -80,6 +80,9 @@ struct RelArgs {
   // dq / dk passes read them (instead of lse_*_in) when non-null.
   double* lse64_out;
   const double* lse64_in;
+  // Forward kernels that precede the loss reduction: the reduction's ticket
+  // counter, which they set to 0 (null elsewhere).
+  unsigned* counter;
 };
 
 // Outputs of the fused forward (one pass: both LSEs and the per-row KL).
@@ -96,6 +99,10 @@ template <bool V>
 struct Flag {
   static constexpr bool value = V;
 };
+
+__device__ __forceinline__ void clear_counter(const RelArgs& a) {
+  if (a.counter != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *a.counter = 0u;
+}
 
 __device__ __forceinline__ bool mask_at(const void* m, int kind, int64_t idx) {
   if (kind == 1) return static_cast<const unsigned char*>(m)[idx] != 0;

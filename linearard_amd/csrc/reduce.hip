@@ -1,8 +1,9 @@
 // Deterministic sum of the per-row KL terms into the 0-d loss.  The
 // reference adds one fp32 atomic per program into a shared scalar
 // (kernel_B.py:216-218), whose order is nondeterministic; here the sum runs
-// in a fixed order in double precision: kReduceBlocks workgroups each sum a
-// contiguous slice into one partial, then one workgroup sums the partials.
+// in a fixed order in double precision: up to kReduceBlocks workgroups each
+// sum a contiguous slice into one partial, and the last of them to finish
+// sums the partials.
 #include "stage_kernels.h"
 
 namespace lard {
@@ -10,6 +11,7 @@ namespace lard {
 constexpr int kReduceThreads = 256;
 
 __device__ __forceinline__ double block_sum(double s, double* part) {
+  __syncthreads();  // part may hold an earlier sum
   part[threadIdx.x] = s;
   __syncthreads();
   for (int stride = kReduceThreads / 2; stride > 0; stride >>= 1) {
@@ -19,38 +21,61 @@ __device__ __forceinline__ double block_sum(double s, double* part) {
   return part[0];
 }
 
-__global__ __launch_bounds__(kReduceThreads) void reduce_partial_kernel(const float* __restrict__ x, int64_t n,
-                                                                        double* __restrict__ partial) {
+// One launch: block i sums slice i (a multiple of 1024 values) into
+// partial[i]; the block that finishes last (ticket counter, which an earlier
+// kernel of the same call set to 0) sums the partials.  Which block that is
+// does not change the result: the partials are always summed in one order.
+// A second launch for the final sum cost 3-5 us of a 40-190 us call.  64
+// workgroups: with 256 the tickets took 9 us (n = 262144) against 5.
+__global__ __launch_bounds__(kReduceThreads) void reduce_sum_kernel(const float* __restrict__ x, int64_t n, int64_t per,
+                                                                    double* partial, unsigned* counter,
+                                                                    float* __restrict__ out) {
   __shared__ double part[kReduceThreads];
-  const int64_t per = (n + kReduceBlocks - 1) / kReduceBlocks;
+  __shared__ bool last;
   const int64_t lo = per * blockIdx.x;
   const int64_t hi = lo + per < n ? lo + per : n;
   double s = 0.0;
-  for (int64_t i = lo + threadIdx.x; i < hi; i += kReduceThreads) s += (double)x[i];
+  int64_t i = lo + 4 * threadIdx.x;
+#pragma unroll 4
+  for (; i + 4 <= hi; i += 4 * kReduceThreads) {  // x is 256-byte aligned and lo a multiple of 1024
+    const f32x4 v = *reinterpret_cast<const f32x4*>(x + i);
+    s += ((double)v[0] + (double)v[1]) + ((double)v[2] + (double)v[3]);
+  }
+  for (; i < hi; ++i) s += (double)x[i];  // the slice's last 1-3 values, one thread
   const double total = block_sum(s, part);
-  if (threadIdx.x == 0) partial[blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(kReduceThreads) void reduce_final_kernel(const double* __restrict__ partial,
-                                                                      float* __restrict__ out) {
-  __shared__ double part[kReduceThreads];
-  double s = 0.0;
-  for (int i = threadIdx.x; i < kReduceBlocks; i += kReduceThreads) s += partial[i];
-  const double total = block_sum(s, part);
-  if (threadIdx.x == 0) out[0] = (float)total;
+  if (threadIdx.x == 0) {
+    // The partials cross the XCDs' L2s: stored and loaded at agent scope
+    // (written through, read past the local L2), the store complete before
+    // the ticket is taken.  A release on the ticket instead would write back
+    // every dirty line of the L2, once per workgroup.
+    __hip_atomic_store(&partial[blockIdx.x], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  s = 0.0;
+  if (threadIdx.x < gridDim.x)  // at most kReduceBlocks <= kReduceThreads partials
+    s = __hip_atomic_load(&partial[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const double sum = block_sum(s, part);
+  if (threadIdx.x == 0) out[0] = (float)sum;
 }
 
 __global__ __launch_bounds__(kReduceThreads) void reduce_zero_kernel(float* __restrict__ out) {
   if (threadIdx.x == 0) out[0] = 0.f;
 }
 
-hipError_t launch_reduce_sum(const float* x, int64_t n, double* partial, float* out, hipStream_t stream) {
+hipError_t launch_reduce_sum(const float* x, int64_t n, double* partial, unsigned* counter, float* out,
+                             hipStream_t stream) {
   if (n <= 0) {
     hipLaunchKernelGGL(reduce_zero_kernel, dim3(1), dim3(kReduceThreads), 0, stream, out);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL(reduce_partial_kernel, dim3(kReduceBlocks), dim3(kReduceThreads), 0, stream, x, n, partial);
-  hipLaunchKernelGGL(reduce_final_kernel, dim3(1), dim3(kReduceThreads), 0, stream, partial, out);
+  static_assert(kReduceBlocks <= kReduceThreads, "one partial per thread in the final sum");
+  const int64_t units = (n + 1023) / 1024;  // of 1024 values, one 16-byte load per thread
+  const int64_t per = (units + kReduceBlocks - 1) / kReduceBlocks * 1024;
+  const unsigned blocks = (unsigned)((n + per - 1) / per);
+  hipLaunchKernelGGL(reduce_sum_kernel, dim3(blocks), dim3(kReduceThreads), 0, stream, x, n, per, partial, counter, out);
   return hipGetLastError();
 }
 

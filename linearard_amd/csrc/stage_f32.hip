@@ -165,6 +165,7 @@ __global__ __launch_bounds__(kF32Threads) void row_f32_kernel(const RelArgs a) {
   const bool row_valid = in_range && mask_at(a.mask, a.mask_kind, (int64_t)b * a.mask_sb + my_i);
   const int64_t row_index = (int64_t)bh * T + my_i;
   const bool two = MODE != MODE_LSE;
+  if constexpr (MODE == MODE_KL || MODE == kModeFused) clear_counter(a);
 
   bool ok = row_valid;
   double lse_s = 0.0, lse_t = 0.0;

@@ -58,6 +58,7 @@ __global__ __launch_bounds__(kStageThreads) void row_kernel(const RelArgs a) {
   const bool row_valid = in_range && mask_at(a.mask, a.mask_kind, (int64_t)b * a.mask_sb + my_i);
   const bool sbf = a.s.bf16 != 0;
   const bool tbf = a.t.bf16 != 0;
+  if constexpr (MODE == MODE_KL) clear_counter(a);
 
   // MODE_DQ: K^T operand of the second GEMM, read transposed from lks
   TrRowTile<DPS, SS> trk;
@@ -507,9 +508,12 @@ hipError_t launch_row_lse(const RelArgs& a, int dps, hipStream_t stream);
 hipError_t launch_row_kl(const RelArgs& a, int dps, int dpt, hipStream_t stream);
 hipError_t launch_row_dq(const RelArgs& a, int dps, int dpt, hipStream_t stream);
 hipError_t launch_col_dk(const RelArgs& a, int dps, int dpt, hipStream_t stream);
-// Loss reduction: out = sum(x[0..n)) through kReduceBlocks double partials.
-constexpr int kReduceBlocks = 512;
-hipError_t launch_reduce_sum(const float* x, int64_t n, double* partial, float* out, hipStream_t stream);
+// Loss reduction: out = sum(x[0..n)) through at most kReduceBlocks double
+// partials; *counter must be 0 when the launch starts (the forward kernels
+// clear it: RelArgs::counter), x 16-byte aligned.
+constexpr int kReduceBlocks = 64;
+hipError_t launch_reduce_sum(const float* x, int64_t n, double* partial, unsigned* counter, float* out,
+                             hipStream_t stream);
 // x[0..n) *= (*dscale) in place (dscale a device scalar; n a multiple of 4,
 // x 16-byte aligned): the chain rule of a gradient computed before dloss.
 hipError_t launch_scale_inplace(float* x, int64_t n, const float* dscale, hipStream_t stream);
