@@ -70,6 +70,28 @@ def test_rope_pair_takes_a_permuted_view_without_a_copy(gpu_available):
     assert torch.equal(a_s, b_s) and torch.equal(a_t, b_t)
 
 
+@pytest.mark.parametrize("B,H,T,D", [
+    (1, 1, 33, 128), (1, 2, 17, 128), (2, 7, 5, 128), (1, 8, 1, 128), (1, 9, 4, 128),  # head groups of 1, 2, 4, 8
+    (1, 8, 9, 64), (1, 5, 23, 48), (1, 16, 3, 16),  # tokens per workgroup: 8, 16 (idle threads), 32
+    (1, 2, 3, 4096), (1, 2, 3, 4128),  # one and two chunk ranges
+])
+def test_rope_pair_workgroup_edges(gpu_available, B, H, T, D):
+    """Every split of a workgroup into head groups, tokens and chunks, whole
+    and ragged, writes what the oracle's rotation gives."""
+    from linearard_amd.rope import rope_inv_freq, rope_pair
+
+    rng = np.random.default_rng(B * 1000 + H * 100 + T + D)
+    x = round_to(rng.standard_normal((B, T, H, D)).astype(np.float32), "bf16")
+    xd = torch.tensor(x, device="cuda").to(torch.bfloat16).permute(0, 2, 1, 3)
+    xs, xt = rope_pair(xd, 10000.0, {"rope_type": "linear", "factor": 4.0})
+    xh = x.transpose(0, 2, 1, 3)
+    pos = np.arange(T, dtype=np.int64)
+    for b in range(B):
+        _check(xt[b], R.rope_apply(xh[b], rope_inv_freq(D, 10000.0).numpy(), pos, "bf16"), xh[b], "bf16")
+        inv_s = rope_inv_freq(D, 10000.0, {"rope_type": "linear", "factor": 4.0}).numpy()
+        _check(xs[b], R.rope_apply(xh[b], inv_s, pos, "bf16"), xh[b], "bf16")
+
+
 def test_rope_pair_rejects_unsupported_head_dims(gpu_available):
     from linearard_amd.rope import rope_pair
 
