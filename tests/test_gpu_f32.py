@@ -84,6 +84,47 @@ def test_f32_autograd_self_relation_matches_the_oracle(gpu_available, ratio):
     check_grad(x.grad.cpu().numpy(), rdx, f"f32-autograd-r{ratio}", bar=F32_BAR)
 
 
+@pytest.mark.parametrize("T", [15, 16, 17, 31, 33, 63, 64, 65, 129])
+@pytest.mark.parametrize("ds,dt,scale", [(8, 8, 1.0), (32, 16, 1.0), (64, 64, 3.0), (64, 128, 1.0), (128, 128, 4.0),
+                                         (256, 256, 1.0)])
+def test_f32_tile_edges_match_the_oracle(gpu_available, T, ds, dt, scale):
+    """Around the 16 rows of a wave, the 32 of a tile and the 64 of a
+    workgroup, for every kernel width (32, 64, 128, 256) and for dims below
+    it (padded with zeros); inputs of scale 3 and 4 have logits over 100, whose
+    exponentials underflow.  Grouped queries, a mask with holes, and a
+    self relation through autograd."""
+    from linearard_amd.attention_KL import attn_kl_align, kl_backward, kl_forward, lse_stats
+
+    rng = np.random.default_rng(T * 7 + ds + dt)
+    for causal, ratio in ((True, None), (False, 0.3), (True, 0.3)):
+        qs, ks, qt, kt, mask = _inputs(rng, 2, 4, 2, 4, T, ds, dt, ratio, scale)
+        a_s, a_t = 1 / math.sqrt(ds), 1 / math.sqrt(dt)
+        d = [to_dev(x, "f32") for x in (qs, ks, qt, kt)]
+        m = mask_to_dev(mask)
+        lse_s, lse_t = lse_stats(d[0], d[1], m, causal, a_s), lse_stats(d[2], d[3], m, causal, a_t)
+        rls, rlt = O.lse_stats(qs, ks, mask, causal, a_s), O.lse_stats(qt, kt, mask, causal, a_t)
+        # a float64 value rounded once to float32
+        np.testing.assert_allclose(lse_s.cpu().numpy(), rls, rtol=2.0 ** -23, atol=1e-7)
+        np.testing.assert_allclose(lse_t.cpu().numpy(), rlt, rtol=2.0 ** -23, atol=1e-7)
+        case = f"f32-edges-c{int(causal)}-r{ratio}-T{T}-ds{ds}-dt{dt}"
+        # the stages work from float32 LSEs, whose rounding (2^-24 of logits up
+        # to 200) is a relative error of P up to 1.2e-5: twice that
+        bar = 2.5e-5 if scale > 1 else F32_BAR
+        loss = float(kl_forward(d[0], d[1], lse_s, d[2], d[3], lse_t, m, causal, a_s, a_t))
+        check_loss(loss, O.kl_forward(qs, ks, rls, qt, kt, rlt, mask, causal, a_s, a_t), case, bar=bar)
+        dq, dk = kl_backward(d[0], d[1], lse_s, d[2], d[3], lse_t, m, causal, a_s, a_t)
+        rq, rk = O.kl_backward(qs, ks, rls, qt, kt, rlt, mask, causal, a_s, a_t)
+        for name, got, want in (("dq", dq, rq), ("dk", dk, rk)):
+            check_grad(got.cpu().numpy(), want, case, name, bar=bar)
+        if ds == dt and scale == 1:  # the autograd pair keeps its LSEs in double
+            x = to_dev(qs, "f32", requires_grad=True)
+            loss = attn_kl_align(x, x, d[2], d[2], attn_mask=m, causal=causal, sm_scale_s=a_s, sm_scale_t=a_t)
+            loss.backward()
+            ref, rdx, _, _, _ = O.attn_kl_align(qs, qs, qt, qt, mask, causal, a_s, a_t, self_relation=True)
+            check_loss(loss.item(), ref, case + "-autograd", bar=1e-6)
+            check_grad(x.grad.cpu().numpy(), rdx, case + "-autograd", bar=1e-6)
+
+
 def test_f32_cfg1_against_eager_pytorch(gpu_available):
     """BASELINE cfg1: B=1, H=32, n=1024, d=128, X_t ~ N(0,1) (seed 0),
     X_s = X_t + 0.1 N(0,1), scale 1/sqrt(d), causal; against float32 eager
