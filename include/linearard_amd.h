@@ -203,6 +203,25 @@ int lard_attn_kl_backward(const lard_tensor4* qs, const lard_tensor4* ks, const 
                           void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * The autograd pair of float32 inputs -- AttnKLAlignFn.forward / backward
+ * (integration.py:8-67), which the reference restricts to fp16/bf16.  The
+ * forward also writes both LSEs in double, lse64_out[2][B, Hq, T] (student,
+ * then teacher); the backward reads them instead of recomputing them from
+ * the operands, as lard_attn_kl_backward does for float32 inputs (the float32
+ * LSEs are too coarse for D = P_s - P_t of a near-identical pair), and needs
+ * no workspace.  Other dtypes are LARD_ERR_UNSUPPORTED.
+ */
+int lard_attn_kl_forward_lse64(const lard_tensor4* qs, const lard_tensor4* ks, const lard_tensor4* qt,
+                               const lard_tensor4* kt, const lard_mask* mask, int causal, float sm_scale_s,
+                               float sm_scale_t, float* lse_s_out, float* lse_t_out, float* loss_out,
+                               double* lse64_out, void* workspace, size_t workspace_bytes, void* stream);
+int lard_attn_kl_backward_lse64(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s,
+                                const lard_tensor4* qt, const lard_tensor4* kt, const float* lse_t,
+                                const double* lse64, const lard_mask* mask, int causal, float sm_scale_s,
+                                float sm_scale_t, const float* dloss, int self_relation, float* dq_out,
+                                float* dk_out, void* stream);
+
+/*
  * Autograd forward with the row side of the backward -- AttnKLAlignFn.forward
  * (integration.py:8-45) for a caller that will run the backward: the same
  * outputs as lard_attn_kl_forward (same workspace) plus

@@ -22,7 +22,10 @@ pass also forms the row side of the gradient (dq before dloss, a float32
 itself), and the backward runs only the column side
 (``lard_attn_kl_backward_colgrad``), which adds itself to that buffer in
 place.  A second backward through the same graph (retain_graph) finds the
-buffer consumed and runs the full ``lard_attn_kl_backward``.
+buffer consumed and runs the full ``lard_attn_kl_backward``.  For float32
+inputs that need a gradient the pair is ``lard_attn_kl_forward_lse64`` /
+``lard_attn_kl_backward_lse64``, which keeps both LSEs in double between the
+passes.
 """
 
 from __future__ import annotations
@@ -87,8 +90,9 @@ class AttnKLAlignFn(torch.autograd.Function):
             _warn_slow_path(d, ss, st)
             path = kernel_path(d, ss, st)[0]
         md = _lib.mask_desc(attn_mask)
-        dq_row = None
-        if path == "throughput" and B * Hq * T > 0 and (ctx.needs_input_grad[0] or ctx.needs_input_grad[1]):
+        dq_row = lse64 = None
+        needs_grad = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
+        if path == "throughput" and B * Hq * T > 0 and needs_grad:
             dq_row = torch.empty((B, Hq, T, Ds), device=dev, dtype=torch.float32)
             ws_bytes = L.lard_attn_kl_forward_rowgrad_workspace_bytes(B, Hq, ks.shape[1], kt.shape[1], T, Ds)
             ws = _workspace(ws_bytes, dev)
@@ -97,6 +101,13 @@ class AttnKLAlignFn(torch.autograd.Function):
                 int(bool(causal)), ss, st, lse_s.data_ptr(), lse_t.data_ptr(), loss.data_ptr(), dq_row.data_ptr(),
                 ws.data_ptr(), ws_bytes, _lib.stream_of(qs))
             _lib.check(rc, "lard_attn_kl_forward_rowgrad")
+        elif path == "float32" and needs_grad:
+            lse64 = torch.empty((2, B, Hq, T), device=dev, dtype=torch.float64)
+            rc = L.lard_attn_kl_forward_lse64(
+                ctypes.byref(d[0]), ctypes.byref(d[1]), ctypes.byref(d[2]), ctypes.byref(d[3]), ctypes.byref(md),
+                int(bool(causal)), ss, st, lse_s.data_ptr(), lse_t.data_ptr(), loss.data_ptr(), lse64.data_ptr(),
+                ws.data_ptr(), ws_bytes, _lib.stream_of(qs))
+            _lib.check(rc, "lard_attn_kl_forward_lse64")
         else:
             rc = L.lard_attn_kl_forward(ctypes.byref(d[0]), ctypes.byref(d[1]), ctypes.byref(d[2]),
                                         ctypes.byref(d[3]), ctypes.byref(md), int(bool(causal)), ss, st,
@@ -107,8 +118,9 @@ class AttnKLAlignFn(torch.autograd.Function):
         saved_mask = attn_mask if attn_mask is not None else torch.empty(0, device=dev)
         ctx.has_row_grad = dq_row is not None
         ctx.row_grad_used = False
-        ctx.save_for_backward(qs, ks, lse_s, qt, kt, lse_t, saved_mask,
-                              dq_row if dq_row is not None else torch.empty(0, device=dev))
+        ctx.has_lse64 = lse64 is not None
+        extra = dq_row if dq_row is not None else lse64 if lse64 is not None else torch.empty(0, device=dev)
+        ctx.save_for_backward(qs, ks, lse_s, qt, kt, lse_t, saved_mask, extra)
         ctx.has_mask = attn_mask is not None
         ctx.causal = bool(causal)
         ctx.sm_scale_s = ss
@@ -119,17 +131,19 @@ class AttnKLAlignFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dloss):
         """integration.py:48-67: stage C and the chain rule with dloss."""
-        qs, ks, lse_s, qt, kt, lse_t, saved_mask, dq_row = ctx.saved_tensors
+        qs, ks, lse_s, qt, kt, lse_t, saved_mask, extra = ctx.saved_tensors
+        dq_row = extra if ctx.has_row_grad else None
         attn_mask = saved_mask if ctx.has_mask else None
         dloss = dloss.detach().to(torch.float32).contiguous()
         B, Hq, T, Ds = qs.shape
         self_rel = ctx.self_relation
         dev = qs.device
         L = _lib.lib()
-        ws_bytes = L.lard_attn_kl_backward_workspace_bytes(B, Hq, ks.shape[1], T, Ds, int(self_rel))
-        ws = _workspace(ws_bytes, dev)
         d = [_lib.tensor4(x) for x in (qs, ks, qt, kt)]
         md = _lib.mask_desc(attn_mask)
+        if not ctx.has_lse64:
+            ws_bytes = L.lard_attn_kl_backward_workspace_bytes(B, Hq, ks.shape[1], T, Ds, int(self_rel))
+            ws = _workspace(ws_bytes, dev)
         if ctx.has_row_grad and not ctx.row_grad_used:
             # the row side came with the forward: the column side adds itself
             # to it in place (self relation) or dq_row becomes dq
@@ -146,6 +160,14 @@ class AttnKLAlignFn(torch.autograd.Function):
             return dq_row, dk, None, None, None, None, None, None
         dk = torch.empty((B, ks.shape[1], T, Ds), device=dev, dtype=torch.float32)
         dq = None if self_rel else torch.empty((B, Hq, T, Ds), device=dev, dtype=torch.float32)
+        if ctx.has_lse64:  # float32 inputs: the forward kept its LSEs in double
+            rc = L.lard_attn_kl_backward_lse64(
+                ctypes.byref(d[0]), ctypes.byref(d[1]), lse_s.data_ptr(), ctypes.byref(d[2]), ctypes.byref(d[3]),
+                lse_t.data_ptr(), extra.data_ptr(), ctypes.byref(md), int(ctx.causal), ctx.sm_scale_s, ctx.sm_scale_t,
+                dloss.data_ptr(), int(self_rel), None if dq is None else dq.data_ptr(), dk.data_ptr(),
+                _lib.stream_of(qs))
+            _lib.check(rc, "lard_attn_kl_backward_lse64")
+            return (dk if self_rel else dq), (None if self_rel else dk), None, None, None, None, None, None
         rc = L.lard_attn_kl_backward(
             ctypes.byref(d[0]), ctypes.byref(d[1]), lse_s.data_ptr(), ctypes.byref(d[2]), ctypes.byref(d[3]),
             lse_t.data_ptr(), ctypes.byref(md), int(ctx.causal), ctx.sm_scale_s, ctx.sm_scale_t, dloss.data_ptr(),

@@ -738,7 +738,7 @@ namespace {
 template <class NeedWorkspace>
 int attn_kl_forward_impl(const lard_tensor4* qs, const lard_tensor4* ks, const lard_tensor4* qt,
                          const lard_tensor4* kt, const lard_mask* mask, int causal, float sm_scale_s,
-                         float sm_scale_t, float* lse_s_out, float* lse_t_out, float* loss_out,
+                         float sm_scale_t, float* lse_s_out, float* lse_t_out, float* loss_out, double* lse64_out,
                          NeedWorkspace need_workspace, void* stream) {
   int rc;
   if ((rc = check_pair(qs, ks, "qs", "ks")) != LARD_OK) return rc;
@@ -807,6 +807,7 @@ int attn_kl_forward_impl(const lard_tensor4* qs, const lard_tensor4* ks, const l
       g.lse_t_out = lse_t_out;
       g.row_out = w.loss.rows;
       g.r.counter = w.loss.counter;
+      g.r.lse64_out = lse64_out;
       if ((rc = hip_status(timed(LARD_KERNEL_FORWARD, st, [&] { return lard::launch_fused_fwd_f32(g, st); }),
                            "attn_kl_forward float32 launch")) != LARD_OK)
         return rc;
@@ -889,7 +890,28 @@ int lard_attn_kl_forward(const lard_tensor4* qs, const lard_tensor4* ks, const l
     return LARD_OK;
   };
   return attn_kl_forward_impl(qs, ks, qt, kt, mask, causal, sm_scale_s, sm_scale_t, lse_s_out, lse_t_out, loss_out,
-                              caller_ws, stream);
+                              nullptr, caller_ws, stream);
+}
+
+int lard_attn_kl_forward_lse64(const lard_tensor4* qs, const lard_tensor4* ks, const lard_tensor4* qt,
+                               const lard_tensor4* kt, const lard_mask* mask, int causal, float sm_scale_s,
+                               float sm_scale_t, float* lse_s_out, float* lse_t_out, float* loss_out,
+                               double* lse64_out, void* workspace, size_t workspace_bytes, void* stream) {
+  int rc;
+  if ((rc = check_pair(qs, ks, "qs", "ks")) != LARD_OK) return rc;
+  if (qs->dtype != LARD_DTYPE_F32) return fail(LARD_ERR_UNSUPPORTED, "the double LSEs are float32 inputs' only");
+  if (qs->size[0] * qs->size[1] * qs->size[2] > 0 &&
+      (lse64_out == nullptr || reinterpret_cast<uintptr_t>(lse64_out) % 8 != 0))
+    return fail(LARD_ERR_INVALID_ARGUMENT, "lse64_out must not be NULL and 8-byte aligned");
+  auto caller_ws = [&](int64_t B, int64_t Hq, int64_t T, void** ws) {
+    const size_t need = lard_attn_kl_forward_workspace_bytes(B, Hq, T);
+    if (workspace == nullptr || workspace_bytes < need)
+      return fail(LARD_ERR_INVALID_ARGUMENT, "workspace too small: need %zu bytes", need);
+    *ws = workspace;
+    return LARD_OK;
+  };
+  return attn_kl_forward_impl(qs, ks, qt, kt, mask, causal, sm_scale_s, sm_scale_t, lse_s_out, lse_t_out, loss_out,
+                              lse64_out, caller_ws, stream);
 }
 
 int lard_attn_kl_forward_noalloc(const lard_tensor4* qs, const lard_tensor4* ks, const lard_tensor4* qt,
@@ -906,7 +928,7 @@ int lard_attn_kl_forward_noalloc(const lard_tensor4* qs, const lard_tensor4* ks,
     return scratch_on(dev, ws);
   };
   return attn_kl_forward_impl(qs, ks, qt, kt, mask, causal, sm_scale_s, sm_scale_t, lse_s_out, lse_t_out, loss_out,
-                              library_ws, stream);
+                              nullptr, library_ws, stream);
 }
 
 size_t lard_attn_kl_backward_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t seq_len,
@@ -922,10 +944,16 @@ size_t lard_attn_kl_backward_workspace_bytes(int64_t batch, int64_t heads, int64
   return bytes > f64 ? bytes : f64;
 }
 
-int lard_attn_kl_backward(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s, const lard_tensor4* qt,
+}  // extern "C"
+
+namespace {
+
+// lard_attn_kl_backward; lse64 (float32 inputs only): both LSEs in double, so
+// no refine pass and no workspace.
+int attn_kl_backward_impl(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s, const lard_tensor4* qt,
                           const lard_tensor4* kt, const float* lse_t, const lard_mask* mask, int causal,
                           float sm_scale_s, float sm_scale_t, const float* dloss, int self_relation, float* dq_out,
-                          float* dk_out, void* workspace, size_t workspace_bytes, void* stream) {
+                          float* dk_out, const double* lse64, void* workspace, size_t workspace_bytes, void* stream) {
   int rc;
   if ((rc = check_two_sided(qs, ks, lse_s, qt, kt, lse_t, mask, sm_scale_s, sm_scale_t)) != LARD_OK) return rc;
   const int64_t B = qs->size[0], Hq = qs->size[1], T = qs->size[2];
@@ -984,7 +1012,9 @@ int lard_attn_kl_backward(const lard_tensor4* qs, const lard_tensor4* ks, const 
                       "attn_kl_backward dk launch");
   }
   const int dps = padded_dim(ds), dpt = padded_dim(dt);
-  if (qs->dtype == LARD_DTYPE_F32) {
+  if (lse64 != nullptr) {
+    a.lse64_in = lse64;
+  } else if (qs->dtype == LARD_DTYPE_F32) {
     // float32: refine both LSEs in double first (the stored ones are float32
     // roundings, too coarse for D = P_s - P_t of a near-identical pair)
     const size_t need = lard_attn_kl_backward_workspace_bytes(B, Hq, ks->size[1], T, ds, self_relation);
@@ -1008,6 +1038,33 @@ int lard_attn_kl_backward(const lard_tensor4* qs, const lard_tensor4* ks, const 
   a.dscale = dloss;
   return hip_status(timed(LARD_KERNEL_COL_GRAD, st, [&] { return lard::launch_col_dk(a, dps, dpt, st); }),
                     "attn_kl_backward dk launch");
+}
+
+}  // namespace
+
+extern "C" {
+
+int lard_attn_kl_backward(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s, const lard_tensor4* qt,
+                          const lard_tensor4* kt, const float* lse_t, const lard_mask* mask, int causal,
+                          float sm_scale_s, float sm_scale_t, const float* dloss, int self_relation, float* dq_out,
+                          float* dk_out, void* workspace, size_t workspace_bytes, void* stream) {
+  return attn_kl_backward_impl(qs, ks, lse_s, qt, kt, lse_t, mask, causal, sm_scale_s, sm_scale_t, dloss, self_relation,
+                               dq_out, dk_out, nullptr, workspace, workspace_bytes, stream);
+}
+
+int lard_attn_kl_backward_lse64(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s,
+                                const lard_tensor4* qt, const lard_tensor4* kt, const float* lse_t,
+                                const double* lse64, const lard_mask* mask, int causal, float sm_scale_s,
+                                float sm_scale_t, const float* dloss, int self_relation, float* dq_out, float* dk_out,
+                                void* stream) {
+  int rc;
+  if ((rc = check_pair(qs, ks, "qs", "ks")) != LARD_OK) return rc;
+  if (qs->dtype != LARD_DTYPE_F32) return fail(LARD_ERR_UNSUPPORTED, "the double LSEs are float32 inputs' only");
+  if (qs->size[0] * qs->size[1] * qs->size[2] > 0 &&
+      (lse64 == nullptr || reinterpret_cast<uintptr_t>(lse64) % 8 != 0))
+    return fail(LARD_ERR_INVALID_ARGUMENT, "lse64 must not be NULL and 8-byte aligned");
+  return attn_kl_backward_impl(qs, ks, lse_s, qt, kt, lse_t, mask, causal, sm_scale_s, sm_scale_t, dloss, self_relation,
+                               dq_out, dk_out, lse64, nullptr, 0, stream);
 }
 
 size_t lard_attn_kl_forward_rowgrad_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads,

@@ -76,7 +76,8 @@ struct RelArgs {
   // dscale is applied).
   const float* weight;
   // float32-input kernels only: the double-precision LSEs of both sides,
-  // [2][B, Hq, T] (student, then teacher).  The refine pass writes them; the
+  // [2][B, Hq, T] (student, then teacher).  The refine pass writes them (and
+  // the fused forward, when non-null); the
   // dq / dk passes read them (instead of lse_*_in) when non-null.
   double* lse64_out;
   const double* lse64_in;

@@ -39,10 +39,10 @@
 // Bound by the double units: a 16x16x4 product takes 64 cycles of a SIMD (77
 // TFLOP/s in a loop of nothing else), and the double VALU work (a score's
 // exponentials, the conversions of the operands) adds to it rather than
-// overlapping.  At B=1, H=32, n=1024, d=128, causal, a fwd+bwd takes 1042 us
-// (LSE refine 235, forward 238, dq 301, dk 334; 25.8 GFLOP of products the
-// path cannot do without would take 340) against 4630 us with VALU FMAs (two
-// conversions and 1.25 LDS reads per four of them).
+// overlapping.  At B=1, H=32, n=1024, d=128, causal, a fwd+bwd takes 821 us
+// (forward 238, dq 301, dk 330; the LSE refine of a backward without the
+// forward's double LSEs 235 more) against 4630 us with VALU FMAs (two
+// conversions and 1.25 LDS reads per four of them) and a refine pass.
 
 #include "stage_f32.h"
 
@@ -444,6 +444,10 @@ __global__ __launch_bounds__(kF32Threads, MAXD <= 128 ? 2 : 1) void f32_kernel(c
       a.lse_out[row_index] = mine_valid ? (float)ls : 0.f;
       a.dq_out[row_index] = mine_valid ? (float)lt : 0.f;  // the teacher's LSE (see launch_fused_fwd_f32)
       a.row_out[row_index] = (float)v;
+      if (a.lse64_out != nullptr) {
+        a.lse64_out[row_index] = mine_valid ? ls : 0.0;
+        a.lse64_out[rows + row_index] = mine_valid ? lt : 0.0;
+      }
     }
   } else if constexpr (MODE == MODE_KL) {
     kl += xor_lanes(kl, 16);

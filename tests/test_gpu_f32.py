@@ -166,6 +166,38 @@ def test_f32_cfg1_against_eager_pytorch(gpu_available):
                bar=max(F32_BAR, 2 * eager_grad))
 
 
+def test_f32_pair_equals_the_refining_backward(gpu_available):
+    """Autograd (double LSEs kept from the forward) against
+    lard_attn_kl_backward (which recomputes them): the same values bitwise,
+    also in a second backward of one graph."""
+    import ctypes
+
+    from linearard_amd import _lib
+    from linearard_amd.attention_KL import attn_kl_align
+
+    rng = np.random.default_rng(5)
+    B, H, T, D = 2, 3, 130, 64
+    mask = mask_to_dev(make_mask(rng, B, T, 0.2))
+    x = to_dev(randn(rng, (B, H, T, D), "f32"), "f32", requires_grad=True)
+    y = to_dev(randn(rng, (B, H, T, D), "f32"), "f32")
+    loss = attn_kl_align(x, x, y, y, attn_mask=mask, causal=True, sm_scale_s=0.1, sm_scale_t=0.1)
+    first, = torch.autograd.grad(loss, [x], retain_graph=True)
+    second, = torch.autograd.grad(loss, [x])
+    assert torch.equal(first, second)
+    L = _lib.lib()
+    lse = [torch.zeros((B, H, T), device="cuda") for _ in range(2)]  # finite: only their finiteness is used
+    dx = torch.empty_like(y)
+    nb = L.lard_attn_kl_backward_workspace_bytes(B, H, H, T, D, 1)
+    ws = torch.empty((nb,), device="cuda", dtype=torch.uint8)
+    d = [ctypes.byref(_lib.tensor4(t)) for t in (x.detach(), y)]
+    one = torch.ones((), device="cuda")
+    rc = L.lard_attn_kl_backward(d[0], d[0], lse[0].data_ptr(), d[1], d[1], lse[1].data_ptr(),
+                                 ctypes.byref(_lib.mask_desc(mask)), 1, 0.1, 0.1, one.data_ptr(), 1, None,
+                                 dx.data_ptr(), ws.data_ptr(), nb, _lib.stream_of(y))
+    assert rc == 0, L.lard_last_error()
+    assert torch.equal(first, dx)
+
+
 def test_f32_needs_f32_on_both_sides(gpu_available):
     from linearard_amd.attention_KL import attn_kl_align
 
