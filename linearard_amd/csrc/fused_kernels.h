@@ -18,29 +18,29 @@
 namespace lard {
 
 template <int DP, bool BF>
-__global__ __launch_bounds__(kStageThreads) void fused_fwd_kernel(const FusedArgs f) {
+__global__ __launch_bounds__(kStageThreads, 2) void fused_fwd_kernel(const FusedArgs f) {
   const RelArgs& a = f.r;
   constexpr int DPS = DP;  // student and teacher share the head dim and dtype on this path
   constexpr int DPT = DP;
-  constexpr int BN = 32;
+  constexpr int BN = kStageTile;
+  constexpr int kBufs = stage_bufs(DPS, DPT, false);
   constexpr int KS = DPS / 16;
   constexpr int KT = DPT / 16;
-  constexpr int SS = DPS + 8;
-  constexpr int ST = DPT + 8;
 
-  __shared__ __attribute__((aligned(16))) u16 lks[BN * SS];
-  __shared__ __attribute__((aligned(16))) u16 lkt[BN * ST];
-  __shared__ int lcol[BN];
+  __shared__ __attribute__((aligned(512))) u16 lks[kBufs][BN * DPS];
+  __shared__ __attribute__((aligned(512))) u16 lkt[kBufs][BN * DPT];
+  __shared__ unsigned lbits[kStageWindow / 32];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int w = tid >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5;
   const int l32 = lane & 31;
   const int T = a.T;
   const int nrb = (T + kStageRows - 1) / kStageRows;
-  const int rb = nrb - 1 - (int)blockIdx.x;
-  const int bh = blockIdx.y;
+  int blk, bh;
+  stage_item(blk, bh);
+  const int rb = nrb - 1 - blk;  // longest causal rows first
   const int b = bh / a.Hq;
   const int h = bh - b * a.Hq;
   const int i0w = rb * kStageRows + w * 32;
@@ -79,37 +79,43 @@ __global__ __launch_bounds__(kStageThreads) void fused_fwd_kernel(const FusedArg
   if (a.causal) nkb = min(nkb, (rb * kStageRows + kStageRows - 1) / BN + 1);
   const int wave_last_kb = a.causal ? (i0w + 31) / BN : nkb - 1;
 
-  // Key tiles go through registers: tile kb + 1 is loaded while tile kb is
-  // consumed.
-  TileRegs<BN, DPS, kStageThreads> rks;
-  TileRegs<BN, DPT, kStageThreads> rkt;
-  rks.load(ks_base, a.s.k_st, 0, T, a.s.dim, tid);
-  rkt.load(kt_base, a.t.k_st, 0, T, a.t.dim, tid);
+  // Tile ring, as in row_kernel.
+  StageCopier<DPS> cps;
+  StageCopier<DPT> cpt;
+  cps.init(ks_base, a.s.k_st, a.s.dim, w, lane);
+  cpt.init(kt_base, a.t.k_st, a.t.dim, w, lane);
+  constexpr bool kUniform = StageCopier<DPS>::TC::kUniform && StageCopier<DPT>::TC::kUniform;
+  constexpr int kPerWave = StageCopier<DPS>::TC::kRowPerWave + StageCopier<DPT>::TC::kRowPerWave;
+  auto issue_tile = [&](int kb, int buf) {
+    cps.issue(lds_addr(lks[buf]), kb * BN, T, w);
+    cpt.issue(lds_addr(lkt[buf]), kb * BN, T, w);
+  };
+  const unsigned gs = row_chunk_xor<DPS>(l32, half), gt = row_chunk_xor<DPT>(l32, half);
+  const TokenBits tok = {lbits, &a, (int64_t)b * a.mask_sb};
+  tok.fill(0, nkb * BN);
+  wait_vmcnt<0>();  // register operands landed before the ring starts
+  issue_tile(0, 0);
+  if (kBufs > 2 && nkb > 1) issue_tile(1, 1);
 
-  for (int kb = 0; kb < nkb; ++kb) {
+  int buf = 0;  // kb % kBufs
+  for (int kb = 0; kb < nkb; ++kb, buf = buf + 1 == kBufs ? 0 : buf + 1) {
     const int j0 = kb * BN;
+    if (kUniform && kBufs > 2 && kb + 1 < nkb)
+      wait_vmcnt<kPerWave>();  // tile kb + 1 in flight
+    else
+      wait_vmcnt<0>();
     __syncthreads();
-    rks.store(lks, SS, tid);
-    rkt.store(lkt, ST, tid);
-    if (kb + 1 < nkb) {
-      rks.load(ks_base, a.s.k_st, j0 + BN, T, a.s.dim, tid);
-      rkt.load(kt_base, a.t.k_st, j0 + BN, T, a.t.dim, tid);
+    if (kb > 0 && tok.starts_window(j0)) {
+      tok.fill(j0, nkb * BN);
+      __syncthreads();
     }
-    if (tid < BN) {
-      const int j = j0 + tid;
-      lcol[tid] = (j < T) && mask_at(a.mask, a.mask_kind, (int64_t)b * a.mask_sb + j);
-    }
-    __syncthreads();
+    if (kb + kBufs - 1 < nkb) issue_tile(kb + kBufs - 1, buf + kBufs - 1 >= kBufs ? buf - 1 : buf + kBufs - 1);
     if (kb > wave_last_kb) continue;
+    const unsigned cm = tok.get(j0);
 
-    f32x16 ss = (f32x16)(0.f);
-    f32x16 st = (f32x16)(0.f);
-#pragma unroll
-    for (int kk = 0; kk < KS; ++kk)
-      ss = mfma32<BF>(*reinterpret_cast<const u16x8*>(lks + l32 * SS + 16 * kk + 8 * half), fq_s[kk], ss);
-#pragma unroll
-    for (int kk = 0; kk < KT; ++kk)
-      st = mfma32<BF>(*reinterpret_cast<const u16x8*>(lkt + l32 * ST + 16 * kk + 8 * half), fq_t[kk], st);
+    f32x16 ss, st;
+    stage_scores<KS, KT, BF ? kTypesBf16 : kTypesF16>(lds_addr(lks[buf]) + gs, lds_addr(lkt[buf]) + gt, fq_s, fq_t, BF, BF,
+                                                      ss, st);
 
     float xs[16], xt[16];
     bool valid[16];
@@ -117,7 +123,7 @@ __global__ __launch_bounds__(kStageThreads) void fused_fwd_kernel(const FusedArg
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int jj = 8 * (r >> 2) + 4 * half + (r & 3);
-      valid[r] = row_valid && lcol[jj] && (!a.causal || j0 + jj <= my_i);
+      valid[r] = row_valid & ((cm >> jj) & 1u) & (!a.causal | (j0 + jj <= my_i));
       xs[r] = valid[r] ? mul_rn(ss[r], a.s.scale) : kNegInf;
       xt[r] = valid[r] ? mul_rn(st[r], a.t.scale) : kNegInf;
       mb_s = fmaxf(mb_s, xs[r]);

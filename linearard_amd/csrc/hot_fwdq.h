@@ -308,43 +308,6 @@ __device__ __forceinline__ void mask_block_q(f32x16& ss, f32x16& st, unsigned bi
 }
 
 
-// A 16-byte LDS load at a byte address.
-__device__ __forceinline__ u16x8 lds_u16x8(unsigned a) {
-  return *(__attribute__((address_space(3))) const u16x8*)(uintptr_t)a;
-}
-// Transposing operand reads (TrOffsets' pattern) with the swizzle's per-lane
-// offsets in XOR form.  The swizzle XORs the chunk index inside a row, so in
-// a 256-byte aligned tile the offset of dim block db is the lane's db = 0
-// offset with address bits 6-7 flipped by db (one base per 8-row half: for
-// D = 128 the two halves swizzle differently), while the 16-row groups and
-// sub-blocks add.  Two registers per lane instead of eight, and the constant
-// parts fold into the reads' offset field; with the offsets in VGPRs the
-// compiler no longer parks them in AGPRs and reads them back every step.
-template <int DP>
-struct TrXor {
-  unsigned base[2];  // bytes
-  __device__ __forceinline__ void init(int lane) {
-    const int g = lane >> 4, u = lane & 15;
-    int dim = 16 * (g & 1) + 4 * (u & 3);
-    if (DP < 32) dim &= DP - 1;
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int row = 8 * r + 4 * (g >> 1) + (u >> 2);
-      base[r] = 2u * ((unsigned)row_chunk_off<DP>(row, dim >> 3) + (dim & 7));
-    }
-  }
-  __device__ __forceinline__ u16x8 read(unsigned tile, int sb, int m, int db) const {
-    s16x4 v[2];
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const unsigned a = ((tile + base[r]) ^ (unsigned)(db << 6)) + (unsigned)((32 * sb + 16 * m) * DP * 2);
-      v[r] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(uintptr_t)a);
-    }
-    typedef short s16x8 __attribute__((ext_vector_type(8)));
-    const s16x8 both = __builtin_shufflevector(v[0], v[1], 0, 1, 2, 3, 4, 5, 6, 7);
-    return __builtin_bit_cast(u16x8, both);
-  }
-};
 // Lazy-maximum bound of the fused kernel: every exponential stays below it,
 // so the float16 operands (largest finite 65504) never overflow.
 constexpr float kLazySumQ = 32768.f;  // 2^15

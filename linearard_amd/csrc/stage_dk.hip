@@ -8,6 +8,14 @@ namespace lard {
 
 template <int DPS>
 static hipError_t launch_dk(const RelArgs& a, int dpt, dim3 grid, hipStream_t stream) {
+  const int types = stage_types(a, true);
+  if (dpt == DPS && types != kTypesAny) {
+    if (types == kTypesBf16)
+      hipLaunchKernelGGL((col_kernel<DPS, DPS, kTypesBf16>), grid, dim3(kStageThreads), 0, stream, a);
+    else
+      hipLaunchKernelGGL((col_kernel<DPS, DPS, kTypesF16>), grid, dim3(kStageThreads), 0, stream, a);
+    return hipGetLastError();
+  }
   switch (dpt) {
 #define X(DP, unused) \
   case DP: hipLaunchKernelGGL((col_kernel<DPS, DP>), grid, dim3(kStageThreads), 0, stream, a); break;

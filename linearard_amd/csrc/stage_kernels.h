@@ -15,53 +15,251 @@
 // DPS/DPT are the head dims padded to a multiple of 16 (D=8 runs as 16 with
 // zero padding, which adds exact zeros to every dot product).  The second
 // GEMM of stage C (dq, dk) reads its transposed operand straight from the
-// row-major tile of the first with ds_read_b64_tr_b16 (TrRowTile).
+// row-major tile of the first with ds_read_b64_tr_b16 (TrXor).
+//
+// Tiles go HBM -> LDS without registers (ring.h) into a ring of two or three
+// tiles, the others in flight while one is consumed, one barrier per tile.
+// (Staged through registers one tile ahead, with two barriers per tile, the
+// 256-wide gradient kernels had no registers left for the tile ahead and
+// waited out every load.)  The loops have no other global
+// loads, whose waits would also wait for the tiles in flight: token validity
+// comes from a bitmap in LDS, the rows' LSEs of the column kernel ride the
+// ring.
+//
+// Bound by the products' and the VALU work's issue in one or two waves per
+// SIMD.  With the ring, the operand reads ahead of the products, the
+// accumulators kept in place and XCD-contiguous heads (below), same-box: D =
+// 256 (B=1, H=16, n=4096, causal, bf16) dq 820 -> 297 us, dk 849 -> 354, the
+// one-pass forward 449 -> 369; D = 128 (B=2, Hq=16, Hkv=4 and 2, n=2048, not
+// causal, f16) LSE 80 -> 75, KL 110 -> 97, dq 293 -> 139, dk 622 -> 371; all
+// results bitwise the same.
 #pragma once
 
 #include "lard_device.h"
+#include "ring.h"
 
 namespace lard {
 
 constexpr int kStageThreads = 256;  // 4 waves
+constexpr int kStageWaves = 4;
 constexpr int kStageRows = 128;     // rows (or columns) owned per workgroup
+constexpr int kStageTile = 32;      // rows per ring tile
+// Tiles of the ring: 3, except where two fit two workgroups per CU and three
+// would not (256-wide kernels without gradient accumulators).
+constexpr int stage_bufs(int dps, int dpt, bool grad) { return !grad && dps + dpt >= 512 ? 2 : 3; }
+constexpr int kStageWindow = 32768; // tokens whose validity bits are in LDS at a time (masked calls)
 
-template <int MODE, int DPS, int DPT>
-__global__ __launch_bounds__(kStageThreads) void row_kernel(const RelArgs a) {
-  constexpr int BN = 32;
+// Input types of an instance: both sides float16, both bfloat16, or read from
+// the arguments.  The tests of the type around the products make the compiler
+// keep every accumulator twice (dq at D = 128: 144 AGPRs against 64), so equal
+// dims and types, the common case, have instances of their own.
+enum StageTypes : int { kTypesF16 = 0, kTypesBf16 = 1, kTypesAny = 2 };
+inline int stage_types(const RelArgs& a, bool two_sided) {
+  if (two_sided && a.s.bf16 != a.t.bf16) return kTypesAny;
+  return a.s.bf16 ? kTypesBf16 : kTypesF16;
+}
+
+// This workgroup's block (of gridDim.x) and head (of gridDim.y), numbered so
+// that each XCD works on a contiguous range of heads: its L2 then holds the
+// head's tiles that all its workgroups walk.  (With heads dealt round robin
+// every XCD streamed every head from beyond its L2: at D = 256, B=1, H=16,
+// n=4096 dq took 451 us against 297, dk 590 against 354.)
+__device__ __forceinline__ void stage_item(int& blk, int& head) {
+  const int item = xcd_item((int)(blockIdx.y * gridDim.x + blockIdx.x), (int)(gridDim.x * gridDim.y));
+  head = item / (int)gridDim.x;
+  blk = item - head * (int)gridDim.x;
+}
+
+// One side's tile copies: rows [row0, row0 + 32) x [0, DP) of one head into a
+// swizzled tile.  Addresses are 64-bit per lane: these kernels also serve
+// heads of 2^31 bytes and more.  Rows >= T copy row T - 1 and chunks >= dim
+// chunk 0 (their contributions are masked, or meet zero operands).
+template <int DP>
+struct StageCopier {
+  using TC = TileCopies<DP, kStageWaves, kStageTile>;
+  static constexpr int CPR = DP / 8;
+  static constexpr int NITER = (TC::kRowInst + kStageWaves - 1) / kStageWaves;
+  static constexpr int RPI = 64 * kStageWaves / CPR;  // rows from one of a wave's copies to its next
+  const u16* src;      // row 0 of the head
+  int64_t stride;      // elements
+  int64_t lane_row;    // this lane's row of the wave's first copy, elements
+  int r0;
+  unsigned c[NITER];   // this lane's chunk of each copy, bytes
+
+  __device__ __forceinline__ void init(const u16* head, int64_t row_stride, int dim, int wave, int lane) {
+    src = head;
+    stride = row_stride;
+    r0 = (64 * wave + lane) / CPR;
+    lane_row = (int64_t)r0 * row_stride;
+#pragma unroll
+    for (int i = 0; i < NITER; ++i) {
+      const int ch = ((64 * wave + lane) % CPR) ^ swz<DP>(r0 + i * RPI);
+      c[i] = ch * 8 < dim ? 16u * ch : 0u;
+    }
+  }
+  __device__ __forceinline__ void issue(unsigned tile, int row0, int T, int wave) const {
+    const bool full = row0 + kStageTile <= T;
+#pragma unroll
+    for (int i = 0; i < NITER; ++i) {
+      const int n = wave + kStageWaves * i;
+      if (TC::kRowInst % kStageWaves != 0 && n >= TC::kRowInst) break;
+      const u16* p = src + (int64_t)(row0 + i * RPI) * stride + lane_row;
+      if (!full) {
+        const int over = row0 + i * RPI + r0 - (T - 1);
+        if (over > 0) p -= (int64_t)over * stride;
+      }
+      lds_async16_at(reinterpret_cast<const char*>(p) + c[i], tile + 1024u * n);
+    }
+  }
+};
+
+// Validity bits of the 32 tokens from j0: from the bitmap, or (no mask) from T.
+struct TokenBits {
+  unsigned* bits;  // LDS, kStageWindow / 32 words
+  const RelArgs* a;
+  int64_t base;    // mask row of the sequence
+
+  // Fills the window holding token j0 with the validity of its tokens below
+  // `last` (all threads; a barrier must follow before get).
+  __device__ __forceinline__ void fill(int j0, int last) const {
+    if (a->mask == nullptr) return;
+    const int w0 = j0 / kStageWindow * kStageWindow;
+    const int end = min(last, w0 + kStageWindow);
+    for (int j = w0 + (int)threadIdx.x; j - (int)(threadIdx.x & 63) < end; j += kStageThreads) {
+      const uint64_t v = __ballot(j < a->T && mask_at(a->mask, a->mask_kind, base + j));
+      if ((threadIdx.x & 63) == 0) {
+        bits[(j - w0) / 32] = (unsigned)v;
+        bits[(j - w0) / 32 + 1] = (unsigned)(v >> 32);
+      }
+    }
+  }
+  __device__ __forceinline__ bool starts_window(int j0) const { return a->mask != nullptr && j0 % kStageWindow == 0; }
+  __device__ __forceinline__ unsigned get(int j0) const {
+    if (a->mask != nullptr) return (unsigned)__builtin_amdgcn_readfirstlane((int)bits[j0 % kStageWindow / 32]);
+    const int n = a->T - j0;
+    return n >= 32 ? ~0u : n > 0 ? (1u << n) - 1u : 0u;
+  }
+};
+
+// acc = A B over K k-steps: A the lane's row chunks at LDS byte address p (see
+// row_chunk_xor), B the register operands.  Operand reads run PD products
+// ahead and scheduling barriers keep that order: left to the scheduler, each
+// product waited for the LDS read issued right before it (about 150 cycles per
+// product instead of 32 with one wave per SIMD).
+template <int K, bool BF, int PD = 4>
+__device__ __forceinline__ void stage_dot(unsigned p, const u16x8* b, f32x16& acc) {
+  u16x8 op[K];
+#pragma unroll
+  for (int i = 0; i < PD && i < K; ++i) op[i] = lds_u16x8(p ^ (unsigned)(i << 5));
+  acc = (f32x16)(0.f);
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    if (i + PD < K) op[i + PD] = lds_u16x8(p ^ (unsigned)((i + PD) << 5));
+    acc = mfma32<BF>(op[i], b[i], acc);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// Both sides' scores.  With the types known and equal dims the two chains
+// alternate (one read-ahead window over both); otherwise one after the other.
+template <int KS, int KT, int DT>
+__device__ __forceinline__ void stage_scores(unsigned ps, unsigned pt, const u16x8* bs, const u16x8* bt, bool sbf,
+                                             bool tbf, f32x16& ss, f32x16& st) {
+  if constexpr (DT != kTypesAny && KS == KT) {
+    constexpr bool BF = DT == kTypesBf16;
+    constexpr int N = 2 * KS, PD = 4;
+    u16x8 op[N];
+    auto load = [&](int i) { op[i] = lds_u16x8(((i & 1) ? pt : ps) ^ (unsigned)((i >> 1) << 5)); };
+#pragma unroll
+    for (int i = 0; i < PD && i < N; ++i) load(i);
+    ss = (f32x16)(0.f);
+    st = (f32x16)(0.f);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      if (i + PD < N) load(i + PD);
+      if (i & 1)
+        st = mfma32<BF>(op[i], bt[i >> 1], st);
+      else
+        ss = mfma32<BF>(op[i], bs[i >> 1], ss);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+    if (sbf)
+      stage_dot<KS, true>(ps, bs, ss);
+    else
+      stage_dot<KS, false>(ps, bs, ss);
+    if (tbf)
+      stage_dot<KT, true>(pt, bt, st);
+    else
+      stage_dot<KT, false>(pt, bt, st);
+  }
+}
+
+// out[db] += (rows of the tile, transposed) x D, D cast to the input type
+// (kernel_C.py:232-253): the gradient product of one 32 x 32 block, operand
+// reads ahead as in stage_dot.
+template <int DP, bool BF, int PD = 4>
+__device__ __forceinline__ void stage_grad(const TrXor<DP>& tr, unsigned tile, const float* pd, f32x16* out) {
+  constexpr int NDB = DP >= 32 ? DP / 32 : 1, N = 2 * NDB;
+  u16x8 op[N];
+#pragma unroll
+  for (int i = 0; i < PD && i < N; ++i) op[i] = tr.read(tile, 0, i / NDB, i % NDB);
+  const u16x8 dv[2] = {to_bits8<BF>(pd), to_bits8<BF>(pd + 8)};
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if (i + PD < N) op[i + PD] = tr.read(tile, 0, (i + PD) / NDB, (i + PD) % NDB);
+    out[i % NDB] = mfma32<BF>(op[i], dv[i / NDB], out[i % NDB]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// 256-wide gradients: the accumulators (128 registers) stay in AGPRs around the
+// loop.  Left alone, the compiler keeps them in VGPRs between tiles and copies
+// all of them to AGPRs and back for every tile's products.
+template <int NDB>
+__device__ __forceinline__ void pin_agprs(f32x16* acc) {
+  if constexpr (NDB == 8) {
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) asm volatile("" : "+a"(acc[db]));
+  }
+}
+
+template <int MODE, int DPS, int DPT, int DT = kTypesAny>
+__global__ __launch_bounds__(kStageThreads, DPS <= 128 || MODE != MODE_DQ ? 2 : 1) void row_kernel(const RelArgs a) {
+  constexpr int BN = kStageTile;
   constexpr bool HAS_T = MODE != MODE_LSE;
   constexpr bool HAS_DQ = MODE == MODE_DQ;
+  constexpr int kBufs = stage_bufs(DPS, HAS_T ? DPT : 0, HAS_DQ);
   constexpr int KS = DPS / 16;
   constexpr int KT = DPT / 16;
-  constexpr int SS = DPS + 8;  // LDS row strides (elements); +8 breaks bank alignment
-  constexpr int ST = DPT + 8;
   constexpr int NDB = DPS >= 32 ? DPS / 32 : 1;  // 32-wide d blocks of dq
 
-  __shared__ __attribute__((aligned(16))) u16 lks[BN * SS];
-  __shared__ __attribute__((aligned(16))) u16 lkt[HAS_T ? BN * ST : 8];
-  __shared__ int lcol[BN];
-  __shared__ int lfull;
+  __shared__ __attribute__((aligned(512))) u16 lks[kBufs][BN * DPS];
+  __shared__ __attribute__((aligned(512))) u16 lkt[HAS_T ? kBufs : 1][HAS_T ? BN * DPT : 8];
+  __shared__ unsigned lbits[kStageWindow / 32];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int w = tid >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5;
   const int l32 = lane & 31;
   const int T = a.T;
   const int nrb = (T + kStageRows - 1) / kStageRows;
-  const int rb = nrb - 1 - (int)blockIdx.x;  // longest causal rows first
-  const int bh = blockIdx.y;
+  int blk, bh;
+  stage_item(blk, bh);
+  const int rb = nrb - 1 - blk;  // longest causal rows first
   const int b = bh / a.Hq;
   const int h = bh - b * a.Hq;
   const int i0w = rb * kStageRows + w * 32;
   const int my_i = i0w + l32;
   const bool in_range = my_i < T;
   const bool row_valid = in_range && mask_at(a.mask, a.mask_kind, (int64_t)b * a.mask_sb + my_i);
-  const bool sbf = a.s.bf16 != 0;
-  const bool tbf = a.t.bf16 != 0;
+  const bool sbf = DT == kTypesAny ? a.s.bf16 != 0 : DT == kTypesBf16;
+  const bool tbf = DT == kTypesAny ? a.t.bf16 != 0 : DT == kTypesBf16;
   if constexpr (MODE == MODE_KL) clear_counter(a);
 
   // MODE_DQ: K^T operand of the second GEMM, read transposed from lks
-  TrRowTile<DPS, SS> trk;
+  TrXor<DPS> trk;
   if constexpr (HAS_DQ) trk.init(lane);
 
   // Query fragments (B operand): lane holds q[i = l32][16kk + 8*half .. +7].
@@ -103,6 +301,7 @@ __global__ __launch_bounds__(kStageThreads) void row_kernel(const RelArgs a) {
   f32x16 dq[HAS_DQ ? NDB : 1];
 #pragma unroll
   for (int db = 0; db < (HAS_DQ ? NDB : 1); ++db) dq[db] = (f32x16)(0.f);
+  if constexpr (HAS_DQ) pin_agprs<NDB>(dq);
 
   const int hs = h / a.s.group;
   const int ht = h / a.t.group;
@@ -113,69 +312,58 @@ __global__ __launch_bounds__(kStageThreads) void row_kernel(const RelArgs a) {
   if (a.causal) nkb = min(nkb, (rb * kStageRows + kStageRows - 1) / BN + 1);
   const int wave_last_kb = a.causal ? (i0w + 31) / BN : nkb - 1;
 
-  // Key tiles go through registers: tile kb + 1 is loaded while tile kb is
-  // consumed (except where the registers would not fit: the largest dq
-  // variants load each tile right before storing it).
-  TileRegs<BN, DPS, kStageThreads> rks;
-  TileRegs<BN, HAS_T ? DPT : 16, kStageThreads> rkt;
-  constexpr bool kPrefetch = !(HAS_DQ && DPS == 256 && DPT >= 128);
-  auto load_tile = [&](int j0) {
-    rks.load(ks_base, a.s.k_st, j0, T, a.s.dim, tid);
-    if constexpr (HAS_T) rkt.load(kt_base, a.t.k_st, j0, T, a.t.dim, tid);
+  // Tile ring (see the head of this file).  Every wave issues the same number
+  // of copies per tile where the chunks divide evenly: "tile kb landed" is
+  // then "at most tile kb + 1's copies in flight".
+  StageCopier<DPS> cps;
+  StageCopier<HAS_T ? DPT : 16> cpt;
+  cps.init(ks_base, a.s.k_st, a.s.dim, w, lane);
+  if constexpr (HAS_T) cpt.init(kt_base, a.t.k_st, a.t.dim, w, lane);
+  constexpr bool kUniform = StageCopier<DPS>::TC::kUniform && (!HAS_T || StageCopier<HAS_T ? DPT : 16>::TC::kUniform);
+  constexpr int kPerWave =
+      StageCopier<DPS>::TC::kRowPerWave + (HAS_T ? StageCopier<HAS_T ? DPT : 16>::TC::kRowPerWave : 0);
+  auto issue_tile = [&](int kb, int buf) {
+    cps.issue(lds_addr(lks[buf]), kb * BN, T, w);
+    if constexpr (HAS_T) cpt.issue(lds_addr(lkt[buf]), kb * BN, T, w);
   };
-  if constexpr (kPrefetch) load_tile(0);
+  const unsigned gs = row_chunk_xor<DPS>(l32, half), gt = row_chunk_xor<HAS_T ? DPT : 16>(l32, half);
+  const TokenBits tok = {lbits, &a, (int64_t)b * a.mask_sb};
+  tok.fill(0, nkb * BN);
+  wait_vmcnt<0>();  // register operands landed before the ring starts (the compiler does not count its copies)
+  issue_tile(0, 0);
+  if (kBufs > 2 && nkb > 1) issue_tile(1, 1);
 
-  for (int kb = 0; kb < nkb; ++kb) {
+  int buf = 0;  // kb % kBufs
+  for (int kb = 0; kb < nkb; ++kb, buf = buf + 1 == kBufs ? 0 : buf + 1) {
     const int j0 = kb * BN;
-    __syncthreads();
-    if constexpr (!kPrefetch) load_tile(j0);
-    rks.store(lks, SS, tid);
-    if constexpr (HAS_T) rkt.store(lkt, ST, tid);
-    if constexpr (kPrefetch) {
-      if (kb + 1 < nkb) load_tile(j0 + BN);
+    if (kUniform && kBufs > 2 && kb + 1 < nkb)
+      wait_vmcnt<kPerWave>();  // tile kb + 1 in flight
+    else
+      wait_vmcnt<0>();
+    __syncthreads();  // tile kb landed in every wave's view, and every wave has left tile kb - 1
+    if (kb > 0 && tok.starts_window(j0)) {
+      tok.fill(j0, nkb * BN);
+      __syncthreads();
     }
-    if (tid < 64) {  // wave 0: key validity, and whether the whole tile is valid
-      bool v = true;
-      if (tid < BN) {
-        const int j = j0 + tid;
-        v = (j < T) && mask_at(a.mask, a.mask_kind, (int64_t)b * a.mask_sb + j);
-        lcol[tid] = v;
-      }
-      const int all = __all(v);
-      if (tid == 0) lfull = all;
-    }
-    __syncthreads();
+    if (kb + kBufs - 1 < nkb) issue_tile(kb + kBufs - 1, buf + kBufs - 1 >= kBufs ? buf - 1 : buf + kBufs - 1);
     if (kb > wave_last_kb) continue;
+    const unsigned tks = lds_addr(lks[buf]), tkt = lds_addr(lkt[HAS_T ? buf : 0]);
+    const unsigned pks = tks + gs, pkt = tkt + gt;  // this lane's row chunks
+    const unsigned cm = tok.get(j0);
 
     // S^T[j][i] = K[j] . Q[i]: A = K tile rows (LDS), B = query fragment.
-    f32x16 ss = (f32x16)(0.f);
-    if (sbf) {
-#pragma unroll
-      for (int kk = 0; kk < KS; ++kk)
-        ss = mfma32<true>(*reinterpret_cast<const u16x8*>(lks + l32 * SS + 16 * kk + 8 * half), fq_s[kk], ss);
-    } else {
-#pragma unroll
-      for (int kk = 0; kk < KS; ++kk)
-        ss = mfma32<false>(*reinterpret_cast<const u16x8*>(lks + l32 * SS + 16 * kk + 8 * half), fq_s[kk], ss);
-    }
-    f32x16 st = (f32x16)(0.f);
-    if constexpr (HAS_T) {
-      if (tbf) {
-#pragma unroll
-        for (int kk = 0; kk < KT; ++kk)
-          st = mfma32<true>(*reinterpret_cast<const u16x8*>(lkt + l32 * ST + 16 * kk + 8 * half), fq_t[kk], st);
-      } else {
-#pragma unroll
-        for (int kk = 0; kk < KT; ++kk)
-          st = mfma32<false>(*reinterpret_cast<const u16x8*>(lkt + l32 * ST + 16 * kk + 8 * half), fq_t[kk], st);
-      }
-    }
+    f32x16 ss, st;
+    if constexpr (HAS_T)
+      stage_scores<KS, KT, DT>(pks, pkt, fq_s, fq_t, sbf, tbf, ss, st);
+    else
+      stage_dot<KS, DT == kTypesBf16>(pks, fq_s, ss);
 
     // Per-element work in two forms: full tiles (every key valid, at or
     // below the diagonal for every row of the wave, every row of the wave
     // valid) skip the per-element validity; the values of the elements both
     // forms compute are identical.
-    const bool full = wave_ok && __builtin_amdgcn_readfirstlane(lfull) != 0 && (!a.causal || j0 + BN - 1 <= i0w);
+    const bool full = wave_ok && cm == ~0u && (!a.causal || j0 + BN - 1 <= i0w);
+    float pd[HAS_DQ ? 16 : 1];  // D
     auto elements = [&](auto full_tag) {
       constexpr bool FULL = decltype(full_tag)::value;
       // Validity of the 16 (i, j) entries this lane holds.
@@ -186,7 +374,7 @@ __global__ __launch_bounds__(kStageThreads) void row_kernel(const RelArgs a) {
           valid[r] = true;
         } else {
           const int jj = 8 * (r >> 2) + 4 * half + (r & 3);
-          valid[r] = ok && lcol[jj] && (!a.causal || j0 + jj <= my_i);
+          valid[r] = ok & ((cm >> jj) & 1u) & (!a.causal | (j0 + jj <= my_i));
         }
       }
 
@@ -220,34 +408,11 @@ __global__ __launch_bounds__(kStageThreads) void row_kernel(const RelArgs a) {
           }
         }
       } else {  // MODE_DQ
-        float pd[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           pd[r] = valid[r] ? fast_exp2((mul_rn(ss[r], a.s.scale) - lse_s) * kLog2e) -
                                  fast_exp2((mul_rn(st[r], a.t.scale) - lse_t) * kLog2e)
                            : 0.f;
-        }
-        u16x8 dv[2];  // dval.to(qs.dtype)  (kernel_C.py:233)
-        if constexpr (DPS == 256) {
-          // one element at a time: the 8-wide conversions need registers
-          // this variant (128 accumulator registers) does not have
-#pragma unroll
-          for (int r = 0; r < 16; ++r) dv[r >> 3][r & 7] = to_bits(pd[r], sbf);
-        } else if (sbf) {
-          dv[0] = to_bits8<true>(pd);
-          dv[1] = to_bits8<true>(pd + 8);
-        } else {
-          dv[0] = to_bits8<false>(pd);
-          dv[1] = to_bits8<false>(pd + 8);
-        }
-        // dq^T[d][i] += sum_j K^T[d][j] D^T[j][i]
-#pragma unroll
-        for (int m = 0; m < 2; ++m) {
-#pragma unroll
-          for (int db = 0; db < NDB; ++db) {
-            const u16x8 aop = trk.read(lks, m, db);
-            dq[db] = sbf ? mfma32<true>(aop, dv[m], dq[db]) : mfma32<false>(aop, dv[m], dq[db]);
-          }
         }
       }
     };
@@ -255,6 +420,13 @@ __global__ __launch_bounds__(kStageThreads) void row_kernel(const RelArgs a) {
       elements(Flag<true>{});
     else
       elements(Flag<false>{});
+    if constexpr (HAS_DQ) {  // dq^T[d][i] += sum_j K^T[d][j] D^T[j][i]
+      if (sbf)
+        stage_grad<DPS, true>(trk, tks, pd, dq);
+      else
+        stage_grad<DPS, false>(trk, tks, pd, dq);
+      pin_agprs<NDB>(dq);
+    }
   }
 
   const int64_t row_index = (int64_t)bh * T + my_i;
@@ -286,30 +458,28 @@ __global__ __launch_bounds__(kStageThreads) void row_kernel(const RelArgs a) {
   }
 }
 
-template <int DPS, int DPT>
-__global__ __launch_bounds__(kStageThreads) void col_kernel(const RelArgs a) {
-  constexpr int BM = 32;
+template <int DPS, int DPT, int DT = kTypesAny>
+__global__ __launch_bounds__(kStageThreads, DPS <= 128 ? 2 : 1) void col_kernel(const RelArgs a) {
+  constexpr int BM = kStageTile;
+  constexpr int kBufs = stage_bufs(DPS, DPT, true);
   constexpr int KS = DPS / 16;
   constexpr int KT = DPT / 16;
-  constexpr int SS = DPS + 8;
-  constexpr int ST = DPT + 8;
   constexpr int NDB = DPS >= 32 ? DPS / 32 : 1;
 
-  __shared__ __attribute__((aligned(16))) u16 lqs[BM * SS];
-  __shared__ __attribute__((aligned(16))) u16 lqt[BM * ST];
-  __shared__ __attribute__((aligned(16))) float llse_s[BM];
-  __shared__ __attribute__((aligned(16))) float llse_t[BM];
-  __shared__ int lok[BM];
-  __shared__ int lfull;
+  __shared__ __attribute__((aligned(512))) u16 lqs[kBufs][BM * DPS];
+  __shared__ __attribute__((aligned(512))) u16 lqt[kBufs][BM * DPT];
+  // the tile rows' LSEs, one copy per wave: student [0, 32), teacher [32, 64)
+  __shared__ __attribute__((aligned(16))) float llse[kBufs][kStageWaves][2 * BM];
+  __shared__ unsigned lbits[kStageWindow / 32];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int w = tid >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5;
   const int l32 = lane & 31;
   const int T = a.T;
-  const int cb = blockIdx.x;  // small cb = longest causal columns, launched first
-  const int bg = blockIdx.y;
+  int cb, bg;  // small cb = longest causal columns, launched first
+  stage_item(cb, bg);
   const int b = bg / a.s.hkv;
   const int g = bg - b * a.s.hkv;
   const int j0w = cb * kStageRows + w * 32;
@@ -317,11 +487,11 @@ __global__ __launch_bounds__(kStageThreads) void col_kernel(const RelArgs a) {
   const bool in_range = my_j < T;
   const bool col_valid = in_range && mask_at(a.mask, a.mask_kind, (int64_t)b * a.mask_sb + my_j);
   const bool wave_cols_ok = __all(col_valid) != 0;
-  const bool sbf = a.s.bf16 != 0;
-  const bool tbf = a.t.bf16 != 0;
+  const bool sbf = DT == kTypesAny ? a.s.bf16 != 0 : DT == kTypesBf16;
+  const bool tbf = DT == kTypesAny ? a.t.bf16 != 0 : DT == kTypesBf16;
 
   // Q^T operand of the second GEMM, read transposed from lqs
-  TrRowTile<DPS, SS> trq;
+  TrXor<DPS> trq;
   trq.init(lane);
 
   // Key fragments (B operand of S[i][j]): lane holds k[j = l32][16kk + 8*half .. +7].
@@ -338,11 +508,14 @@ __global__ __launch_bounds__(kStageThreads) void col_kernel(const RelArgs a) {
   f32x16 dk[NDB];
 #pragma unroll
   for (int db = 0; db < NDB; ++db) dk[db] = (f32x16)(0.f);
+  pin_agprs<NDB>(dk);
 
   const int nib = (T + BM - 1) / BM;
   const int ib_first = a.causal ? (cb * kStageRows) / BM : 0;
   const int wave_first_ib = a.causal ? j0w / BM : 0;
   int loaded_ht = -1;
+  const unsigned gs = row_chunk_xor<DPS>(l32, half), gt = row_chunk_xor<DPT>(l32, half);
+  const TokenBits tok = {lbits, &a, (int64_t)b * a.mask_sb};
 
   for (int hh = 0; hh < a.s.group; ++hh) {
     const int h = g * a.s.group + hh;
@@ -360,118 +533,73 @@ __global__ __launch_bounds__(kStageThreads) void col_kernel(const RelArgs a) {
     const u16* qs_base = a.s.q + (int64_t)b * a.s.q_sb + (int64_t)h * a.s.q_sh;
     const u16* qt_base = a.t.q + (int64_t)b * a.t.q_sb + (int64_t)h * a.t.q_sh;
 
-    // Query tiles and their rows' validity and LSEs go through registers:
-    // tile ib + 1 is loaded while tile ib is consumed (except where the
-    // registers would not fit: the largest variants load each tile right
-    // before storing it).
-    constexpr bool kPrefetch = !(DPS == 256 && DPT >= 128);
-    TileRegs<BM, DPS, kStageThreads> rqs;
-    TileRegs<BM, DPT, kStageThreads> rqt;
-    float nls = 0.f, nlt = 0.f;
-    bool nrv = false;
-    auto load_tile = [&](int i0) {
-      rqs.load(qs_base, a.s.q_st, i0, T, a.s.dim, tid);
-      rqt.load(qt_base, a.t.q_st, i0, T, a.t.dim, tid);
-      if (tid < BM) {
-        const int i = i0 + tid;
-        nrv = false;
-        nls = nlt = 0.f;
-        if (i < T) {
-          nrv = mask_at(a.mask, a.mask_kind, (int64_t)b * a.mask_sb + i);
-          nls = a.lse_s_in[bh * T + i];
-          nlt = a.lse_t_in[bh * T + i];
-        }
-      }
+    // Tile ring, as in row_kernel; the LSEs ride along (4 bytes per lane:
+    // lanes 0-31 student rows, 32-63 teacher rows, rows >= T row T - 1's).
+    StageCopier<DPS> cps;
+    StageCopier<DPT> cpt;
+    cps.init(qs_base, a.s.q_st, a.s.dim, w, lane);
+    cpt.init(qt_base, a.t.q_st, a.t.dim, w, lane);
+    constexpr bool kUniform = StageCopier<DPS>::TC::kUniform && StageCopier<DPT>::TC::kUniform;
+    constexpr int kPerWave = StageCopier<DPS>::TC::kRowPerWave + StageCopier<DPT>::TC::kRowPerWave + 1;
+    const float* lse_src = (half ? a.lse_t_in : a.lse_s_in) + bh * T;
+    auto issue_tile = [&](int ib, int buf) {
+      cps.issue(lds_addr(lqs[buf]), ib * BM, T, w);
+      cpt.issue(lds_addr(lqt[buf]), ib * BM, T, w);
+      lds_async4_at(lse_src + min(ib * BM + l32, T - 1), lds_addr(llse[buf][w]));
     };
-    if constexpr (kPrefetch) {
-      if (ib_first < nib) load_tile(ib_first * BM);
+    if (ib_first < nib) {
+      __syncthreads();  // every wave is done with the previous head's ring
+      tok.fill(ib_first * BM, nib * BM);
+      wait_vmcnt<0>();  // register operands landed before the ring starts
+      issue_tile(ib_first, 0);
+      if (ib_first + 1 < nib) issue_tile(ib_first + 1, 1);
     }
 
-    for (int ib = ib_first; ib < nib; ++ib) {
+    int buf = 0;  // (ib - ib_first) % kBufs
+    for (int ib = ib_first; ib < nib; ++ib, buf = buf + 1 == kBufs ? 0 : buf + 1) {
       const int i0 = ib * BM;
+      if (kUniform && ib + 1 < nib)
+        wait_vmcnt<kPerWave>();
+      else
+        wait_vmcnt<0>();
       __syncthreads();
-      if constexpr (!kPrefetch) load_tile(i0);
-      rqs.store(lqs, SS, tid);
-      rqt.store(lqt, ST, tid);
-      const float ls = nls, lt = nlt;
-      const bool rv = nrv;
-      if constexpr (kPrefetch) {
-        if (ib + 1 < nib) load_tile(i0 + BM);
+      if (ib > ib_first && tok.starts_window(i0)) {
+        tok.fill(i0, nib * BM);
+        __syncthreads();
       }
-      if (tid < 64) {  // wave 0: row validity and LSEs, and whether every row is valid
-        bool v = true;
-        if (tid < BM) {
-          v = rv && (ls != kNegInf) && (lt != kNegInf);
-          lok[tid] = v;
-          llse_s[tid] = (ls == kNegInf) ? 0.f : ls;
-          llse_t[tid] = (lt == kNegInf) ? 0.f : lt;
-        }
-        const int all = __all(v);
-        if (tid == 0) lfull = all;
-      }
-      __syncthreads();
+      if (ib + kBufs - 1 < nib) issue_tile(ib + kBufs - 1, buf + kBufs - 1 >= kBufs ? buf - 1 : buf + kBufs - 1);
       if (ib < wave_first_ib) continue;
+      const unsigned tqs = lds_addr(lqs[buf]);
+      const unsigned pqs = tqs + gs, pqt = lds_addr(lqt[buf]) + gt;  // this lane's row chunks
+      const float* const lse = llse[buf][w];
+      // rows in the valid set: valid token, both LSEs finite (kernel_C.py:155-161)
+      const uint64_t fin = __ballot(lse[lane] != kNegInf);
+      const unsigned rm = tok.get(i0) & (unsigned)fin & (unsigned)(fin >> 32);
 
       // S[i][j] = Q[i] . K[j]: A = query tile rows (LDS), B = key fragment.
-      f32x16 ss = (f32x16)(0.f);
-      f32x16 st = (f32x16)(0.f);
-      if (sbf) {
-#pragma unroll
-        for (int kk = 0; kk < KS; ++kk)
-          ss = mfma32<true>(*reinterpret_cast<const u16x8*>(lqs + l32 * SS + 16 * kk + 8 * half), fk_s[kk], ss);
-      } else {
-#pragma unroll
-        for (int kk = 0; kk < KS; ++kk)
-          ss = mfma32<false>(*reinterpret_cast<const u16x8*>(lqs + l32 * SS + 16 * kk + 8 * half), fk_s[kk], ss);
-      }
-      if (tbf) {
-#pragma unroll
-        for (int kk = 0; kk < KT; ++kk)
-          st = mfma32<true>(*reinterpret_cast<const u16x8*>(lqt + l32 * ST + 16 * kk + 8 * half), fk_t[kk], st);
-      } else {
-#pragma unroll
-        for (int kk = 0; kk < KT; ++kk)
-          st = mfma32<false>(*reinterpret_cast<const u16x8*>(lqt + l32 * ST + 16 * kk + 8 * half), fk_t[kk], st);
-      }
+      f32x16 ss, st;
+      stage_scores<KS, KT, DT>(pqs, pqt, fk_s, fk_t, sbf, tbf, ss, st);
 
       // Per-element work in two forms: full tiles (every row of the tile and
       // every column of the wave valid, the whole tile at or below the
       // diagonal) skip the per-element validity; the values of the elements
       // both forms compute are identical.
-      const bool full =
-          wave_cols_ok && __builtin_amdgcn_readfirstlane(lfull) != 0 && (!a.causal || j0w + 31 <= i0);
+      const bool full = wave_cols_ok && rm == ~0u && (!a.causal || j0w + 31 <= i0);
+      float pd[16];  // D
       auto elements = [&](auto full_tag) {
         constexpr bool FULL = decltype(full_tag)::value;
-        float pd[16];
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
           const int ii0 = 8 * r4 + 4 * half;
-          const f32x4 ls4 = *reinterpret_cast<const f32x4*>(llse_s + ii0);
-          const f32x4 lt4 = *reinterpret_cast<const f32x4*>(llse_t + ii0);
+          const f32x4 ls4 = *reinterpret_cast<const f32x4*>(lse + ii0);
+          const f32x4 lt4 = *reinterpret_cast<const f32x4*>(lse + BM + ii0);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int r = 4 * r4 + e;
-            const bool v = FULL || (lok[ii0 + e] && col_valid && (!a.causal || my_j <= i0 + ii0 + e));
+            const bool v = FULL || (((rm >> (ii0 + e)) & 1u) & col_valid & (!a.causal | (my_j <= i0 + ii0 + e)));
             pd[r] = v ? fast_exp2((mul_rn(ss[r], a.s.scale) - ls4[e]) * kLog2e) -
                             fast_exp2((mul_rn(st[r], a.t.scale) - lt4[e]) * kLog2e)
                       : 0.f;
-          }
-        }
-        u16x8 dv[2];  // kernel_C.py:233
-        if (sbf) {
-          dv[0] = to_bits8<true>(pd);
-          dv[1] = to_bits8<true>(pd + 8);
-        } else {
-          dv[0] = to_bits8<false>(pd);
-          dv[1] = to_bits8<false>(pd + 8);
-        }
-        // dk^T[d][j] += sum_i Q^T[d][i] D[i][j]
-#pragma unroll
-        for (int m = 0; m < 2; ++m) {
-#pragma unroll
-          for (int db = 0; db < NDB; ++db) {
-            const u16x8 aop = trq.read(lqs, m, db);
-            dk[db] = sbf ? mfma32<true>(aop, dv[m], dk[db]) : mfma32<false>(aop, dv[m], dk[db]);
           }
         }
       };
@@ -479,6 +607,12 @@ __global__ __launch_bounds__(kStageThreads) void col_kernel(const RelArgs a) {
         elements(Flag<true>{});
       else
         elements(Flag<false>{});
+      // dk^T[d][j] += sum_i Q^T[d][i] D[i][j]
+      if (sbf)
+        stage_grad<DPS, true>(trq, tqs, pd, dk);
+      else
+        stage_grad<DPS, false>(trq, tqs, pd, dk);
+      pin_agprs<NDB>(dk);
     }
   }
 

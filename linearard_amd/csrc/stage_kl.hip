@@ -7,6 +7,14 @@ namespace lard {
 
 template <int DPS>
 static hipError_t launch_kl(const RelArgs& a, int dpt, dim3 grid, hipStream_t stream) {
+  const int types = stage_types(a, true);
+  if (dpt == DPS && types != kTypesAny) {
+    if (types == kTypesBf16)
+      hipLaunchKernelGGL((row_kernel<MODE_KL, DPS, DPS, kTypesBf16>), grid, dim3(kStageThreads), 0, stream, a);
+    else
+      hipLaunchKernelGGL((row_kernel<MODE_KL, DPS, DPS, kTypesF16>), grid, dim3(kStageThreads), 0, stream, a);
+    return hipGetLastError();
+  }
   switch (dpt) {
 #define X(DP, unused) \
   case DP: hipLaunchKernelGGL((row_kernel<MODE_KL, DPS, DP>), grid, dim3(kStageThreads), 0, stream, a); break;

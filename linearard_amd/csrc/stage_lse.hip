@@ -10,7 +10,12 @@ hipError_t launch_row_lse(const RelArgs& a, int dps, hipStream_t stream) {
   const dim3 grid((a.T + kStageRows - 1) / kStageRows, a.B * a.Hq);
   switch (dps) {
 #define X(DP, unused) \
-  case DP: hipLaunchKernelGGL((row_kernel<MODE_LSE, DP, 16>), grid, dim3(kStageThreads), 0, stream, a); break;
+  case DP:                                                                                                        \
+    if (stage_types(a, false) == kTypesBf16)                                                                      \
+      hipLaunchKernelGGL((row_kernel<MODE_LSE, DP, 16, kTypesBf16>), grid, dim3(kStageThreads), 0, stream, a);    \
+    else                                                                                                          \
+      hipLaunchKernelGGL((row_kernel<MODE_LSE, DP, 16, kTypesF16>), grid, dim3(kStageThreads), 0, stream, a);     \
+    break;
     LARD_DP_CASES(X, 0)
 #undef X
     default: return hipErrorInvalidValue;
