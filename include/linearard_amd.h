@@ -117,6 +117,20 @@ int lard_kl_backward(const lard_tensor4* qs, const lard_tensor4* ks, const float
                      const lard_mask* mask, int causal, float sm_scale_s, float sm_scale_t,
                      float* dq_out, float* dk_out, void* stream);
 
+/* lard_kl_backward with scratch: when the student has fewer key than query
+ * heads and the key blocks alone would leave CUs idle, each block's dk sum is
+ * cut into parts (query heads, ranges of query tiles) that run as workgroups
+ * of their own and are added up in a fixed order.  workspace: 16-byte aligned,
+ * lard_kl_backward_workspace_bytes(...) bytes (0 where nothing is cut; a
+ * smaller or NULL workspace is accepted and runs uncut). */
+size_t lard_kl_backward_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t seq_len,
+                                        int64_t head_dim);
+int lard_kl_backward_ws(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s,
+                     const lard_tensor4* qt, const lard_tensor4* kt, const float* lse_t,
+                     const lard_mask* mask, int causal, float sm_scale_s, float sm_scale_t,
+                     float* dq_out, float* dk_out, void* workspace,
+                        size_t workspace_bytes, void* stream);
+
 /* Kernels of the autograd calls (lard_attn_kl_forward / _backward), by operands. */
 #define LARD_PATH_THROUGHPUT 0     /* the throughput kernels: one-pass forward (with the row-side gradient), column backward */
 #define LARD_PATH_FUSED_FORWARD 1  /* one-pass forward, stage-kernel backward (several times slower) */
@@ -178,9 +192,10 @@ int lard_attn_kl_forward_noalloc(const lard_tensor4* qs, const lard_tensor4* ks,
                                  void* stream);
 
 /* Workspace needed by lard_attn_kl_backward (bytes): one validity byte per
- * token and two log2-domain row normalisers per query row.  kv_heads,
- * head_dim and self_relation do not change the size; they are kept so the
- * call describes the whole problem. */
+ * token and two log2-domain row normalisers per query row, and with kv_heads
+ * < heads on a small grid the parts of the dk sums (as
+ * lard_kl_backward_ws).  self_relation does not change the size; it is kept so
+ * the call describes the whole problem. */
 size_t lard_attn_kl_backward_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t seq_len,
                                              int64_t head_dim, int self_relation);
 

@@ -31,8 +31,13 @@ def kl_backward(qs, ks, lse_s, qt, kt, lse_t, attn_mask=None, causal=True, sm_sc
     dk = torch.empty((B, ks.shape[1], T, Ds), device=qs.device, dtype=torch.float32)
     d = [_lib.tensor4(x) for x in (qs, ks, qt, kt)]
     md = _lib.mask_desc(attn_mask)
-    rc = _lib.lib().lard_kl_backward(ctypes.byref(d[0]), ctypes.byref(d[1]), lse_s.data_ptr(), ctypes.byref(d[2]),
-                                     ctypes.byref(d[3]), lse_t.data_ptr(), ctypes.byref(md), int(bool(causal)),
-                                     sm_scale_s, sm_scale_t, dq.data_ptr(), dk.data_ptr(), _lib.stream_of(qs))
-    _lib.check(rc, "lard_kl_backward")
+    L = _lib.lib()
+    # scratch of the dk sums (grouped queries on a small grid; 0 bytes elsewhere)
+    ws_bytes = L.lard_kl_backward_workspace_bytes(B, Hq, ks.shape[1], T, Ds) if qs.dtype != torch.float32 else 0
+    ws = torch.empty((ws_bytes,), device=qs.device, dtype=torch.uint8) if ws_bytes > 0 else None
+    rc = L.lard_kl_backward_ws(ctypes.byref(d[0]), ctypes.byref(d[1]), lse_s.data_ptr(), ctypes.byref(d[2]),
+                               ctypes.byref(d[3]), lse_t.data_ptr(), ctypes.byref(md), int(bool(causal)),
+                               sm_scale_s, sm_scale_t, dq.data_ptr(), dk.data_ptr(),
+                               None if ws is None else ws.data_ptr(), ws_bytes, _lib.stream_of(qs))
+    _lib.check(rc, "lard_kl_backward_ws")
     return dq, dk

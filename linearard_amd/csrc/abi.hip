@@ -5,6 +5,7 @@
 // returns, plus the alignment rules of the 16-byte vector loads.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <cstdarg>
@@ -367,9 +368,33 @@ struct BwdWs {
   int* first2;
   float* nl_s;
   float* nl_t;
+  float* dk_part;  // null unless the dk sums are cut (dk_cut)
 };
 
-BwdWs bwd_layout(void* base, int64_t B, int64_t Hq, int64_t T, size_t* bytes) {
+// How a grouped-query dk sum is cut (RelArgs::dk_part): `split` ranges of
+// query tiles times the group's heads, 0 for one workgroup per key block.
+// rows: key rows per workgroup.  One workgroup per key block sums its whole
+// group (4 heads of 24 tiles on 48 of 256 CUs: 149 us of a 239 us fwd+bwd at
+// B=2, Hq=16, Hkv=4, n=1531, d=64), so a grid below one workgroup per CU is
+// cut by heads, and by query tiles (of 64, at least 4 each) until there are
+// two per CU.  Larger grids keep the sum in registers: the parts cost a write
+// and a read of group * split float32 copies of dk (at most 256 * 8 key blocks
+// of them, 256 MB at d = 128).
+int dk_cut(int64_t B, int64_t Hq, int64_t Hkv, int64_t T, int64_t rows) {
+  if (Hkv <= 0 || Hq <= Hkv || T <= 0) return 0;
+  const int64_t wgs = (T + rows - 1) / rows * B * Hkv;
+  if (wgs >= 256) return 0;
+  int64_t split = 512 / (wgs * (Hq / Hkv));
+  const int64_t most = (T + 255) / 256;
+  if (split > most) split = most;
+  return (int)(split < 1 ? 1 : split > 8 ? 8 : split);
+}
+
+int64_t dk_part_floats(int64_t B, int64_t Hq, int64_t Hkv, int64_t T, int64_t D, int64_t rows) {
+  return (int64_t)dk_cut(B, Hq, Hkv, T, rows) * B * Hq * T * D;
+}
+
+BwdWs bwd_layout(void* base, int64_t B, int64_t Hq, int64_t T, size_t* bytes, int64_t part_floats = 0) {
   Carver c(base);
   BwdWs w;
   const int64_t Tp = padded_len(T);
@@ -377,8 +402,20 @@ BwdWs bwd_layout(void* base, int64_t B, int64_t Hq, int64_t T, size_t* bytes) {
   w.first2 = c.take<int>(2 * B);
   w.nl_s = c.take<float>(B * Hq * Tp);
   w.nl_t = c.take<float>(B * Hq * Tp);
+  w.dk_part = part_floats > 0 ? c.take<float>(part_floats) : nullptr;
   if (bytes != nullptr) *bytes = c.bytes();
   return w;
+}
+
+// The stage kernels' dk sums in parts, when they are cut and `workspace` (16-byte
+// aligned) holds them.
+void cut_stage_dk(lard::RelArgs& a, void* workspace, size_t workspace_bytes) {
+  const int64_t floats = dk_part_floats(a.B, a.Hq, a.s.hkv, a.T, a.s.dim, lard::kStageRows);
+  if (floats == 0 || workspace == nullptr || workspace_bytes < (size_t)floats * 4 ||
+      reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
+    return;
+  a.dk_part = static_cast<float*>(workspace);
+  a.dk_split = dk_cut(a.B, a.Hq, a.s.hkv, a.T, lard::kStageRows);
 }
 
 // Opt-in launch timing (lard_timing_*): event pairs recorded around the
@@ -696,9 +733,16 @@ int lard_kl_forward(const lard_tensor4* qs, const lard_tensor4* ks, const float*
   return hip_status(lard::launch_reduce_sum(nullptr, 0, nullptr, nullptr, loss_out, st), "kl_forward reduce launch");
 }
 
-int lard_kl_backward(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s, const lard_tensor4* qt,
+size_t lard_kl_backward_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t seq_len,
+                                        int64_t head_dim) {
+  if (batch <= 0 || heads <= 0 || seq_len <= 0 || head_dim <= 0) return 0;
+  return (size_t)dk_part_floats(batch, heads, kv_heads, seq_len, head_dim, lard::kStageRows) * sizeof(float);
+}
+
+int lard_kl_backward_ws(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s, const lard_tensor4* qt,
                      const lard_tensor4* kt, const float* lse_t, const lard_mask* mask, int causal, float sm_scale_s,
-                     float sm_scale_t, float* dq_out, float* dk_out, void* stream) {
+                     float sm_scale_t, float* dq_out, float* dk_out, void* workspace, size_t workspace_bytes,
+                        void* stream) {
   int rc;
   if ((rc = check_two_sided(qs, ks, lse_s, qt, kt, lse_t, mask, sm_scale_s, sm_scale_t)) != LARD_OK) return rc;
   const int64_t B = qs->size[0], Hq = qs->size[1], T = qs->size[2];
@@ -717,8 +761,18 @@ int lard_kl_backward(const lard_tensor4* qs, const lard_tensor4* ks, const float
   if ((rc = hip_status(timed(LARD_KERNEL_ROW_GRAD, st, [&] { return lard::launch_row_dq(a, dps, dpt, st); }),
                        "kl_backward dq launch")) != LARD_OK)
     return rc;
-  return hip_status(timed(LARD_KERNEL_COL_GRAD, st, [&] { return lard::launch_col_dk(a, dps, dpt, st); }),
-                    "kl_backward dk launch");
+  if (qs->dtype != LARD_DTYPE_F32) cut_stage_dk(a, workspace, workspace_bytes);
+  if ((rc = hip_status(timed(LARD_KERNEL_COL_GRAD, st, [&] { return lard::launch_col_dk(a, dps, dpt, st); }),
+                       "kl_backward dk launch")) != LARD_OK)
+    return rc;
+  return hip_status(lard::launch_finish_grads(nullptr, 0, nullptr, a, st), "kl_backward dk sum launch");
+}
+
+int lard_kl_backward(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s, const lard_tensor4* qt,
+                     const lard_tensor4* kt, const float* lse_t, const lard_mask* mask, int causal, float sm_scale_s,
+                     float sm_scale_t, float* dq_out, float* dk_out, void* stream) {
+  return lard_kl_backward_ws(qs, ks, lse_s, qt, kt, lse_t, mask, causal, sm_scale_s, sm_scale_t, dq_out, dk_out, nullptr,
+                             0, stream);
 }
 
 size_t lard_attn_kl_forward_workspace_bytes(int64_t batch, int64_t heads, int64_t seq_len) {
@@ -934,14 +988,16 @@ int lard_attn_kl_forward_noalloc(const lard_tensor4* qs, const lard_tensor4* ks,
 size_t lard_attn_kl_backward_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t seq_len,
                                              int64_t head_dim, int self_relation) {
   if (batch <= 0 || heads <= 0 || seq_len <= 0) return 0;
-  (void)kv_heads;
-  (void)head_dim;
   (void)self_relation;
+  // grouped queries: the parts of the dk sums, of the throughput kernels
+  // (with the rest) or of the stage kernels (alone)
   size_t bytes = 0;
-  bwd_layout(nullptr, batch, heads, seq_len, &bytes);
+  bwd_layout(nullptr, batch, heads, seq_len, &bytes,
+             dk_part_floats(batch, heads, kv_heads, seq_len, head_dim, lard::kRows));
+  const size_t stage = align256((size_t)dk_part_floats(batch, heads, kv_heads, seq_len, head_dim, lard::kStageRows) * 4);
   // float32 inputs: both sides' LSEs in double (the refine pass)
   const size_t f64 = align256((size_t)(2 * batch * heads * seq_len) * sizeof(double));
-  return bytes > f64 ? bytes : f64;
+  return std::max(bytes, std::max(stage, f64));
 }
 
 }  // extern "C"
@@ -984,7 +1040,8 @@ int attn_kl_backward_impl(const lard_tensor4* qs, const lard_tensor4* ks, const 
       return fail(LARD_ERR_INVALID_ARGUMENT, "workspace too small: need %zu bytes", need);
     if ((rc = check_blocks(B, Hq, T)) != LARD_OK) return rc;
     const int Tp = (int)padded_len(T);
-    const BwdWs w = bwd_layout(workspace, B, Hq, T, nullptr);
+    const int64_t parts = dk_part_floats(B, Hq, ks->size[1], T, ds, lard::kRows);
+    const BwdWs w = bwd_layout(workspace, B, Hq, T, nullptr, parts);
     if ((rc = hip_status(lard::launch_token_prep(lard::token_prep(a, Tp, w.tok_ok, w.first2, nullptr), (int)B, st),
                          "attn_kl_backward token prep launch")) != LARD_OK)
       return rc;
@@ -1008,8 +1065,12 @@ int attn_kl_backward_impl(const lard_tensor4* qs, const lard_tensor4* ks, const 
     f.r.dk_out = dk_out;
     f.r.dk_add = self_relation ? dk_out : nullptr;
     f.r.dscale = dloss;
-    return hip_status(timed(LARD_KERNEL_COL_GRAD, st, [&] { return lard::launch_hot_bwd(f, padded_dim(ds), bf, st); }),
-                      "attn_kl_backward dk launch");
+    f.r.dk_part = w.dk_part;
+    f.r.dk_split = dk_cut(B, Hq, ks->size[1], T, lard::kRows);
+    if ((rc = hip_status(timed(LARD_KERNEL_COL_GRAD, st, [&] { return lard::launch_hot_bwd(f, padded_dim(ds), bf, st); }),
+                         "attn_kl_backward dk launch")) != LARD_OK)
+      return rc;
+    return hip_status(lard::launch_finish_grads(nullptr, 0, nullptr, f.r, st), "attn_kl_backward dk sum launch");
   }
   const int dps = padded_dim(ds), dpt = padded_dim(dt);
   if (lse64 != nullptr) {
@@ -1036,8 +1097,12 @@ int attn_kl_backward_impl(const lard_tensor4* qs, const lard_tensor4* ks, const 
   a.dk_out = dk_out;
   a.dk_add = self_relation ? dk_out : nullptr;
   a.dscale = dloss;
-  return hip_status(timed(LARD_KERNEL_COL_GRAD, st, [&] { return lard::launch_col_dk(a, dps, dpt, st); }),
-                    "attn_kl_backward dk launch");
+  // these shapes need no workspace: without one the dk sums are not cut
+  if (qs->dtype != LARD_DTYPE_F32) cut_stage_dk(a, workspace, workspace_bytes);
+  if ((rc = hip_status(timed(LARD_KERNEL_COL_GRAD, st, [&] { return lard::launch_col_dk(a, dps, dpt, st); }),
+                       "attn_kl_backward dk launch")) != LARD_OK)
+    return rc;
+  return hip_status(lard::launch_finish_grads(nullptr, 0, nullptr, a, st), "attn_kl_backward dk sum launch");
 }
 
 }  // namespace
@@ -1160,8 +1225,10 @@ int lard_attn_kl_backward_colgrad(const lard_tensor4* qs, const lard_tensor4* ks
   if ((rc = check_blocks(B, Hq, T)) != LARD_OK) return rc;
   const hipStream_t st = static_cast<hipStream_t>(stream);
   const int Tp = (int)padded_len(T);
-  const BwdWs w = bwd_layout(workspace, B, Hq, T, nullptr);
+  const BwdWs w = bwd_layout(workspace, B, Hq, T, nullptr, dk_part_floats(B, Hq, ks->size[1], T, ds, lard::kRows));
   lard::HotArgs f{};
+  f.r.dk_part = w.dk_part;
+  f.r.dk_split = dk_cut(B, Hq, ks->size[1], T, lard::kRows);
   fill_side(f.r.s, qs, ks, Hq, sm_scale_s);
   fill_side(f.r.t, qt, kt, Hq, sm_scale_t);
   fill_common(f.r, B, Hq, T, mask, causal);
@@ -1184,8 +1251,8 @@ int lard_attn_kl_backward_colgrad(const lard_tensor4* qs, const lard_tensor4* ks
                        "attn_kl_backward_colgrad dk launch")) != LARD_OK)
     return rc;
   if (self_relation) return ok();
-  return hip_status(lard::launch_scale_inplace(dq_row, B * Hq * T * qs->size[3], dloss, st),
-                    "attn_kl_backward_colgrad dq scale launch");
+  return hip_status(lard::launch_finish_grads(dq_row, B * Hq * T * qs->size[3], dloss, f.r, st),
+                    "attn_kl_backward_colgrad finish launch");
 }
 
 size_t lard_attn_kl_batched_workspace_bytes(const lard_relation* rels, int nrel) {

@@ -178,7 +178,7 @@ hipError_t launch_hot_dq(const HotArgs& f, int dp, bool bf16, hipStream_t stream
 }
 
 hipError_t launch_hot_bwd(const HotArgs& f, int dp, bool bf16, hipStream_t stream) {
-  const int n = row_blocks(f.r, f.r.s.hkv);
+  const int n = bwd_items(f);
   return bf16 ? hot_bwd_kernel_dispatch<true>(f, dp, n, stream) : hot_bwd_kernel_dispatch<false>(f, dp, n, stream);
 }
 

@@ -779,8 +779,13 @@ __device__ __forceinline__ void hot_bwd_body(const HotArgs& f, int item) {
   const int l32 = lane & 31;
   const int T = a.T;
   const int ncb = (T + kRows - 1) / kRows;
-  const int bg = item / ncb;
-  const int cb = item - bg * ncb;  // small cb = longest causal columns first
+  const int bgp = item / ncb;
+  const int cb = item - bgp * ncb;  // small cb = longest causal columns first
+  // the part of this key block's sum (RelArgs::dk_part), or all of it
+  const int split = a.dk_part != nullptr ? a.dk_split : 1, parts = dk_parts(a);
+  const int bg = bgp / parts;
+  const int part = bgp - bg * parts;
+  const int part_h = part / split, part_s = part - part_h * split;
   const int b = bg / a.s.hkv;
   const int g = bg - b * a.s.hkv;
   const int j0w = cb * kRows + w * 32;
@@ -808,8 +813,10 @@ __device__ __forceinline__ void hot_bwd_body(const HotArgs& f, int item) {
   // Query tiles run from the last one down to this block's diagonal: all
   // workgroups in flight then read the same tile at the same time (one L2
   // fill serves the XCD), instead of each starting at its own diagonal.
-  const int ntiles = causal ? ntile_all - (cb * kRows) / kTile : ntile_all;
-  auto tile_of = [&](int it) { return ntile_all - 1 - it; };
+  const int ntiles_sum = causal ? ntile_all - (cb * kRows) / kTile : ntile_all;
+  const int tile0 = ntiles_sum * part_s / split;  // this part's tiles of the stream
+  const int ntiles = ntiles_sum * (part_s + 1) / split - tile0;
+  auto tile_of = [&](int it) { return ntile_all - 1 - tile0 - it; };
   RowCopier<DP, kWaves> cp_s, cp_t;
   cp_s.init((int)a.s.q_st, a.s.dim, w, lane);
   cp_t.init((int)a.t.q_st, a.t.dim, w, lane);
@@ -824,7 +831,8 @@ __device__ __forceinline__ void hot_bwd_body(const HotArgs& f, int item) {
   tro.init(lane);
   int loaded_ht = -1;
 
-  for (int hh = 0; hh < a.s.group; ++hh) {
+  const int hh_end = a.dk_part != nullptr ? part_h + 1 : a.s.group;
+  for (int hh = part_h; hh < hh_end; ++hh) {
     const int h = g * a.s.group + hh;
     const int ht = h / a.t.group;
     if (ht != loaded_ht) {
@@ -929,8 +937,9 @@ __device__ __forceinline__ void hot_bwd_body(const HotArgs& f, int item) {
   }
 
   if (in_range) {
-    const int64_t off = ((int64_t)bg * T + my_j) * a.s.dim;
-    float* out = a.dk_out + off;
+    const bool whole = a.dk_part == nullptr;
+    const int64_t off = ((int64_t)bgp * T + my_j) * a.s.dim;  // bgp == bg when whole
+    float* out = (whole ? a.dk_out : a.dk_part) + off;
     const float fs = a.s.scale;
     const float mult = (a.dscale != nullptr ? *a.dscale : 1.f) * (a.weight != nullptr ? *a.weight : 1.f);
 #pragma unroll
@@ -941,8 +950,8 @@ __device__ __forceinline__ void hot_bwd_body(const HotArgs& f, int item) {
         if (d0 < a.s.dim) {
           f32x4 v = {dk[db][4 * gq] * fs, dk[db][4 * gq + 1] * fs, dk[db][4 * gq + 2] * fs, dk[db][4 * gq + 3] * fs};
           if (!col_valid) v = (f32x4)(0.f);  // masked key columns get no gradient (kernel_C.py:252-253)
-          if (a.dk_add != nullptr) v += *reinterpret_cast<const f32x4*>(a.dk_add + off + d0);
-          if (a.dscale != nullptr || a.weight != nullptr) v *= mult;
+          if (whole && a.dk_add != nullptr) v += *reinterpret_cast<const f32x4*>(a.dk_add + off + d0);
+          if (whole && (a.dscale != nullptr || a.weight != nullptr)) v *= mult;
           *reinterpret_cast<f32x4*>(out + d0) = v;
         }
       }
@@ -970,7 +979,7 @@ static_assert(sizeof(HotBatch) <= 4096, "HotBatch exceeds the 4 KiB kernel-argum
 // work items (workgroups) of one relation: row blocks x B x heads
 __host__ __device__ inline int fwd_items(const HotArgs& f) { return (f.r.T + kRows - 1) / kRows * f.r.B * f.r.Hq; }
 __host__ __device__ inline int bwd_items(const HotArgs& f) {
-  return (f.r.T + kRows - 1) / kRows * f.r.B * f.r.s.hkv;
+  return (f.r.T + kRows - 1) / kRows * f.r.B * f.r.s.hkv * dk_parts(f.r);
 }
 
 // relation r of batch item g (uniform: a short scalar loop)

@@ -71,6 +71,13 @@ struct RelArgs {
   //   dk_out = (scale_s * dk + dk_add) * (*dscale)
   const float* dk_add;  // [B, Hkv_s, T, Ds] or null (self relation: the row-side term dq)
   const float* dscale;  // device scalar or null (autograd's dloss)
+  // dk kernels, grouped queries on a grid too small for the chip: each key
+  // block's sum over its group's heads and dk_split ranges of query tiles is
+  // cut into group * dk_split parts, one workgroup each, written (scaled by
+  // scale_s only) to dk_part [B * Hkv_s][group * dk_split][T, Ds]; the finish
+  // kernel adds them up (null: one workgroup sums everything into dk_out).
+  float* dk_part;
+  int dk_split;
   // Throughput kernels only: device scalar or null, the relation's weight in
   // a batched loss (multiplies the per-row KL, and the gradient wherever
   // dscale is applied).

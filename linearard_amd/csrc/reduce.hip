@@ -79,20 +79,45 @@ hipError_t launch_reduce_sum(const float* x, int64_t n, double* partial, unsigne
   return hipGetLastError();
 }
 
-__global__ __launch_bounds__(kReduceThreads) void scale_inplace_kernel(float* __restrict__ x, int64_t n4,
-                                                                        const float* __restrict__ dscale) {
-  const float s = *dscale;
-  f32x4* v = reinterpret_cast<f32x4*>(x);
-  for (int64_t i = (int64_t)blockIdx.x * kReduceThreads + threadIdx.x; i < n4; i += (int64_t)gridDim.x * kReduceThreads)
-    v[i] *= s;
+// The first nscale blocks scale x; the others add up the parts of dk, four
+// floats per thread, in the order of the parts.
+__global__ __launch_bounds__(kReduceThreads) void finish_grads_kernel(float* __restrict__ x, int64_t n4,
+                                                                       const float* __restrict__ dscale, int nscale,
+                                                                       const float* __restrict__ part, int parts,
+                                                                       int64_t head4, int64_t total4,
+                                                                       const float* __restrict__ dk_scale,
+                                                                       float* __restrict__ dk) {
+  const int64_t tid = threadIdx.x;
+  if ((int)blockIdx.x < nscale) {
+    const float s = *dscale;
+    f32x4* v = reinterpret_cast<f32x4*>(x);
+    for (int64_t i = (int64_t)blockIdx.x * kReduceThreads + tid; i < n4; i += (int64_t)nscale * kReduceThreads) v[i] *= s;
+    return;
+  }
+  const float s = dk_scale != nullptr ? *dk_scale : 1.f;
+  const int64_t step = (int64_t)(gridDim.x - nscale) * kReduceThreads;
+  for (int64_t i = (int64_t)(blockIdx.x - nscale) * kReduceThreads + tid; i < total4; i += step) {
+    const int64_t bg = i / head4;
+    const f32x4* p = reinterpret_cast<const f32x4*>(part) + bg * parts * head4 + (i - bg * head4);
+    f32x4 v = p[0];
+    for (int k = 1; k < parts; ++k) v += p[k * head4];
+    if (dk_scale != nullptr) v *= s;
+    reinterpret_cast<f32x4*>(dk)[i] = v;
+  }
 }
 
-hipError_t launch_scale_inplace(float* x, int64_t n, const float* dscale, hipStream_t stream) {
-  if (n <= 0 || dscale == nullptr) return hipSuccess;
-  const int64_t n4 = n / 4;
-  const int64_t want = (n4 + kReduceThreads - 1) / kReduceThreads;
-  const int blocks = (int)(want < 4096 ? want : 4096);
-  hipLaunchKernelGGL(scale_inplace_kernel, dim3(blocks), dim3(kReduceThreads), 0, stream, x, n4, dscale);
+hipError_t launch_finish_grads(float* x, int64_t n, const float* dscale, const RelArgs& a, hipStream_t stream) {
+  const auto blocks = [](int64_t n4) {
+    const int64_t want = (n4 + kReduceThreads - 1) / kReduceThreads;
+    return (int)(want < 4096 ? want : 4096);
+  };
+  const int nscale = x != nullptr && dscale != nullptr && n > 0 ? blocks(n / 4) : 0;
+  const int parts = dk_parts(a);
+  const int64_t head4 = (int64_t)a.T * a.s.dim / 4, total4 = a.dk_part != nullptr ? (int64_t)a.B * a.s.hkv * head4 : 0;
+  const int ndk = total4 > 0 ? blocks(total4) : 0;
+  if (nscale + ndk == 0) return hipSuccess;
+  hipLaunchKernelGGL(finish_grads_kernel, dim3(nscale + ndk), dim3(kReduceThreads), 0, stream, x, n / 4, dscale, nscale,
+                     a.dk_part, parts, head4, total4, a.dscale, a.dk_out);
   return hipGetLastError();
 }
 

@@ -28,7 +28,7 @@ static hipError_t launch_dk(const RelArgs& a, int dpt, dim3 grid, hipStream_t st
 
 hipError_t launch_col_dk(const RelArgs& a, int dps, int dpt, hipStream_t stream) {
   if (a.s.f32) return launch_col_dk_f32(a, stream);  // float32 inputs (both sides)
-  const dim3 grid((a.T + kStageRows - 1) / kStageRows, a.B * a.s.hkv);
+  const dim3 grid((a.T + kStageRows - 1) / kStageRows, a.B * a.s.hkv * dk_parts(a));
   switch (dps) {
 #define X(DP, unused) \
   case DP: return launch_dk<DP>(a, dpt, grid, stream);

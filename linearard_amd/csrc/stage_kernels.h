@@ -213,6 +213,9 @@ __device__ __forceinline__ void stage_grad(const TrXor<DP>& tr, unsigned tile, c
   }
 }
 
+// Parts of a key block's dk sum (RelArgs::dk_part).
+__host__ __device__ inline int dk_parts(const RelArgs& a) { return a.dk_part != nullptr ? a.s.group * a.dk_split : 1; }
+
 // 256-wide gradients: the accumulators (128 registers) stay in AGPRs around the
 // loop.  Left alone, the compiler keeps them in VGPRs between tiles and copies
 // all of them to AGPRs and back for every tile's products.
@@ -478,8 +481,13 @@ __global__ __launch_bounds__(kStageThreads, DPS <= 128 ? 2 : 1) void col_kernel(
   const int half = lane >> 5;
   const int l32 = lane & 31;
   const int T = a.T;
-  int cb, bg;  // small cb = longest causal columns, launched first
-  stage_item(cb, bg);
+  int cb, bgp;  // small cb = longest causal columns, launched first
+  stage_item(cb, bgp);
+  // the part of this key block's sum (RelArgs::dk_part), or all of it
+  const int split = a.dk_part != nullptr ? a.dk_split : 1, parts = dk_parts(a);
+  const int bg = bgp / parts;
+  const int part = bgp - bg * parts;
+  const int part_h = part / split, part_s = part - part_h * split;
   const int b = bg / a.s.hkv;
   const int g = bg - b * a.s.hkv;
   const int j0w = cb * kStageRows + w * 32;
@@ -510,14 +518,17 @@ __global__ __launch_bounds__(kStageThreads, DPS <= 128 ? 2 : 1) void col_kernel(
   for (int db = 0; db < NDB; ++db) dk[db] = (f32x16)(0.f);
   pin_agprs<NDB>(dk);
 
-  const int nib = (T + BM - 1) / BM;
-  const int ib_first = a.causal ? (cb * kStageRows) / BM : 0;
+  const int nib_all = (T + BM - 1) / BM;
+  const int ib_all = a.causal ? (cb * kStageRows) / BM : 0;
+  const int ib_first = ib_all + (nib_all - ib_all) * part_s / split;  // this part's tiles
+  const int nib = ib_all + (nib_all - ib_all) * (part_s + 1) / split;
   const int wave_first_ib = a.causal ? j0w / BM : 0;
   int loaded_ht = -1;
   const unsigned gs = row_chunk_xor<DPS>(l32, half), gt = row_chunk_xor<DPT>(l32, half);
   const TokenBits tok = {lbits, &a, (int64_t)b * a.mask_sb};
 
-  for (int hh = 0; hh < a.s.group; ++hh) {
+  const int hh_end = a.dk_part != nullptr ? part_h + 1 : a.s.group;
+  for (int hh = part_h; hh < hh_end; ++hh) {
     const int h = g * a.s.group + hh;
     const int ht = h / a.t.group;
     if (ht != loaded_ht) {
@@ -617,8 +628,9 @@ __global__ __launch_bounds__(kStageThreads, DPS <= 128 ? 2 : 1) void col_kernel(
   }
 
   if (in_range) {
-    const int64_t off = ((int64_t)bg * T + my_j) * a.s.dim;
-    float* out = a.dk_out + off;
+    const bool whole = a.dk_part == nullptr;
+    const int64_t off = ((int64_t)bgp * T + my_j) * a.s.dim;  // bgp == bg when whole
+    float* out = (whole ? a.dk_out : a.dk_part) + off;
     const float f = a.s.scale;
     const float mult = a.dscale != nullptr ? *a.dscale : 1.f;  // chain rule (integration.py:63-64)
 #pragma unroll
@@ -628,8 +640,8 @@ __global__ __launch_bounds__(kStageThreads, DPS <= 128 ? 2 : 1) void col_kernel(
         const int d0 = 32 * db + 8 * gq + 4 * half;
         if (d0 < a.s.dim) {
           f32x4 v = {dk[db][4 * gq] * f, dk[db][4 * gq + 1] * f, dk[db][4 * gq + 2] * f, dk[db][4 * gq + 3] * f};
-          if (a.dk_add != nullptr) v += *reinterpret_cast<const f32x4*>(a.dk_add + off + d0);
-          if (a.dscale != nullptr) v *= mult;
+          if (whole && a.dk_add != nullptr) v += *reinterpret_cast<const f32x4*>(a.dk_add + off + d0);
+          if (whole && a.dscale != nullptr) v *= mult;
           *reinterpret_cast<f32x4*>(out + d0) = v;
         }
       }
@@ -648,8 +660,10 @@ hipError_t launch_col_dk(const RelArgs& a, int dps, int dpt, hipStream_t stream)
 constexpr int kReduceBlocks = 64;
 hipError_t launch_reduce_sum(const float* x, int64_t n, double* partial, unsigned* counter, float* out,
                              hipStream_t stream);
-// x[0..n) *= (*dscale) in place (dscale a device scalar; n a multiple of 4,
-// x 16-byte aligned): the chain rule of a gradient computed before dloss.
-hipError_t launch_scale_inplace(float* x, int64_t n, const float* dscale, hipStream_t stream);
+// x[0..n) *= (*dscale) in place (dscale a device scalar, null: nothing to do;
+// n a multiple of 4, x 16-byte aligned): the chain rule of a gradient computed
+// before dloss.  When a.dk_part is not null the same launch also adds up the
+// parts: dk_out = (*a.dscale) * sum of the parts.
+hipError_t launch_finish_grads(float* x, int64_t n, const float* dscale, const RelArgs& a, hipStream_t stream);
 
 }  // namespace lard
