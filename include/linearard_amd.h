@@ -285,6 +285,19 @@ int lard_attn_kl_backward_colgrad(const lard_tensor4* qs, const lard_tensor4* ks
                                   void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * lard_attn_kl_backward_colgrad with the gradients written in the input dtype
+ * (float16 / bfloat16, rounded once from the float32 values that entry point
+ * writes): what autograd hands to 16-bit inputs, without a cast pass.  dq_row
+ * is only read.  self_relation != 0: dk_out is the whole gradient, dq_out
+ * unused.  Contiguous outputs, 8-byte aligned.
+ */
+int lard_attn_kl_backward_colgrad16(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s,
+                                    const lard_tensor4* qt, const lard_tensor4* kt, const float* lse_t,
+                                    const lard_mask* mask, int causal, float sm_scale_s, float sm_scale_t,
+                                    const float* dloss, int self_relation, const float* dq_row, void* dq_out,
+                                    void* dk_out, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * One self relation of a batched relation loss: the student tensor xs is
  * both q and k, the teacher tensor xt likewise -- the call
  * attn_kl_align(x_s, x_s, x_t, x_t) of train.py:380-402.  lse_s / lse_t
@@ -357,6 +370,15 @@ int lard_attn_kl_batched_forward_rowgrad(const lard_relation* rels, int nrel, co
 int lard_attn_kl_batched_backward_colgrad(const lard_relation* rels, int nrel, const lard_mask* mask, int causal,
                                           float sm_scale_s, float sm_scale_t, const float* weights,
                                           const float* dloss, void* workspace, size_t workspace_bytes, void* stream);
+
+/* lard_attn_kl_batched_backward_colgrad with the gradients in the input dtype:
+ * dx_out[r] ([B, H, T, D] contiguous, 8-byte aligned; an array of nrel device
+ * pointers in host memory) receives the gradient of xs, rels[r].dxs is only
+ * read. */
+int lard_attn_kl_batched_backward_colgrad16(const lard_relation* rels, int nrel, const lard_mask* mask, int causal,
+                                            float sm_scale_s, float sm_scale_t, const float* weights,
+                                            const float* dloss, void* const* dx_out, void* workspace,
+                                            size_t workspace_bytes, void* stream);
 
 /*
  * RoPE pair producer -- the step before the path: each model's rotary

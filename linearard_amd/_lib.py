@@ -116,6 +116,13 @@ SIGNATURES = {
     "lard_attn_kl_backward_colgrad": (ctypes.c_int, [_T4P, _T4P, _FP, _T4P, _T4P, _FP, _MP, ctypes.c_int,
                                                      ctypes.c_float, ctypes.c_float, _FP, ctypes.c_int, _FP, _FP,
                                                      ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "lard_attn_kl_backward_colgrad16": (ctypes.c_int, [_T4P, _T4P, _FP, _T4P, _T4P, _FP, _MP, ctypes.c_int,
+                                                       ctypes.c_float, ctypes.c_float, _FP, ctypes.c_int, _FP, _FP,
+                                                       _FP, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "lard_attn_kl_batched_backward_colgrad16": (ctypes.c_int, [_RP, ctypes.c_int, _MP, ctypes.c_int, ctypes.c_float,
+                                                               ctypes.c_float, _FP, _FP,
+                                                               ctypes.POINTER(ctypes.c_void_p), ctypes.c_void_p,
+                                                               ctypes.c_size_t, ctypes.c_void_p]),
     "lard_attn_kl_batched_workspace_bytes": (ctypes.c_size_t, [_RP, ctypes.c_int]),
     "lard_attn_kl_batched_forward_rowgrad": (ctypes.c_int, [_RP, ctypes.c_int, _MP, ctypes.c_int, ctypes.c_float,
                                                             ctypes.c_float, _FP, _FP, ctypes.c_void_p,

@@ -13,10 +13,10 @@ launch per 8 relations (``lard_attn_kl_batched_forward`` / ``_backward``):
 the relations' row blocks share one grid even when their head counts differ
 (Q/Q 32 heads next to K/K 8).  When the students need gradients the forward
 is ``lard_attn_kl_batched_forward_rowgrad``, which also leaves the row side
-of every gradient in the float32 buffers the backward returns, and the
-backward (``lard_attn_kl_batched_backward_colgrad``) adds the column side in
-place; a second backward through the same graph runs the full
-``lard_attn_kl_batched_backward``.  ``relation_kl_loss`` builds the weights of
+of every gradient in float32 buffers, and the backward
+(``lard_attn_kl_batched_backward_colgrad16``) adds the column side and writes
+the gradients in the inputs' dtype (the buffers are only read, so a second
+backward through the same graph does the same).  ``relation_kl_loss`` builds the weights of
 the train.py formula from the layers' tensors.  Batches outside the batched
 kernels (different head dims, D = 256, extreme scales) go relation by
 relation through the single-relation entry points inside the same autograd
@@ -109,7 +109,6 @@ class AttnKLBatchedFn(torch.autograd.Function):
 
         saved_mask = attn_mask if attn_mask is not None else torch.empty(0, device=dev)
         ctx.has_row_grad = row_grad is not None
-        ctx.row_grad_used = False
         ctx.save_for_backward(weights, saved_mask, *xs, *xt, *lse_s, *lse_t, *(row_grad or []))
         ctx.n = n
         ctx.has_mask = attn_mask is not None
@@ -131,16 +130,16 @@ class AttnKLBatchedFn(torch.autograd.Function):
         L = _lib.lib()
         md = _lib.mask_desc(attn_mask)
         stream = _lib.stream_of(xs[0])
-        if ctx.has_row_grad and not ctx.row_grad_used:
-            ctx.row_grad_used = True
-            dxs = list(saved[2 + 4 * n:2 + 5 * n])
-            rels = _relations(xs, xt, lse_s, lse_t, dxs)
+        if ctx.has_row_grad:
+            rels = _relations(xs, xt, lse_s, lse_t, saved[2 + 4 * n:2 + 5 * n])
             ws_bytes = L.lard_attn_kl_batched_workspace_bytes(rels, n)
             ws = _workspace(ws_bytes, dev)
-            rc = L.lard_attn_kl_batched_backward_colgrad(rels, n, ctypes.byref(md), int(ctx.causal), ctx.ss[0],
-                                                         ctx.st[0], weights.data_ptr(), dloss.data_ptr(),
-                                                         ws.data_ptr(), ws_bytes, stream)
-            _lib.check(rc, "lard_attn_kl_batched_backward_colgrad")
+            dxs = [torch.empty(x.shape, device=dev, dtype=x.dtype) for x in xs]
+            out = (ctypes.c_void_p * n)(*(x.data_ptr() for x in dxs))
+            rc = L.lard_attn_kl_batched_backward_colgrad16(rels, n, ctypes.byref(md), int(ctx.causal), ctx.ss[0],
+                                                           ctx.st[0], weights.data_ptr(), dloss.data_ptr(), out,
+                                                           ws.data_ptr(), ws_bytes, stream)
+            _lib.check(rc, "lard_attn_kl_batched_backward_colgrad16")
             return (None, None, None, None, None, None, *dxs, *([None] * n))
         dxs = [torch.empty(x.shape, device=dev, dtype=torch.float32) for x in xs]
         if ctx.batched:

@@ -20,9 +20,9 @@ kernels, the forward is ``lard_attn_kl_forward_rowgrad`` instead: the same
 pass also forms the row side of the gradient (dq before dloss, a float32
 [B, Hq, T, Ds] buffer kept for the backward, O(n d) like the gradient
 itself), and the backward runs only the column side
-(``lard_attn_kl_backward_colgrad``), which adds itself to that buffer in
-place.  A second backward through the same graph (retain_graph) finds the
-buffer consumed and runs the full ``lard_attn_kl_backward``.  For float32
+(``lard_attn_kl_backward_colgrad16``), which adds that buffer to itself and
+writes the gradient in the inputs' dtype (the buffer is only read: a second
+backward through the same graph does the same).  For float32
 inputs that need a gradient the pair is ``lard_attn_kl_forward_lse64`` /
 ``lard_attn_kl_backward_lse64``, which keeps both LSEs in double between the
 passes.
@@ -117,7 +117,6 @@ class AttnKLAlignFn(torch.autograd.Function):
 
         saved_mask = attn_mask if attn_mask is not None else torch.empty(0, device=dev)
         ctx.has_row_grad = dq_row is not None
-        ctx.row_grad_used = False
         ctx.has_lse64 = lse64 is not None
         extra = dq_row if dq_row is not None else lse64 if lse64 is not None else torch.empty(0, device=dev)
         ctx.save_for_backward(qs, ks, lse_s, qt, kt, lse_t, saved_mask, extra)
@@ -144,20 +143,18 @@ class AttnKLAlignFn(torch.autograd.Function):
         if not ctx.has_lse64:
             ws_bytes = L.lard_attn_kl_backward_workspace_bytes(B, Hq, ks.shape[1], T, Ds, int(self_rel))
             ws = _workspace(ws_bytes, dev)
-        if ctx.has_row_grad and not ctx.row_grad_used:
+        if ctx.has_row_grad:
             # the row side came with the forward: the column side adds itself
-            # to it in place (self relation) or dq_row becomes dq
-            ctx.row_grad_used = True
-            dk = dq_row if self_rel else torch.empty((B, ks.shape[1], T, Ds), device=dev, dtype=torch.float32)
-            rc = L.lard_attn_kl_backward_colgrad(
+            # to it (self relation), or it becomes dq; both in the inputs' dtype
+            dk = torch.empty((B, ks.shape[1], T, Ds), device=dev, dtype=qs.dtype)
+            dq = None if self_rel else torch.empty((B, Hq, T, Ds), device=dev, dtype=qs.dtype)
+            rc = L.lard_attn_kl_backward_colgrad16(
                 ctypes.byref(d[0]), ctypes.byref(d[1]), lse_s.data_ptr(), ctypes.byref(d[2]), ctypes.byref(d[3]),
                 lse_t.data_ptr(), ctypes.byref(md), int(ctx.causal), ctx.sm_scale_s, ctx.sm_scale_t,
-                dloss.data_ptr(), int(self_rel), dq_row.data_ptr(), dk.data_ptr(), ws.data_ptr(), ws_bytes,
-                _lib.stream_of(qs))
-            _lib.check(rc, "lard_attn_kl_backward_colgrad")
-            if self_rel:
-                return dk, None, None, None, None, None, None, None
-            return dq_row, dk, None, None, None, None, None, None
+                dloss.data_ptr(), int(self_rel), dq_row.data_ptr(), None if dq is None else dq.data_ptr(),
+                dk.data_ptr(), ws.data_ptr(), ws_bytes, _lib.stream_of(qs))
+            _lib.check(rc, "lard_attn_kl_backward_colgrad16")
+            return (dk if self_rel else dq), (None if self_rel else dk), None, None, None, None, None, None
         dk = torch.empty((B, ks.shape[1], T, Ds), device=dev, dtype=torch.float32)
         dq = None if self_rel else torch.empty((B, Hq, T, Ds), device=dev, dtype=torch.float32)
         if ctx.has_lse64:  # float32 inputs: the forward kept its LSEs in double

@@ -765,7 +765,7 @@ int lard_kl_backward_ws(const lard_tensor4* qs, const lard_tensor4* ks, const fl
   if ((rc = hip_status(timed(LARD_KERNEL_COL_GRAD, st, [&] { return lard::launch_col_dk(a, dps, dpt, st); }),
                        "kl_backward dk launch")) != LARD_OK)
     return rc;
-  return hip_status(lard::launch_finish_grads(nullptr, 0, nullptr, a, st), "kl_backward dk sum launch");
+  return hip_status(lard::launch_finish_grads(nullptr, nullptr, 0, a, st), "kl_backward dk sum launch");
 }
 
 int lard_kl_backward(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s, const lard_tensor4* qt,
@@ -1070,7 +1070,7 @@ int attn_kl_backward_impl(const lard_tensor4* qs, const lard_tensor4* ks, const 
     if ((rc = hip_status(timed(LARD_KERNEL_COL_GRAD, st, [&] { return lard::launch_hot_bwd(f, padded_dim(ds), bf, st); }),
                          "attn_kl_backward dk launch")) != LARD_OK)
       return rc;
-    return hip_status(lard::launch_finish_grads(nullptr, 0, nullptr, f.r, st), "attn_kl_backward dk sum launch");
+    return hip_status(lard::launch_finish_grads(nullptr, nullptr, 0, f.r, st), "attn_kl_backward dk sum launch");
   }
   const int dps = padded_dim(ds), dpt = padded_dim(dt);
   if (lse64 != nullptr) {
@@ -1102,7 +1102,7 @@ int attn_kl_backward_impl(const lard_tensor4* qs, const lard_tensor4* ks, const 
   if ((rc = hip_status(timed(LARD_KERNEL_COL_GRAD, st, [&] { return lard::launch_col_dk(a, dps, dpt, st); }),
                        "attn_kl_backward dk launch")) != LARD_OK)
     return rc;
-  return hip_status(lard::launch_finish_grads(nullptr, 0, nullptr, a, st), "attn_kl_backward dk sum launch");
+  return hip_status(lard::launch_finish_grads(nullptr, nullptr, 0, a, st), "attn_kl_backward dk sum launch");
 }
 
 }  // namespace
@@ -1199,16 +1199,23 @@ int lard_attn_kl_forward_rowgrad(const lard_tensor4* qs, const lard_tensor4* ks,
                     "attn_kl_forward_rowgrad reduce launch");
 }
 
-int lard_attn_kl_backward_colgrad(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s,
-                                  const lard_tensor4* qt, const lard_tensor4* kt, const float* lse_t,
-                                  const lard_mask* mask, int causal, float sm_scale_s, float sm_scale_t,
-                                  const float* dloss, int self_relation, float* dq_row, float* dk_out,
-                                  void* workspace, size_t workspace_bytes, void* stream) {
+}  // extern "C"
+
+namespace {
+
+// lard_attn_kl_backward_colgrad; dq16 / dk16: the gradients in the input type
+// instead of float32 (dq_row is then only read).
+int backward_colgrad_impl(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s, const lard_tensor4* qt,
+                          const lard_tensor4* kt, const float* lse_t, const lard_mask* mask, int causal,
+                          float sm_scale_s, float sm_scale_t, const float* dloss, int self_relation, float* dq_row,
+                          float* dk_out, lard::u16* dq16, lard::u16* dk16, void* workspace, size_t workspace_bytes,
+                          void* stream) {
   int rc;
   if ((rc = check_two_sided(qs, ks, lse_s, qt, kt, lse_t, mask, sm_scale_s, sm_scale_t)) != LARD_OK) return rc;
   const int64_t B = qs->size[0], Hq = qs->size[1], T = qs->size[2];
   if (B * Hq * T == 0) return ok();
-  if (dk_out == nullptr || dq_row == nullptr) return fail(LARD_ERR_INVALID_ARGUMENT, "dq_row and dk_out must not be NULL");
+  if ((dk_out == nullptr && dk16 == nullptr) || dq_row == nullptr)
+    return fail(LARD_ERR_INVALID_ARGUMENT, "dq_row and dk_out must not be NULL");
   if (self_relation) {
     if (ks->size[1] != Hq || qs->data != ks->data || qs->stride[0] != ks->stride[0] ||
         qs->stride[1] != ks->stride[1] || qs->stride[2] != ks->stride[2])
@@ -1244,6 +1251,7 @@ int lard_attn_kl_backward_colgrad(const lard_tensor4* qs, const lard_tensor4* ks
   f.nl_s = w.nl_s;
   f.nl_t = w.nl_t;
   f.r.dk_out = dk_out;
+  f.r.dk16 = dk16;
   f.r.dk_add = self_relation ? dq_row : nullptr;
   f.r.dscale = dloss;
   const bool bf = qs->dtype == LARD_DTYPE_BF16;
@@ -1251,8 +1259,38 @@ int lard_attn_kl_backward_colgrad(const lard_tensor4* qs, const lard_tensor4* ks
                        "attn_kl_backward_colgrad dk launch")) != LARD_OK)
     return rc;
   if (self_relation) return ok();
-  return hip_status(lard::launch_finish_grads(dq_row, B * Hq * T * qs->size[3], dloss, f.r, st),
+  return hip_status(lard::launch_finish_grads(dq_row, dq16, B * Hq * T * qs->size[3], f.r, st),
                     "attn_kl_backward_colgrad finish launch");
+}
+
+}  // namespace
+
+extern "C" {
+
+int lard_attn_kl_backward_colgrad(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s,
+                                  const lard_tensor4* qt, const lard_tensor4* kt, const float* lse_t,
+                                  const lard_mask* mask, int causal, float sm_scale_s, float sm_scale_t,
+                                  const float* dloss, int self_relation, float* dq_row, float* dk_out,
+                                  void* workspace, size_t workspace_bytes, void* stream) {
+  return backward_colgrad_impl(qs, ks, lse_s, qt, kt, lse_t, mask, causal, sm_scale_s, sm_scale_t, dloss, self_relation,
+                               dq_row, dk_out, nullptr, nullptr, workspace, workspace_bytes, stream);
+}
+
+int lard_attn_kl_backward_colgrad16(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s,
+                                    const lard_tensor4* qt, const lard_tensor4* kt, const float* lse_t,
+                                    const lard_mask* mask, int causal, float sm_scale_s, float sm_scale_t,
+                                    const float* dloss, int self_relation, const float* dq_row, void* dq_out,
+                                    void* dk_out, void* workspace, size_t workspace_bytes, void* stream) {
+  if (dk_out == nullptr || (!self_relation && dq_out == nullptr) || reinterpret_cast<uintptr_t>(dk_out) % 8 != 0 ||
+      reinterpret_cast<uintptr_t>(dq_out) % 8 != 0) {
+    // an empty problem writes nothing
+    if (qs == nullptr || qs->size[0] * qs->size[1] * qs->size[2] > 0)
+      return fail(LARD_ERR_INVALID_ARGUMENT, "dq_out and dk_out must not be NULL and 8-byte aligned");
+  }
+  return backward_colgrad_impl(qs, ks, lse_s, qt, kt, lse_t, mask, causal, sm_scale_s, sm_scale_t, dloss, self_relation,
+                               const_cast<float*>(dq_row), nullptr,
+                               self_relation ? nullptr : static_cast<lard::u16*>(dq_out),
+                               static_cast<lard::u16*>(dk_out), workspace, workspace_bytes, stream);
 }
 
 size_t lard_attn_kl_batched_workspace_bytes(const lard_relation* rels, int nrel) {
@@ -1473,13 +1511,22 @@ int lard_attn_kl_batched_forward_rowgrad(const lard_relation* rels, int nrel, co
                     "batched forward_rowgrad reduce launch");
 }
 
-int lard_attn_kl_batched_backward_colgrad(const lard_relation* rels, int nrel, const lard_mask* mask, int causal,
-                                          float sm_scale_s, float sm_scale_t, const float* weights,
-                                          const float* dloss, void* workspace, size_t workspace_bytes, void* stream) {
+}  // extern "C"
+
+namespace {
+
+// lard_attn_kl_batched_backward_colgrad; dx16: each relation's gradient in the
+// input type instead (rels[r].dxs is then only read).
+int batched_colgrad_impl(const lard_relation* rels, int nrel, const lard_mask* mask, int causal, float sm_scale_s,
+                         float sm_scale_t, const float* weights, const float* dloss, void* const* dx16,
+                         void* workspace, size_t workspace_bytes, void* stream) {
   int rc;
   if ((rc = check_batch(rels, nrel, mask, sm_scale_s, sm_scale_t)) != LARD_OK) return rc;
   int64_t rows = 0;
   for (int r = 0; r < nrel; ++r) {
+    if (dx16 != nullptr && rel_rows(rels[r]) > 0 &&
+        (dx16[r] == nullptr || reinterpret_cast<uintptr_t>(dx16[r]) % 8 != 0))
+      return fail(LARD_ERR_INVALID_ARGUMENT, "relation %d: dx_out must not be NULL and 8-byte aligned", r);
     if (rel_rows(rels[r]) > 0 && (rels[r].lse_s == nullptr || rels[r].lse_t == nullptr || rels[r].dxs == nullptr))
       return fail(LARD_ERR_INVALID_ARGUMENT, "relation %d: lse inputs and dxs must not be NULL", r);
     rows += rel_rows(rels[r]);
@@ -1517,6 +1564,7 @@ int lard_attn_kl_batched_backward_colgrad(const lard_relation* rels, int nrel, c
       rp.rel[rp.n++] = row_prep(f);
       f.r.dk_out = rels[r].dxs;
       f.r.dk_add = rels[r].dxs;
+      f.r.dk16 = dx16 != nullptr ? static_cast<lard::u16*>(dx16[r]) : nullptr;
       f.r.dscale = dloss;
       f.r.weight = weights != nullptr ? weights + r : nullptr;
       mk.rel[mk.n++] = f;
@@ -1529,6 +1577,26 @@ int lard_attn_kl_batched_backward_colgrad(const lard_relation* rels, int nrel, c
       return rc;
   }
   return ok();
+}
+
+}  // namespace
+
+extern "C" {
+
+int lard_attn_kl_batched_backward_colgrad(const lard_relation* rels, int nrel, const lard_mask* mask, int causal,
+                                          float sm_scale_s, float sm_scale_t, const float* weights,
+                                          const float* dloss, void* workspace, size_t workspace_bytes, void* stream) {
+  return batched_colgrad_impl(rels, nrel, mask, causal, sm_scale_s, sm_scale_t, weights, dloss, nullptr, workspace,
+                              workspace_bytes, stream);
+}
+
+int lard_attn_kl_batched_backward_colgrad16(const lard_relation* rels, int nrel, const lard_mask* mask, int causal,
+                                            float sm_scale_s, float sm_scale_t, const float* weights,
+                                            const float* dloss, void* const* dx_out, void* workspace,
+                                            size_t workspace_bytes, void* stream) {
+  if (dx_out == nullptr) return fail(LARD_ERR_INVALID_ARGUMENT, "dx_out must not be NULL");
+  return batched_colgrad_impl(rels, nrel, mask, causal, sm_scale_s, sm_scale_t, weights, dloss, dx_out, workspace,
+                              workspace_bytes, stream);
 }
 
 int lard_rope_pair(const lard_tensor4* x, const float* inv_freq_t, const float* inv_freq_s, float att_t, float att_s,

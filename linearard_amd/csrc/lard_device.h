@@ -78,6 +78,9 @@ struct RelArgs {
   // kernel adds them up (null: one workgroup sums everything into dk_out).
   float* dk_part;
   int dk_split;
+  // Throughput kernels: dk rounded to the input type here instead of dk_out
+  // (null: float32 to dk_out).
+  u16* dk16;
   // Throughput kernels only: device scalar or null, the relation's weight in
   // a batched loss (multiplies the per-row KL, and the gradient wherever
   // dscale is applied).
@@ -147,6 +150,18 @@ __device__ __forceinline__ u16x8 to_bits8(const float* x) {
     return __builtin_bit_cast(u16x8, __builtin_convertvector(v, bf16x8));
   } else {
     return __builtin_bit_cast(u16x8, __builtin_convertvector(v, f16x8));
+  }
+}
+
+// to_bits for 4 floats at once.
+template <bool BF>
+__device__ __forceinline__ u16x4 to_bits4(f32x4 v) {
+  if constexpr (BF) {
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(u16x4, __builtin_convertvector(v, bf16x4));
+  } else {
+    typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(u16x4, __builtin_convertvector(v, f16x4));
   }
 }
 

@@ -79,45 +79,65 @@ hipError_t launch_reduce_sum(const float* x, int64_t n, double* partial, unsigne
   return hipGetLastError();
 }
 
-// The first nscale blocks scale x; the others add up the parts of dk, four
-// floats per thread, in the order of the parts.
-__global__ __launch_bounds__(kReduceThreads) void finish_grads_kernel(float* __restrict__ x, int64_t n4,
-                                                                       const float* __restrict__ dscale, int nscale,
-                                                                       const float* __restrict__ part, int parts,
-                                                                       int64_t head4, int64_t total4,
-                                                                       const float* __restrict__ dk_scale,
-                                                                       float* __restrict__ dk) {
+// Four floats as they are, or rounded to the 16-bit input type.
+__device__ __forceinline__ void store_grad(float* out, u16* out16, bool bf, int64_t i4, f32x4 v) {
+  if (out16 != nullptr)
+    reinterpret_cast<u16x4*>(out16)[i4] = bf ? to_bits4<true>(v) : to_bits4<false>(v);
+  else
+    reinterpret_cast<f32x4*>(out)[i4] = v;
+}
+
+struct FinishArgs {
+  float* x;              // dq before dloss (scaled in place unless x16 is given)
+  u16* x16;
+  int64_t n4;
+  const float* dscale;   // null: 1
+  int nscale;            // the first workgroups scale x; the others add up the parts of dk
+  const float* part;
+  int parts;
+  int64_t head4, total4;
+  float* dk;
+  u16* dk16;
+  int bf;
+};
+
+// Four floats per thread; the parts are added in their order.
+__global__ __launch_bounds__(kReduceThreads) void finish_grads_kernel(const FinishArgs f) {
   const int64_t tid = threadIdx.x;
-  if ((int)blockIdx.x < nscale) {
-    const float s = *dscale;
-    f32x4* v = reinterpret_cast<f32x4*>(x);
-    for (int64_t i = (int64_t)blockIdx.x * kReduceThreads + tid; i < n4; i += (int64_t)nscale * kReduceThreads) v[i] *= s;
+  const float s = f.dscale != nullptr ? *f.dscale : 1.f;
+  if ((int)blockIdx.x < f.nscale) {
+    for (int64_t i = (int64_t)blockIdx.x * kReduceThreads + tid; i < f.n4; i += (int64_t)f.nscale * kReduceThreads)
+      store_grad(f.x, f.x16, f.bf != 0, i, reinterpret_cast<const f32x4*>(f.x)[i] * s);
     return;
   }
-  const float s = dk_scale != nullptr ? *dk_scale : 1.f;
-  const int64_t step = (int64_t)(gridDim.x - nscale) * kReduceThreads;
-  for (int64_t i = (int64_t)(blockIdx.x - nscale) * kReduceThreads + tid; i < total4; i += step) {
-    const int64_t bg = i / head4;
-    const f32x4* p = reinterpret_cast<const f32x4*>(part) + bg * parts * head4 + (i - bg * head4);
+  const int64_t step = (int64_t)((int)gridDim.x - f.nscale) * kReduceThreads;
+  for (int64_t i = (int64_t)((int)blockIdx.x - f.nscale) * kReduceThreads + tid; i < f.total4; i += step) {
+    const int64_t bg = i / f.head4;
+    const f32x4* p = reinterpret_cast<const f32x4*>(f.part) + bg * f.parts * f.head4 + (i - bg * f.head4);
     f32x4 v = p[0];
-    for (int k = 1; k < parts; ++k) v += p[k * head4];
-    if (dk_scale != nullptr) v *= s;
-    reinterpret_cast<f32x4*>(dk)[i] = v;
+    for (int k = 1; k < f.parts; ++k) v += p[k * f.head4];
+    if (f.dscale != nullptr) v *= s;
+    store_grad(f.dk, f.dk16, f.bf != 0, i, v);
   }
 }
 
-hipError_t launch_finish_grads(float* x, int64_t n, const float* dscale, const RelArgs& a, hipStream_t stream) {
+hipError_t launch_finish_grads(float* x, u16* x16, int64_t n, const RelArgs& a, hipStream_t stream) {
   const auto blocks = [](int64_t n4) {
     const int64_t want = (n4 + kReduceThreads - 1) / kReduceThreads;
     return (int)(want < 4096 ? want : 4096);
   };
-  const int nscale = x != nullptr && dscale != nullptr && n > 0 ? blocks(n / 4) : 0;
-  const int parts = dk_parts(a);
-  const int64_t head4 = (int64_t)a.T * a.s.dim / 4, total4 = a.dk_part != nullptr ? (int64_t)a.B * a.s.hkv * head4 : 0;
-  const int ndk = total4 > 0 ? blocks(total4) : 0;
-  if (nscale + ndk == 0) return hipSuccess;
-  hipLaunchKernelGGL(finish_grads_kernel, dim3(nscale + ndk), dim3(kReduceThreads), 0, stream, x, n / 4, dscale, nscale,
-                     a.dk_part, parts, head4, total4, a.dscale, a.dk_out);
+  FinishArgs f{};
+  f.x = x, f.x16 = x16, f.n4 = n / 4;
+  f.dscale = a.dscale;
+  f.nscale = x != nullptr && (a.dscale != nullptr || x16 != nullptr) && n > 0 ? blocks(f.n4) : 0;
+  f.part = a.dk_part, f.parts = dk_parts(a);
+  f.head4 = (int64_t)a.T * a.s.dim / 4;
+  f.total4 = a.dk_part != nullptr ? (int64_t)a.B * a.s.hkv * f.head4 : 0;
+  f.dk = a.dk_out, f.dk16 = a.dk16;
+  f.bf = a.s.bf16;
+  const int ndk = f.total4 > 0 ? blocks(f.total4) : 0;
+  if (f.nscale + ndk == 0) return hipSuccess;
+  hipLaunchKernelGGL(finish_grads_kernel, dim3(f.nscale + ndk), dim3(kReduceThreads), 0, stream, f);
   return hipGetLastError();
 }
 

@@ -660,10 +660,11 @@ hipError_t launch_col_dk(const RelArgs& a, int dps, int dpt, hipStream_t stream)
 constexpr int kReduceBlocks = 64;
 hipError_t launch_reduce_sum(const float* x, int64_t n, double* partial, unsigned* counter, float* out,
                              hipStream_t stream);
-// x[0..n) *= (*dscale) in place (dscale a device scalar, null: nothing to do;
-// n a multiple of 4, x 16-byte aligned): the chain rule of a gradient computed
-// before dloss.  When a.dk_part is not null the same launch also adds up the
-// parts: dk_out = (*a.dscale) * sum of the parts.
-hipError_t launch_finish_grads(float* x, int64_t n, const float* dscale, const RelArgs& a, hipStream_t stream);
+// x[0..n) *= (*a.dscale) in place (the chain rule of a gradient computed
+// before dloss; a.dscale null: nothing to do), or, with x16, x16 = x times
+// *a.dscale rounded to the input type (n a multiple of 4, x 16-byte aligned).
+// When a.dk_part is not null the same launch also adds up the parts: dk_out
+// (or dk16) = (*a.dscale) * sum of the parts.
+hipError_t launch_finish_grads(float* x, u16* x16, int64_t n, const RelArgs& a, hipStream_t stream);
 
 }  // namespace lard

@@ -47,10 +47,9 @@ def test_cut_dk_matches_the_oracle(gpu_available, dtype, B, hq, hkv, T, D, causa
     _, rq, rk, _, _ = O.attn_kl_align(qs, ks, qt, kt, mask, causal, a, a)
     loss = attn_kl_align(d[0], d[1], d[2], d[3], attn_mask=m, causal=causal, sm_scale_s=a, sm_scale_t=a)
     two = 2.0 * loss  # dloss = 2 through the parts
-    for again in range(2):  # the autograd pair, then the general backward of the same graph
-        dq, dk = torch.autograd.grad(two, d[:2], retain_graph=True)
-        check_grad(dq.float().cpu().numpy(), 2.0 * rq, case + f"-{again}", "dq")
-        check_grad(dk.float().cpu().numpy(), 2.0 * rk, case + f"-{again}", "dk")
+    dq, dk = torch.autograd.grad(two, d[:2])
+    check_grad(dq.float().cpu().numpy(), 2.0 * rq, case, "dq")
+    check_grad(dk.float().cpu().numpy(), 2.0 * rk, case, "dk")
     x = [t.detach() for t in d]
     ls, lt = lse_stats(x[0], x[1], m, causal, a), lse_stats(x[2], x[3], m, causal, a)
     dq, dk = kl_backward(x[0], x[1], ls, x[2], x[3], lt, m, causal, a, a)
@@ -63,3 +62,106 @@ def test_cut_dk_matches_the_oracle(gpu_available, dtype, B, hq, hkv, T, D, causa
     assert rc == 0, L.lard_last_error()
     assert torch.equal(dq, dq0)
     assert float((dk - dk0).abs().max()) <= 1e-5 * float(dk0.abs().max())
+
+
+def _general_backward(L, x, lse, mask, causal, a, dloss, self_rel):
+    """lard_attn_kl_backward (both sides recomputed; no row side kept)."""
+    B, hq, T, D = x[0].shape
+    hkv = x[1].shape[1]
+    dq = None if self_rel else torch.empty((B, hq, T, D), device="cuda")
+    dk = torch.empty((B, hkv, T, D), device="cuda")
+    nb = L.lard_attn_kl_backward_workspace_bytes(B, hq, hkv, T, D, int(self_rel))
+    ws = torch.empty((nb,), device="cuda", dtype=torch.uint8)
+    p = [ctypes.byref(_lib.tensor4(t)) for t in x]
+    rc = L.lard_attn_kl_backward(p[0], p[1], lse[0].data_ptr(), p[2], p[3], lse[1].data_ptr(),
+                                 ctypes.byref(_lib.mask_desc(mask)), int(causal), a, a, dloss.data_ptr(),
+                                 int(self_rel), None if dq is None else dq.data_ptr(), dk.data_ptr(), ws.data_ptr(),
+                                 nb, _lib.stream_of(dk))
+    assert rc == 0, L.lard_last_error()
+    return dq, dk
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("self_rel,hkv,T,D", [(True, 4, 333, 128), (True, 4, 65, 8), (False, 2, 900, 64), (False, 4, 130, 32)])
+def test_gradients_in_the_input_dtype(gpu_available, dtype, self_rel, hkv, T, D):
+    """colgrad16 is colgrad rounded once, bitwise, and both agree with the
+    general backward (cut or not) and the oracle; a second backward of one
+    graph repeats the first."""
+    from linearard_amd.attention_KL import attn_kl_align
+
+    B, hq, causal = 2, 4, True
+    qs, ks, qt, kt, mask = _problem(T * 3 + D, dtype, B, hq, hkv, T, D, 0.3)
+    if self_rel:
+        ks, kt = qs, qt
+    m = mask_to_dev(mask)
+    a = 1 / math.sqrt(D)
+    xq, yq = to_dev(qs, dtype, requires_grad=True), to_dev(qt, dtype)
+    xk, yk = (xq, yq) if self_rel else (to_dev(ks, dtype, requires_grad=True), to_dev(kt, dtype))
+    wrt = [xq] if self_rel else [xq, xk]
+    loss = 1.5 * attn_kl_align(xq, xk, yq, yk, attn_mask=m, causal=causal, sm_scale_s=a, sm_scale_t=a)
+    got = torch.autograd.grad(loss, wrt, retain_graph=True)
+    again = torch.autograd.grad(loss, wrt)
+    assert all(g.dtype == xq.dtype and torch.equal(g, h) for g, h in zip(got, again))
+    L = _lib.lib()
+    x = [t.detach() for t in (xq, xk, yq, yk)]
+    d = [_lib.tensor4(t) for t in x]
+    p = [ctypes.byref(t) for t in d]
+    md, st = _lib.mask_desc(m), _lib.stream_of(x[0])
+    lse = [torch.empty((B, hq, T), device="cuda") for _ in range(2)]
+    out, dloss = torch.empty((), device="cuda"), torch.full((), 1.5, device="cuda")
+    dq_row = torch.empty((B, hq, T, D), device="cuda")
+    nb = L.lard_attn_kl_forward_rowgrad_workspace_bytes(B, hq, hkv, hkv, T, D)
+    ws = torch.empty((nb,), device="cuda", dtype=torch.uint8)
+    rc = L.lard_attn_kl_forward_rowgrad(*p, ctypes.byref(md), int(causal), a, a, lse[0].data_ptr(), lse[1].data_ptr(),
+                                        out.data_ptr(), dq_row.data_ptr(), ws.data_ptr(), nb, st)
+    assert rc == 0, L.lard_last_error()
+    dk = torch.empty((B, hkv, T, D), device="cuda")
+    nb = L.lard_attn_kl_backward_workspace_bytes(B, hq, hkv, T, D, int(self_rel))
+    ws = torch.empty((nb,), device="cuda", dtype=torch.uint8)
+    rc = L.lard_attn_kl_backward_colgrad(p[0], p[1], lse[0].data_ptr(), p[2], p[3], lse[1].data_ptr(), ctypes.byref(md),
+                                         int(causal), a, a, dloss.data_ptr(), int(self_rel), dq_row.data_ptr(),
+                                         dk.data_ptr(), ws.data_ptr(), nb, st)
+    assert rc == 0, L.lard_last_error()
+    f32 = [dk] if self_rel else [dq_row, dk]
+    for g, f in zip(got, f32):
+        assert torch.equal(g, f.to(g.dtype))
+    gq, gk = _general_backward(L, x, lse, m, causal, a, dloss, self_rel)
+    ref = O.attn_kl_align(qs, ks, qt, kt, mask, causal, a, a, dloss=1.5, self_relation=self_rel)
+    case = f"grad16-{dtype}-{int(self_rel)}-{hkv}-{T}-{D}"
+    for name, g, f, r in zip(("dX",) if self_rel else ("dq", "dk"), got, (gk,) if self_rel else (gq, gk), ref[1:3]):
+        check_grad(g.float().cpu().numpy(), r, case, name)
+        check_grad(f.cpu().numpy(), r, case + "-general", name)
+
+
+def test_batched_gradients_against_the_general_batched_backward(gpu_available):
+    """Autograd's batched gradients (input dtype, row side from the forward)
+    and lard_attn_kl_batched_backward (both sides recomputed) agree within the
+    gradient bar, relation by relation."""
+    from linearard_amd.attention_KL.batched import _relations, attn_kl_align_batched
+
+    rng = np.random.default_rng(77)
+    B, T, D, heads = 2, 200, 64, [4, 1, 2]
+    xs = [to_dev(randn(rng, (B, h, T, D), "bf16"), "bf16", requires_grad=True) for h in heads]
+    xt = [to_dev(randn(rng, (B, h, T, D), "bf16"), "bf16") for h in heads]
+    m = mask_to_dev(make_mask(rng, B, T, 0.2))
+    w = torch.tensor([0.5, 2.0, 1.0], device="cuda")
+    loss = attn_kl_align_batched(xs, xt, w, attn_mask=m, sm_scale_s=0.1, sm_scale_t=0.1)
+    got = torch.autograd.grad(loss, xs)
+    L, n = _lib.lib(), len(xs)
+    s = [x.detach() for x in xs]
+    lse_s = [torch.empty(x.shape[:3], device="cuda") for x in s]
+    lse_t = [torch.empty(x.shape[:3], device="cuda") for x in s]
+    dx = [torch.empty(x.shape, device="cuda") for x in s]
+    rels = _relations(s, xt, lse_s, lse_t, dx)
+    nb = L.lard_attn_kl_batched_workspace_bytes(rels, n)
+    ws = torch.empty((nb,), device="cuda", dtype=torch.uint8)
+    out, one = torch.empty((), device="cuda"), torch.ones((), device="cuda")
+    md = _lib.mask_desc(m)
+    rc = L.lard_attn_kl_batched_forward(rels, n, ctypes.byref(md), 1, 0.1, 0.1, w.data_ptr(), out.data_ptr(),
+                                        ws.data_ptr(), nb, _lib.stream_of(out))
+    assert rc == 0, L.lard_last_error()
+    rc = L.lard_attn_kl_batched_backward(rels, n, ctypes.byref(md), 1, 0.1, 0.1, w.data_ptr(), one.data_ptr(),
+                                         ws.data_ptr(), nb, _lib.stream_of(out))
+    assert rc == 0, L.lard_last_error()
+    for r, (g, f) in enumerate(zip(got, dx)):
+        check_grad(g.float().cpu().numpy(), f.cpu().numpy(), f"batched-general-rel{r}")
