@@ -12,6 +12,7 @@ from __future__ import annotations
 import ctypes
 import os
 import re
+import struct
 
 import torch
 
@@ -185,43 +186,67 @@ def check(rc: int, what: str) -> None:
         raise RuntimeError(f"{what} failed (status {rc}): {msg}")
 
 
+# One packed copy per descriptor: written field by field, the descriptors of a
+# forward and backward took a fifth of the host time of a small call (3.5 us a
+# tensor, 1.3 us packed).
+_PACK4 = struct.Struct("@P4q4qi4x")
+_PACK3 = struct.Struct("@P3q3qi4x")
+_PACK_MASK = struct.Struct("@Pi4x2q2q")
+_PACK_REL = struct.Struct("@3P")
+
+
+def _pack4(t: torch.Tensor) -> bytes:
+    return _PACK4.pack(t.data_ptr(), *t.shape, *t.stride(), DTYPE_CODES[t.dtype])
+
+
 def tensor4(t: torch.Tensor) -> Tensor4:
-    d = Tensor4()
-    d.data = t.data_ptr()
-    for i in range(4):
-        d.size[i] = t.shape[i]
-        d.stride[i] = t.stride(i)
-    d.dtype = DTYPE_CODES[t.dtype]
-    return d
+    return Tensor4.from_buffer_copy(_pack4(t))
+
+
+def relations(xs, xt, lse_s, lse_t, dxs=None):
+    """``lard_relation[n]``; lse_s, lse_t, dxs: device addresses per relation."""
+    n = len(xs)
+    dxs = dxs if dxs is not None else [0] * n
+    return (Relation * n).from_buffer_copy(b"".join(
+        _pack4(xs[r]) + _pack4(xt[r]) + _PACK_REL.pack(lse_s[r], lse_t[r], dxs[r]) for r in range(n)))
+
+
+def stat_buffer(sizes, device):
+    """One float32 tensor that holds len(sizes) arrays, and their addresses
+    (256-byte aligned)."""
+    buf = torch.empty((sum((n + 63) // 64 for n in sizes) * 64,), device=device, dtype=torch.float32)
+    return buf, stat_addresses(buf, sizes)
+
+
+def stat_addresses(buf, sizes):
+    """The addresses of stat_buffer's arrays."""
+    at, out = buf.data_ptr(), []
+    for n in sizes:
+        out.append(at)
+        at += (n + 63) // 64 * 256
+    return out
+
+
+def loss_grad(g: torch.Tensor) -> torch.Tensor:
+    """The gradient autograd hands to a backward, as the float32 the kernels read."""
+    if g.dtype == torch.float32 and g.is_contiguous():
+        return g
+    return g.detach().to(torch.float32).contiguous()
 
 
 def logits_desc(t: torch.Tensor) -> Logits:
     """A [B, K, V] tensor (a [R, V] one is read as B = 1, K = R)."""
     if t.ndim == 2:
         t = t.unsqueeze(0)
-    d = Logits()
-    d.data = t.data_ptr()
-    for i in range(3):
-        d.size[i] = t.shape[i]
-        d.stride[i] = t.stride(i)
-    d.dtype = LOGITS_DTYPE_CODES[t.dtype]
-    return d
+    return Logits.from_buffer_copy(_PACK3.pack(t.data_ptr(), *t.shape, *t.stride(), LOGITS_DTYPE_CODES[t.dtype]))
 
 
 def mask_desc(m) -> Mask:
-    d = Mask()
     if m is None:
-        d.data = None
-        d.kind = 0
-        return d
-    d.data = m.data_ptr()
-    d.kind = MASK_CODES[m.dtype]
-    for i in range(2):
-        d.size[i] = m.shape[i]
-        d.stride[i] = m.stride(i)
-    return d
+        return Mask()  # no data, kind 0
+    return Mask.from_buffer_copy(_PACK_MASK.pack(m.data_ptr(), MASK_CODES[m.dtype], *m.shape, *m.stride()))
 
 
 def stream_of(t: torch.Tensor) -> int:
     """The current torch stream of the tensor's device, as a hipStream_t."""
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.device.index)

@@ -55,33 +55,34 @@ def check_relations(qs, ks, qt, kt, strided_ok=False):
     accepted -- e.g. the [B,T,H,D] projections of train.py:133-142 seen as
     [B,H,T,D] -- and the library checks its alignment."""
     for t, n in ((qs, "qs"), (ks, "ks"), (qt, "qt"), (kt, "kt")):
-        require(isinstance(t, torch.Tensor), f"{n} must be a torch.Tensor")
+        if not isinstance(t, torch.Tensor):
+            raise AssertionError(f"{n} must be a torch.Tensor")
     require(qs.is_cuda and ks.is_cuda and qt.is_cuda and kt.is_cuda, "Q/K must be on CUDA")
-    require(qs.dtype in _INPUT_TYPES, "qs dtype supports only fp16/bf16/fp32")
-    require(ks.dtype in _INPUT_TYPES, "ks dtype supports only fp16/bf16/fp32")
-    require(qt.dtype in _INPUT_TYPES, "qt dtype supports only fp16/bf16/fp32")
-    require(kt.dtype in _INPUT_TYPES, "kt dtype supports only fp16/bf16/fp32")
-    require((qs.dtype == torch.float32) == (qt.dtype == torch.float32),
-            "float32 inputs need float32 on both sides")
-    require(qs.dtype == ks.dtype, "qs/ks dtype must match")
-    require(qt.dtype == kt.dtype, "qt/kt dtype must match")
-    require(qs.ndim == 4 and ks.ndim == 4, "qs/ks shape must be [B,H,T,Ds]")
-    require(qt.ndim == 4 and kt.ndim == 4, "qt/kt shape must be [B,H,T,Dt]")
-    require(qs.shape[0] == ks.shape[0], "qs/ks B must match")
-    require(qs.shape[2] == ks.shape[2], "qs/ks T must match")
-    require(qs.shape[3] == ks.shape[3], "qs/ks Ds must match")
-    require(qt.shape[0] == kt.shape[0], "qt/kt B must match")
-    require(qt.shape[2] == kt.shape[2], "qt/kt T must match")
-    require(qt.shape[3] == kt.shape[3], "qt/kt Dt must match")
+    tqs, tks, tqt, tkt = qs.dtype, ks.dtype, qt.dtype, kt.dtype
+    require(tqs in _INPUT_TYPES, "qs dtype supports only fp16/bf16/fp32")
+    require(tks in _INPUT_TYPES, "ks dtype supports only fp16/bf16/fp32")
+    require(tqt in _INPUT_TYPES, "qt dtype supports only fp16/bf16/fp32")
+    require(tkt in _INPUT_TYPES, "kt dtype supports only fp16/bf16/fp32")
+    require((tqs == torch.float32) == (tqt == torch.float32), "float32 inputs need float32 on both sides")
+    require(tqs == tks, "qs/ks dtype must match")
+    require(tqt == tkt, "qt/kt dtype must match")
+    nqs, nks, nqt, nkt = tuple(qs.shape), tuple(ks.shape), tuple(qt.shape), tuple(kt.shape)
+    require(len(nqs) == 4 and len(nks) == 4, "qs/ks shape must be [B,H,T,Ds]")
+    require(len(nqt) == 4 and len(nkt) == 4, "qt/kt shape must be [B,H,T,Dt]")
+    B, Hq, T, Ds = nqs
+    B2, Hq2, T2, Dt = nqt
+    require(B == nks[0], "qs/ks B must match")
+    require(T == nks[2], "qs/ks T must match")
+    require(Ds == nks[3], "qs/ks Ds must match")
+    require(B2 == nkt[0], "qt/kt B must match")
+    require(T2 == nkt[2], "qt/kt T must match")
+    require(Dt == nkt[3], "qt/kt Dt must match")
     if not strided_ok:
         require(qs.is_contiguous() and ks.is_contiguous(), "qs/ks must be contiguous")
         require(qt.is_contiguous() and kt.is_contiguous(), "qt/kt must be contiguous")
     require(qs.stride(-1) == 1 and ks.stride(-1) == 1, "qs/ks last-dim stride must be 1")
     require(qt.stride(-1) == 1 and kt.stride(-1) == 1, "qt/kt last-dim stride must be 1")
-    B, Hq, T, Ds = qs.shape
-    B2, Hq2, T2, Dt = qt.shape
-    Hkv_s = ks.shape[1]
-    Hkv_t = kt.shape[1]
+    Hkv_s, Hkv_t = nks[1], nkt[1]
     require((B, Hq, T) == (B2, Hq2, T2), "student/teacher B/Hq/T must align")
     require(Hkv_s > 0 and Hq % Hkv_s == 0, "Hq must be divisible by Hkv_s")
     require(Hkv_t > 0 and Hq % Hkv_t == 0, "Hq must be divisible by Hkv_t")

@@ -39,17 +39,6 @@ def _workspace(nbytes: int, device) -> torch.Tensor:
     return torch.empty((nbytes if nbytes > 0 else 1,), device=device, dtype=torch.uint8)
 
 
-def _relations(xs, xt, lse_s, lse_t, dxs=None):
-    arr = (_lib.Relation * len(xs))()
-    for r in range(len(xs)):
-        arr[r].xs = _lib.tensor4(xs[r])
-        arr[r].xt = _lib.tensor4(xt[r])
-        arr[r].lse_s = lse_s[r].data_ptr()
-        arr[r].lse_t = lse_t[r].data_ptr()
-        arr[r].dxs = None if dxs is None else dxs[r].data_ptr()
-    return arr
-
-
 class AttnKLBatchedFn(torch.autograd.Function):
     """Forward: sum_r w_r KL_r.  Backward: the gradient of every student
     tensor xs[r] (teachers, weights, mask, flags and scales get None)."""
@@ -69,8 +58,9 @@ class AttnKLBatchedFn(torch.autograd.Function):
         require(weights.shape == (n,), "weights must hold one value per relation")
 
         L = _lib.lib()
-        lse_s = [torch.empty(x.shape[:3], device=dev, dtype=torch.float32) for x in xs]
-        lse_t = [torch.empty(x.shape[:3], device=dev, dtype=torch.float32) for x in xs]
+        rows = [B * x.shape[1] * T for x in xs]
+        lse, at = _lib.stat_buffer(rows + rows, dev)
+        lse_s, lse_t = at[:n], at[n:]
         loss = torch.empty((), device=dev, dtype=torch.float32)
         md = _lib.mask_desc(attn_mask)
         stream = _lib.stream_of(xs[0])
@@ -80,7 +70,7 @@ class AttnKLBatchedFn(torch.autograd.Function):
             want_grad = any(ctx.needs_input_grad[6:6 + n])
             if want_grad:
                 row_grad = [torch.empty(x.shape, device=dev, dtype=torch.float32) for x in xs]
-            rels = _relations(xs, xt, lse_s, lse_t, row_grad)
+            rels = _lib.relations(xs, xt, lse_s, lse_t, row_grad and [x.data_ptr() for x in row_grad])
             ws_bytes = (L.lard_attn_kl_batched_rowgrad_workspace_bytes(rels, n) if want_grad
                         else L.lard_attn_kl_batched_workspace_bytes(rels, n))
             ws = _workspace(ws_bytes, dev)
@@ -102,16 +92,14 @@ class AttnKLBatchedFn(torch.autograd.Function):
                 d = [_lib.tensor4(x) for x in (xs[r], xt[r])]
                 rc = L.lard_attn_kl_forward(ctypes.byref(d[0]), ctypes.byref(d[0]), ctypes.byref(d[1]),
                                             ctypes.byref(d[1]), ctypes.byref(md), int(bool(causal)), ss[r], st[r],
-                                            lse_s[r].data_ptr(), lse_t[r].data_ptr(), losses[r:r + 1].data_ptr(),
+                                            lse_s[r], lse_t[r], losses[r:r + 1].data_ptr(),
                                             ws.data_ptr(), ws_bytes, stream)
                 _lib.check(rc, "lard_attn_kl_forward")
             loss = (losses * weights).sum()
 
-        saved_mask = attn_mask if attn_mask is not None else torch.empty(0, device=dev)
         ctx.has_row_grad = row_grad is not None
-        ctx.save_for_backward(weights, saved_mask, *xs, *xt, *lse_s, *lse_t, *(row_grad or []))
+        ctx.save_for_backward(weights, attn_mask, lse, *xs, *xt, *(row_grad or []))
         ctx.n = n
-        ctx.has_mask = attn_mask is not None
         ctx.causal = bool(causal)
         ctx.ss, ctx.st = ss, st
         ctx.batched = batched
@@ -121,17 +109,17 @@ class AttnKLBatchedFn(torch.autograd.Function):
     def backward(ctx, dloss):
         n = ctx.n
         saved = ctx.saved_tensors
-        weights, saved_mask = saved[0], saved[1]
-        xs, xt = saved[2:2 + n], saved[2 + n:2 + 2 * n]
-        lse_s, lse_t = saved[2 + 2 * n:2 + 3 * n], saved[2 + 3 * n:2 + 4 * n]
-        attn_mask = saved_mask if ctx.has_mask else None
-        dloss = dloss.detach().to(torch.float32).contiguous()
+        weights, attn_mask, lse = saved[:3]
+        xs, xt = saved[3:3 + n], saved[3 + n:3 + 2 * n]
+        at = _lib.stat_addresses(lse, [x.shape[0] * x.shape[1] * x.shape[2] for x in xs] * 2)
+        lse_s, lse_t = at[:n], at[n:]
+        dloss = _lib.loss_grad(dloss)
         dev = xs[0].device
         L = _lib.lib()
         md = _lib.mask_desc(attn_mask)
         stream = _lib.stream_of(xs[0])
         if ctx.has_row_grad:
-            rels = _relations(xs, xt, lse_s, lse_t, saved[2 + 4 * n:2 + 5 * n])
+            rels = _lib.relations(xs, xt, lse_s, lse_t, [x.data_ptr() for x in saved[3 + 2 * n:]])
             ws_bytes = L.lard_attn_kl_batched_workspace_bytes(rels, n)
             ws = _workspace(ws_bytes, dev)
             dxs = [torch.empty(x.shape, device=dev, dtype=x.dtype) for x in xs]
@@ -143,7 +131,7 @@ class AttnKLBatchedFn(torch.autograd.Function):
             return (None, None, None, None, None, None, *dxs, *([None] * n))
         dxs = [torch.empty(x.shape, device=dev, dtype=torch.float32) for x in xs]
         if ctx.batched:
-            rels = _relations(xs, xt, lse_s, lse_t, dxs)
+            rels = _lib.relations(xs, xt, lse_s, lse_t, [x.data_ptr() for x in dxs])
             ws_bytes = L.lard_attn_kl_batched_workspace_bytes(rels, n)
             ws = _workspace(ws_bytes, dev)
             rc = L.lard_attn_kl_batched_backward(rels, n, ctypes.byref(md), int(ctx.causal), ctx.ss[0], ctx.st[0],
@@ -158,8 +146,8 @@ class AttnKLBatchedFn(torch.autograd.Function):
                 ws = _workspace(ws_bytes, dev)
                 d = [_lib.tensor4(x) for x in (xs[r], xt[r])]
                 rc = L.lard_attn_kl_backward(
-                    ctypes.byref(d[0]), ctypes.byref(d[0]), lse_s[r].data_ptr(), ctypes.byref(d[1]),
-                    ctypes.byref(d[1]), lse_t[r].data_ptr(), ctypes.byref(md), int(ctx.causal), ctx.ss[r], ctx.st[r],
+                    ctypes.byref(d[0]), ctypes.byref(d[0]), lse_s[r], ctypes.byref(d[1]),
+                    ctypes.byref(d[1]), lse_t[r], ctypes.byref(md), int(ctx.causal), ctx.ss[r], ctx.st[r],
                     scaled[r:r + 1].data_ptr(), 1, None, dxs[r].data_ptr(), ws.data_ptr(), ws_bytes, stream)
                 _lib.check(rc, "lard_attn_kl_backward")
         return (None, None, None, None, None, None, *dxs, *([None] * n))
@@ -186,6 +174,29 @@ def attn_kl_align_batched(xs, xt, weights=None, attn_mask=None, causal=True, sm_
     return AttnKLBatchedFn.apply(weights, attn_mask, causal, sm_scale_s, sm_scale_t, len(xs), *xs, *xt)
 
 
+def denominators(qs, attn_mask, dev, repeat=1, fn=None):
+    """float32 [len(qs) * repeat]: ``fn`` of each layer's denom (train.py:403-406:
+    B * Hq * T, or mask.sum().clamp_min(1) * Hq with Hq the layer's query
+    heads), each ``repeat`` times.  Layers with the same denom share one, so the
+    launches do not grow with the layers."""
+    valid, made, out = None, {}, []
+    for q in qs:
+        B, Hq, T, _ = q.shape
+        key = Hq if attn_mask is not None else B * Hq * T
+        if key not in made:
+            if attn_mask is None:  # a fill on the device: a host tensor here would be a synchronising copy
+                d = torch.full((), float(key), device=dev, dtype=torch.float32)
+            else:
+                if valid is None:
+                    valid = attn_mask.sum().clamp_min(1).to(torch.float32)
+                d = valid * Hq
+            made[key] = d if fn is None else fn(d)
+        out += [made[key]] * repeat
+    if len(made) == 1:
+        return out[0].repeat(len(out))
+    return torch.stack(out)
+
+
 def relation_kl_loss(qs, ks, vs, qt, kt, vt, attn_mask=None, sm_scale_s=None, sm_scale_t=None):
     """The attention-relation loss of train.py:360-410 in batched launches.
 
@@ -202,18 +213,11 @@ def relation_kl_loss(qs, ks, vs, qt, kt, vt, attn_mask=None, sm_scale_s=None, sm
     dev = qs[0].device
     if attn_mask is not None and attn_mask.device != dev:
         attn_mask = attn_mask.to(dev)
-    xs, xt, w = [], [], []
+    xs, xt = [], []
     for layer in range(L):
-        B, Hq, T, _ = qs[layer].shape
-        if attn_mask is None:  # a fill on the device: a host tensor here would be a synchronising copy
-            denom = torch.full((), float(B * Hq * T), device=dev, dtype=torch.float32)
-        else:
-            denom = attn_mask.sum().clamp_min(1).to(torch.float32) * Hq
-        wl = 1.0 / (denom * max(1, L))
         for s_, t_ in ((qs[layer], qt[layer]), (ks[layer], kt[layer]), (vs[layer], vt[layer])):
             xs.append(s_)
             xt.append(t_)
-            w.append(wl)
-    weights = torch.stack(w).to(torch.float32)
+    weights = denominators(qs, attn_mask, dev, 3, lambda d: 1.0 / (d * L))
     return attn_kl_align_batched(xs, xt, weights, attn_mask=attn_mask, causal=True, sm_scale_s=sm_scale_s,
                                  sm_scale_t=sm_scale_t)

@@ -58,14 +58,23 @@ def kernel_path(d, ss: float, st: float):
     return PATH_NAMES[rc], L.lard_last_error().decode()
 
 
-def _warn_slow_path(d, ss: float, st: float) -> None:
-    """One RuntimeWarning per condition that moves a call off the throughput
-    kernels (the stage composition is about 4x slower at d=128)."""
+def _warn_slow_path(d, ss: float, st: float) -> str:
+    """The path's name, with one RuntimeWarning per condition that moves a call
+    off the throughput kernels (the stage composition is about 4x slower at d=128)."""
     name, why = kernel_path(d, ss, st)
     if name != "throughput" and why not in _WARNED:
         _WARNED.add(why)
         warnings.warn(f"attn_kl_align: {why}: these inputs run the {name} kernels, not the throughput "
                       f"kernels (several times slower)", RuntimeWarning, stacklevel=3)
+    return name
+
+
+def _descs(qs, ks, qt, kt):
+    """The operands' descriptors (one per tensor: a self relation has two)."""
+    d = [_lib.tensor4(qs), None, _lib.tensor4(qt), None]
+    d[1] = d[0] if ks is qs else _lib.tensor4(ks)
+    d[3] = d[2] if kt is qt else _lib.tensor4(kt)
+    return d
 
 
 class AttnKLAlignFn(torch.autograd.Function):
@@ -79,48 +88,38 @@ class AttnKLAlignFn(torch.autograd.Function):
 
         L = _lib.lib()
         dev = qs.device
-        lse_s = torch.empty((B, Hq, T), device=dev, dtype=torch.float32)
-        lse_t = torch.empty((B, Hq, T), device=dev, dtype=torch.float32)
+        rows = B * Hq * T
+        lse, (lse_s, lse_t) = _lib.stat_buffer((rows, rows), dev)
         loss = torch.empty((), device=dev, dtype=torch.float32)
-        ws_bytes = L.lard_attn_kl_forward_workspace_bytes(B, Hq, T)
-        ws = _workspace(ws_bytes, dev)
-        d = [_lib.tensor4(x) for x in (qs, ks, qt, kt)]
-        path = "throughput"
-        if B * Hq * T > 0:
-            _warn_slow_path(d, ss, st)
-            path = kernel_path(d, ss, st)[0]
+        d = _descs(qs, ks, qt, kt)
+        p = [ctypes.byref(x) for x in d]
+        path = _warn_slow_path(d, ss, st) if rows > 0 else "throughput"
         md = _lib.mask_desc(attn_mask)
+        stream = _lib.stream_of(qs)
         dq_row = lse64 = None
         needs_grad = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
-        if path == "throughput" and B * Hq * T > 0 and needs_grad:
+        row_side = path == "throughput" and rows > 0 and needs_grad
+        ws_bytes = (L.lard_attn_kl_forward_rowgrad_workspace_bytes(B, Hq, ks.shape[1], kt.shape[1], T, Ds) if row_side
+                    else L.lard_attn_kl_forward_workspace_bytes(B, Hq, T))
+        ws = _workspace(ws_bytes, dev)
+        if row_side:
             dq_row = torch.empty((B, Hq, T, Ds), device=dev, dtype=torch.float32)
-            ws_bytes = L.lard_attn_kl_forward_rowgrad_workspace_bytes(B, Hq, ks.shape[1], kt.shape[1], T, Ds)
-            ws = _workspace(ws_bytes, dev)
-            rc = L.lard_attn_kl_forward_rowgrad(
-                ctypes.byref(d[0]), ctypes.byref(d[1]), ctypes.byref(d[2]), ctypes.byref(d[3]), ctypes.byref(md),
-                int(bool(causal)), ss, st, lse_s.data_ptr(), lse_t.data_ptr(), loss.data_ptr(), dq_row.data_ptr(),
-                ws.data_ptr(), ws_bytes, _lib.stream_of(qs))
+            rc = L.lard_attn_kl_forward_rowgrad(*p, ctypes.byref(md), int(bool(causal)), ss, st, lse_s, lse_t,
+                                                loss.data_ptr(), dq_row.data_ptr(), ws.data_ptr(), ws_bytes, stream)
             _lib.check(rc, "lard_attn_kl_forward_rowgrad")
         elif path == "float32" and needs_grad:
             lse64 = torch.empty((2, B, Hq, T), device=dev, dtype=torch.float64)
-            rc = L.lard_attn_kl_forward_lse64(
-                ctypes.byref(d[0]), ctypes.byref(d[1]), ctypes.byref(d[2]), ctypes.byref(d[3]), ctypes.byref(md),
-                int(bool(causal)), ss, st, lse_s.data_ptr(), lse_t.data_ptr(), loss.data_ptr(), lse64.data_ptr(),
-                ws.data_ptr(), ws_bytes, _lib.stream_of(qs))
+            rc = L.lard_attn_kl_forward_lse64(*p, ctypes.byref(md), int(bool(causal)), ss, st, lse_s, lse_t,
+                                              loss.data_ptr(), lse64.data_ptr(), ws.data_ptr(), ws_bytes, stream)
             _lib.check(rc, "lard_attn_kl_forward_lse64")
         else:
-            rc = L.lard_attn_kl_forward(ctypes.byref(d[0]), ctypes.byref(d[1]), ctypes.byref(d[2]),
-                                        ctypes.byref(d[3]), ctypes.byref(md), int(bool(causal)), ss, st,
-                                        lse_s.data_ptr(), lse_t.data_ptr(), loss.data_ptr(), ws.data_ptr(), ws_bytes,
-                                        _lib.stream_of(qs))
+            rc = L.lard_attn_kl_forward(*p, ctypes.byref(md), int(bool(causal)), ss, st, lse_s, lse_t,
+                                        loss.data_ptr(), ws.data_ptr(), ws_bytes, stream)
             _lib.check(rc, "lard_attn_kl_forward")
 
-        saved_mask = attn_mask if attn_mask is not None else torch.empty(0, device=dev)
         ctx.has_row_grad = dq_row is not None
         ctx.has_lse64 = lse64 is not None
-        extra = dq_row if dq_row is not None else lse64 if lse64 is not None else torch.empty(0, device=dev)
-        ctx.save_for_backward(qs, ks, lse_s, qt, kt, lse_t, saved_mask, extra)
-        ctx.has_mask = attn_mask is not None
+        ctx.save_for_backward(qs, ks, qt, kt, lse, attn_mask, dq_row if dq_row is not None else lse64)
         ctx.causal = bool(causal)
         ctx.sm_scale_s = ss
         ctx.sm_scale_t = st
@@ -130,50 +129,39 @@ class AttnKLAlignFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dloss):
         """integration.py:48-67: stage C and the chain rule with dloss."""
-        qs, ks, lse_s, qt, kt, lse_t, saved_mask, extra = ctx.saved_tensors
-        dq_row = extra if ctx.has_row_grad else None
-        attn_mask = saved_mask if ctx.has_mask else None
-        dloss = dloss.detach().to(torch.float32).contiguous()
+        qs, ks, qt, kt, lse, attn_mask, extra = ctx.saved_tensors
+        dloss = _lib.loss_grad(dloss)
         B, Hq, T, Ds = qs.shape
+        Hkv = ks.shape[1]
         self_rel = ctx.self_relation
         dev = qs.device
         L = _lib.lib()
-        d = [_lib.tensor4(x) for x in (qs, ks, qt, kt)]
+        ps, pk, pt, pkt = [ctypes.byref(x) for x in _descs(qs, ks, qt, kt)]
+        lse_s, lse_t = _lib.stat_addresses(lse, (B * Hq * T,) * 2)
         md = _lib.mask_desc(attn_mask)
-        if not ctx.has_lse64:
-            ws_bytes = L.lard_attn_kl_backward_workspace_bytes(B, Hq, ks.shape[1], T, Ds, int(self_rel))
-            ws = _workspace(ws_bytes, dev)
-        if ctx.has_row_grad:
-            # the row side came with the forward: the column side adds itself
-            # to it (self relation), or it becomes dq; both in the inputs' dtype
-            dk = torch.empty((B, ks.shape[1], T, Ds), device=dev, dtype=qs.dtype)
-            dq = None if self_rel else torch.empty((B, Hq, T, Ds), device=dev, dtype=qs.dtype)
-            rc = L.lard_attn_kl_backward_colgrad16(
-                ctypes.byref(d[0]), ctypes.byref(d[1]), lse_s.data_ptr(), ctypes.byref(d[2]), ctypes.byref(d[3]),
-                lse_t.data_ptr(), ctypes.byref(md), int(ctx.causal), ctx.sm_scale_s, ctx.sm_scale_t,
-                dloss.data_ptr(), int(self_rel), dq_row.data_ptr(), None if dq is None else dq.data_ptr(),
-                dk.data_ptr(), ws.data_ptr(), ws_bytes, _lib.stream_of(qs))
-            _lib.check(rc, "lard_attn_kl_backward_colgrad16")
-            return (dk if self_rel else dq), (None if self_rel else dk), None, None, None, None, None, None
-        dk = torch.empty((B, ks.shape[1], T, Ds), device=dev, dtype=torch.float32)
-        dq = None if self_rel else torch.empty((B, Hq, T, Ds), device=dev, dtype=torch.float32)
+        stream = _lib.stream_of(qs)
+        head = (ps, pk, lse_s, pt, pkt, lse_t)
+        opts = (ctypes.byref(md), int(ctx.causal), ctx.sm_scale_s, ctx.sm_scale_t, dloss.data_ptr(), int(self_rel))
+        # the row side may have come with the forward: the column side then adds
+        # itself to it (self relation), or it becomes dq; both in the inputs' dtype
+        dtype = qs.dtype if ctx.has_row_grad else torch.float32
+        dk = torch.empty((B, Hkv, T, Ds), device=dev, dtype=dtype)
+        dq = None if self_rel else torch.empty((B, Hq, T, Ds), device=dev, dtype=dtype)
+        out = (None if dq is None else dq.data_ptr(), dk.data_ptr())
         if ctx.has_lse64:  # float32 inputs: the forward kept its LSEs in double
-            rc = L.lard_attn_kl_backward_lse64(
-                ctypes.byref(d[0]), ctypes.byref(d[1]), lse_s.data_ptr(), ctypes.byref(d[2]), ctypes.byref(d[3]),
-                lse_t.data_ptr(), extra.data_ptr(), ctypes.byref(md), int(ctx.causal), ctx.sm_scale_s, ctx.sm_scale_t,
-                dloss.data_ptr(), int(self_rel), None if dq is None else dq.data_ptr(), dk.data_ptr(),
-                _lib.stream_of(qs))
+            rc = L.lard_attn_kl_backward_lse64(*head, extra.data_ptr(), *opts, *out, stream)
             _lib.check(rc, "lard_attn_kl_backward_lse64")
-            return (dk if self_rel else dq), (None if self_rel else dk), None, None, None, None, None, None
-        rc = L.lard_attn_kl_backward(
-            ctypes.byref(d[0]), ctypes.byref(d[1]), lse_s.data_ptr(), ctypes.byref(d[2]), ctypes.byref(d[3]),
-            lse_t.data_ptr(), ctypes.byref(md), int(ctx.causal), ctx.sm_scale_s, ctx.sm_scale_t, dloss.data_ptr(),
-            int(self_rel), None if dq is None else dq.data_ptr(), dk.data_ptr(), ws.data_ptr(), ws_bytes,
-            _lib.stream_of(qs))
-        _lib.check(rc, "lard_attn_kl_backward")
-        if self_rel:
-            return dk, None, None, None, None, None, None, None
-        return dq, dk, None, None, None, None, None, None
+        else:
+            ws_bytes = L.lard_attn_kl_backward_workspace_bytes(B, Hq, Hkv, T, Ds, int(self_rel))
+            ws = _workspace(ws_bytes, dev)
+            if ctx.has_row_grad:
+                rc = L.lard_attn_kl_backward_colgrad16(*head, *opts, extra.data_ptr(), *out, ws.data_ptr(), ws_bytes,
+                                                       stream)
+                _lib.check(rc, "lard_attn_kl_backward_colgrad16")
+            else:
+                rc = L.lard_attn_kl_backward(*head, *opts, *out, ws.data_ptr(), ws_bytes, stream)
+                _lib.check(rc, "lard_attn_kl_backward")
+        return (dk if self_rel else dq), (None if self_rel else dk), None, None, None, None, None, None
 
 
 def attn_kl_align(qs, ks, qt, kt, attn_mask=None, causal=True, sm_scale_s=None, sm_scale_t=None):

@@ -34,6 +34,7 @@ import torch
 
 from .attention_KL import attn_kl_align_batched
 from .attention_KL._checks import require
+from .attention_KL.batched import denominators
 from .logits_kl import logits_kl
 
 __all__ = ["DistillLoss", "distillation_loss"]
@@ -46,18 +47,6 @@ class DistillLoss(NamedTuple):
     Q_loss: torch.Tensor        # sum over layers of the Q/Q KL / denom (train.py:407)
     K_loss: torch.Tensor
     V_loss: torch.Tensor
-
-
-def _denoms(xs: Sequence[torch.Tensor], attn_mask, dev):
-    """denom of every layer (train.py:403-406), as float32 device scalars."""
-    out = []
-    for q in xs:
-        B, Hq, T, _ = q.shape
-        if attn_mask is None:  # a device fill, not a host tensor (no synchronising copy)
-            out.append(torch.full((), float(B * Hq * T), device=dev, dtype=torch.float32))
-        else:
-            out.append(attn_mask.sum().clamp_min(1).to(torch.float32) * Hq)
-    return out
 
 
 def distillation_loss(qs: Sequence[torch.Tensor], ks: Sequence[torch.Tensor], vs: Sequence[torch.Tensor],
@@ -81,7 +70,7 @@ def distillation_loss(qs: Sequence[torch.Tensor], ks: Sequence[torch.Tensor], vs
     dev = qs[0].device
     if attn_mask is not None and attn_mask.device != dev:
         attn_mask = attn_mask.to(dev)
-    w = torch.stack(_denoms(qs, attn_mask, dev)).reciprocal()   # 1 / denom per layer
+    w = denominators(qs, attn_mask, dev, fn=torch.reciprocal)   # 1 / denom per layer
 
     def kind(xs_, xt_):
         return attn_kl_align_batched(list(xs_), list(xt_), w, attn_mask=attn_mask, causal=True,

@@ -50,7 +50,7 @@ def _aligned(x: torch.Tensor) -> torch.Tensor:
 
 def _padded_empty(shape, dtype, device) -> torch.Tensor:
     """Uninitialised tensor of `shape` whose rows are 16-byte aligned."""
-    vec = 16 // torch.empty((), dtype=dtype).element_size()
+    vec = 16 // dtype.itemsize
     V = shape[-1]
     Vp = (V + vec - 1) // vec * vec
     buf = torch.empty((*shape[:-1], Vp), device=device, dtype=dtype)
@@ -81,19 +81,18 @@ class LogitsKLFn(torch.autograd.Function):
         B, K, V = t.shape
         rows = B * K
         dev = t.device
-        lse_t = torch.empty((rows,), device=dev, dtype=torch.float32)
-        lse_s = torch.empty((rows,), device=dev, dtype=torch.float32)
+        lse, (lse_t, lse_s) = _lib.stat_buffer((rows, rows), dev)
         kl_rows = torch.empty((rows,), device=dev, dtype=torch.float32)
         loss = torch.empty((), device=dev, dtype=torch.float32)
         L = _lib.lib()
         ws_bytes = L.lard_logits_kl_workspace_bytes(rows, V)
         ws = torch.empty((max(ws_bytes, 16),), device=dev, dtype=torch.uint8)
         dt, ds = _lib.logits_desc(t), _lib.logits_desc(s)
-        rc = L.lard_logits_kl_forward(ctypes.byref(dt), ctypes.byref(ds), T, lse_t.data_ptr(), lse_s.data_ptr(),
+        rc = L.lard_logits_kl_forward(ctypes.byref(dt), ctypes.byref(ds), T, lse_t, lse_s,
                                       kl_rows.data_ptr(), loss.data_ptr(), ws.data_ptr(), ws_bytes,
                                       _lib.stream_of(t))
         _lib.check(rc, "lard_logits_kl_forward")
-        ctx.save_for_backward(t, s, lse_t, lse_s, kl_rows)
+        ctx.save_for_backward(t, s, lse, kl_rows)
         ctx.temperature = T
         ctx.reduction = reduction
         ctx.in_shape = t_logits.shape
@@ -103,13 +102,14 @@ class LogitsKLFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        t, s, lse_t, lse_s, kl_rows = ctx.saved_tensors
+        t, s, lse, kl_rows = ctx.saved_tensors
         need_t, need_s = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         if not (need_t or need_s):
             return None, None, None, None
         B, K, V = t.shape
         rows = B * K
-        g = g.detach().to(torch.float32).contiguous()
+        g = _lib.loss_grad(g)
+        lse_t, lse_s = _lib.stat_addresses(lse, (rows, rows))
         if ctx.reduction == "mean":
             per_row, row_scale = 0, (1.0 / rows if rows > 0 else 0.0)
         else:
@@ -121,7 +121,7 @@ class LogitsKLFn(torch.autograd.Function):
         L = _lib.lib()
         dt, ds = _lib.logits_desc(t), _lib.logits_desc(s)
         rc = L.lard_logits_kl_backward(
-            ctypes.byref(dt), ctypes.byref(ds), ctx.temperature, lse_t.data_ptr(), lse_s.data_ptr(),
+            ctypes.byref(dt), ctypes.byref(ds), ctx.temperature, lse_t, lse_s,
             kl_rows.data_ptr(), g.data_ptr(), per_row, row_scale,
             ctypes.byref(dgt) if dgt is not None else None, ctypes.byref(dgs) if dgs is not None else None,
             _lib.stream_of(t))

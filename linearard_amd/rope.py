@@ -143,8 +143,9 @@ def _length_key(rope_scaling, seq_len, max_position_embeddings):
 
 def _cached_parameters(dim, base, rope_scaling, max_position_embeddings, seq_len, device):
     """rope_parameters with the table moved to `device`, from a bounded LRU cache."""
-    key = (dim, float(base), json.dumps(rope_scaling, sort_keys=True), max_position_embeddings,
-           _length_key(rope_scaling, seq_len, max_position_embeddings), str(device))
+    length = None if rope_scaling is None else _length_key(rope_scaling, seq_len, max_position_embeddings)
+    key = (dim, float(base), None if rope_scaling is None else json.dumps(rope_scaling, sort_keys=True),
+           max_position_embeddings, length, device if isinstance(device, str) else (device.type, device.index))
     hit = _FREQ_CACHE.get(key)
     if hit is not None:
         _FREQ_CACHE.move_to_end(key)

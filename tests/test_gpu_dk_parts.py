@@ -137,7 +137,7 @@ def test_batched_gradients_against_the_general_batched_backward(gpu_available):
     """Autograd's batched gradients (input dtype, row side from the forward)
     and lard_attn_kl_batched_backward (both sides recomputed) agree within the
     gradient bar, relation by relation."""
-    from linearard_amd.attention_KL.batched import _relations, attn_kl_align_batched
+    from linearard_amd.attention_KL.batched import attn_kl_align_batched
 
     rng = np.random.default_rng(77)
     B, T, D, heads = 2, 200, 64, [4, 1, 2]
@@ -152,7 +152,7 @@ def test_batched_gradients_against_the_general_batched_backward(gpu_available):
     lse_s = [torch.empty(x.shape[:3], device="cuda") for x in s]
     lse_t = [torch.empty(x.shape[:3], device="cuda") for x in s]
     dx = [torch.empty(x.shape, device="cuda") for x in s]
-    rels = _relations(s, xt, lse_s, lse_t, dx)
+    rels = _lib.relations(s, xt, *([t.data_ptr() for t in ts] for ts in (lse_s, lse_t, dx)))
     nb = L.lard_attn_kl_batched_workspace_bytes(rels, n)
     ws = torch.empty((nb,), device="cuda", dtype=torch.uint8)
     out, one = torch.empty((), device="cuda"), torch.ones((), device="cuda")
