@@ -39,7 +39,7 @@ __global__ __launch_bounds__(kStageThreads, 2) void fused_fwd_kernel(const Fused
   const int T = a.T;
   const int nrb = (T + kStageRows - 1) / kStageRows;
   int blk, bh;
-  stage_item(blk, bh);
+  stage_item(blk, bh, a.causal, (int)(sizeof(lks) + sizeof(lkt)));
   const int rb = nrb - 1 - blk;  // longest causal rows first
   const int b = bh / a.Hq;
   const int h = bh - b * a.Hq;

@@ -97,7 +97,7 @@ hipError_t launch_row_prep(RowPrepBatch& p, int B, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// One flat grid; the kernels map blockIdx.x to work items with xcd_item().
+// One flat grid; the kernels map blockIdx.x to work items with work_item().
 #define LARD_HOT_DISPATCH(KERNEL)                                                                    \
   template <bool BF>                                                                                 \
   static hipError_t KERNEL##_dispatch(const HotArgs& f, int dp, int nblocks, hipStream_t stream) {  \

@@ -692,11 +692,11 @@ __host__ __device__ inline int fwdq_items(const HotArgs& f) { return (f.r.T + kR
 
 template <int DP, bool BF>
 __global__ __launch_bounds__(kWavesQ * 64) void hot_fwdq_kernel(const HotArgs f) {
-  hot_fwdq_body<DP, BF>(f, xcd_item(blockIdx.x, fwdq_items(f)));
+  hot_fwdq_body<DP, BF>(f, rel_item<DP>(f, fwdq_items(f), kRowsQ));
 }
 template <int DP, bool BF>
 __global__ __launch_bounds__(kWavesQ * 64) void hot_fwdq_batch_kernel(const HotBatch m) {
-  const int g = xcd_item(blockIdx.x, m.first[m.n]);
+  const int g = batch_item<DP>(m, kRowsQ);
   const int r = batch_relation(m, g);
   hot_fwdq_body<DP, BF>(m.rel[r], g - m.first[r]);
 }

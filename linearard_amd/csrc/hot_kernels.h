@@ -996,33 +996,49 @@ __device__ __forceinline__ int batch_relation(const HotBatch& m, int g) {
   return r;
 }
 
+// Workgroups of a throughput kernel that share a CU: the rings of the 128-wide
+// kernels fill its LDS.
+constexpr int hot_wgs(int dp) { return dp >= 128 ? 1 : 2; }
+
+// The workgroup's item of a batch (the relations share T, so one list of heads
+// with the same blocks) and of one relation.
+template <int DP>
+__device__ __forceinline__ int batch_item(const HotBatch& m, int rows) {
+  const RelArgs& a = m.rel[0].r;
+  return work_item(blockIdx.x, m.first[m.n], (a.T + rows - 1) / rows, a.causal, hot_wgs(DP));
+}
+template <int DP>
+__device__ __forceinline__ int rel_item(const HotArgs& f, int n, int rows) {
+  return work_item(blockIdx.x, n, (f.r.T + rows - 1) / rows, f.r.causal, hot_wgs(DP));
+}
+
 template <int DP, bool BF>
 __global__ __launch_bounds__(kWaves * 64) void hot_fwd_kernel(const HotArgs f) {
-  hot_fwd_body<DP, BF>(f, xcd_item(blockIdx.x, fwd_items(f)));
+  hot_fwd_body<DP, BF>(f, rel_item<DP>(f, fwd_items(f), kRows));
 }
 template <int DP, bool BF>
 __global__ __launch_bounds__(kWaves * 64) void hot_dq_kernel(const HotArgs f) {
-  hot_dq_body<DP, BF>(f, xcd_item(blockIdx.x, fwd_items(f)));
+  hot_dq_body<DP, BF>(f, rel_item<DP>(f, fwd_items(f), kRows));
 }
 template <int DP, bool BF>
 __global__ __launch_bounds__(kWaves * 64) void hot_bwd_kernel(const HotArgs f) {
-  hot_bwd_body<DP, BF>(f, xcd_item(blockIdx.x, bwd_items(f)));
+  hot_bwd_body<DP, BF>(f, rel_item<DP>(f, bwd_items(f), kRows));
 }
 template <int DP, bool BF>
 __global__ __launch_bounds__(kWaves * 64) void hot_fwd_batch_kernel(const HotBatch m) {
-  const int g = xcd_item(blockIdx.x, m.first[m.n]);
+  const int g = batch_item<DP>(m, kRows);
   const int r = batch_relation(m, g);
   hot_fwd_body<DP, BF>(m.rel[r], g - m.first[r]);
 }
 template <int DP, bool BF>
 __global__ __launch_bounds__(kWaves * 64) void hot_dq_batch_kernel(const HotBatch m) {
-  const int g = xcd_item(blockIdx.x, m.first[m.n]);
+  const int g = batch_item<DP>(m, kRows);
   const int r = batch_relation(m, g);
   hot_dq_body<DP, BF>(m.rel[r], g - m.first[r]);
 }
 template <int DP, bool BF>
 __global__ __launch_bounds__(kWaves * 64) void hot_bwd_batch_kernel(const HotBatch m) {
-  const int g = xcd_item(blockIdx.x, m.first[m.n]);
+  const int g = batch_item<DP>(m, kRows);
   const int r = batch_relation(m, g);
   hot_bwd_body<DP, BF>(m.rel[r], g - m.first[r]);
 }

@@ -22,6 +22,53 @@ __device__ __forceinline__ int xcd_item(int bid, int n) {
   return x * base + min(x, rem) + m;
 }
 
+// CUs of an XCD, LDS of a CU, and the workgroups with `bytes` of it that share
+// a CU (at most `most`).
+constexpr int kXcdCus = 32;
+constexpr int kCuLds = 160 * 1024;
+constexpr int wgs_per_cu(int bytes, int most) { return kCuLds / bytes < most ? (kCuLds / bytes > 1 ? kCuLds / bytes : 1) : most; }
+
+// The same for a causal list of n = heads * nblk items, where item h * nblk + i
+// is head h's i-th longest block (lengths nblk, nblk - 1, ..., 1) and a CU
+// holds `wgs` workgroups at once.  Taken head after head, the longest block of
+// an XCD's last head starts when the CUs have only short ones left beside it:
+// 16 blocks, 4 heads an XCD end after 25 units of 17.  So
+// - an XCD works on as many heads together as make two rounds of its
+//   workgroups, longest blocks of all of them first (longer heads one by one:
+//   128 blocks already end level, and fewer heads share the L2);
+// - heads that do not divide by the XCDs are dealt block by block over all
+//   XCDs first (dealt in runs, one XCD got a head's long half: 236 units of
+//   204 at 12 heads of 16 blocks);
+// - if everything is resident at once, the second round runs backwards: a CU
+//   then shares a long block with a short one.
+// Before -> after, us: dk of 32 heads at T 4096, D 128 (16 blocks) 320 -> 239,
+// of 16 x 2 heads at T 1531, D 64 48 -> 38; the forward of that call 74 -> 58,
+// of 16 heads at T 4096, D 256 379 -> 303; 64 + 2 * 16 heads of T 2048 in one
+// batch 714 -> 669 (forward), 470 -> 422 (dk); 32 heads at T 8192 854 -> 783.
+__host__ __device__ __forceinline__ int causal_item(int bid, int n, int nblk, int wgs) {
+  const int heads = n / nblk, own = heads / kXcds, left = heads - kXcds * own;
+  const int x = bid % kXcds, dealt = (left * nblk + kXcds - 1 - x) / kXcds;
+  int k = bid / kXcds;
+  if (k < dealt) {
+    const int m = x + kXcds * k;
+    return (kXcds * own + m % left) * nblk + m / left;
+  }
+  k -= dealt;
+  const int many = (2 * wgs * kXcdCus + nblk) / (nblk + 1);  // heads together
+  const int groups = own >= 2 * many ? own / many : 1;
+  const int g = min(k / (many * nblk), groups - 1);
+  const int h0 = g * many, size = g == groups - 1 ? own - h0 : many;  // the last group takes the rest
+  int m = k - h0 * nblk;
+  if (dealt + own * nblk <= wgs * kXcdCus && (m / kXcdCus & 1)) {
+    const int row = m / kXcdCus * kXcdCus;
+    m = row + min(kXcdCus, own * nblk - row) - 1 - (m - row);
+  }
+  return (x * own + h0 + m % size) * nblk + m / size;
+}
+
+__device__ __forceinline__ int work_item(int bid, int n, int nblk, int causal, int wgs) {
+  return causal ? causal_item(bid, n, nblk, wgs) : xcd_item(bid, n);
+}
 
 // LDS byte address of a pointer into a __shared__ array.  Taken where the
 // array itself is named (lds_addr(lk[buf][0])), the cast folds to the

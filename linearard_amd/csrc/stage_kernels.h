@@ -64,8 +64,10 @@ inline int stage_types(const RelArgs& a, bool two_sided) {
 // head's tiles that all its workgroups walk.  (With heads dealt round robin
 // every XCD streamed every head from beyond its L2: at D = 256, B=1, H=16,
 // n=4096 dq took 451 us against 297, dk 590 against 354.)
-__device__ __forceinline__ void stage_item(int& blk, int& head) {
-  const int item = xcd_item((int)(blockIdx.y * gridDim.x + blockIdx.x), (int)(gridDim.x * gridDim.y));
+// lds: the kernel's bytes of it, which say how many workgroups share a CU.
+__device__ __forceinline__ void stage_item(int& blk, int& head, int causal, int lds) {
+  const int item = work_item((int)(blockIdx.y * gridDim.x + blockIdx.x), (int)(gridDim.x * gridDim.y), (int)gridDim.x,
+                             causal, wgs_per_cu(lds, 4));
   head = item / (int)gridDim.x;
   blk = item - head * (int)gridDim.x;
 }
@@ -249,7 +251,7 @@ __global__ __launch_bounds__(kStageThreads, DPS <= 128 || MODE != MODE_DQ ? 2 : 
   const int T = a.T;
   const int nrb = (T + kStageRows - 1) / kStageRows;
   int blk, bh;
-  stage_item(blk, bh);
+  stage_item(blk, bh, a.causal, (int)(sizeof(lks) + sizeof(lkt)));
   const int rb = nrb - 1 - blk;  // longest causal rows first
   const int b = bh / a.Hq;
   const int h = bh - b * a.Hq;
@@ -482,7 +484,7 @@ __global__ __launch_bounds__(kStageThreads, DPS <= 128 ? 2 : 1) void col_kernel(
   const int l32 = lane & 31;
   const int T = a.T;
   int cb, bgp;  // small cb = longest causal columns, launched first
-  stage_item(cb, bgp);
+  stage_item(cb, bgp, a.causal, (int)(sizeof(lqs) + sizeof(lqt)));
   // the part of this key block's sum (RelArgs::dk_part), or all of it
   const int split = a.dk_part != nullptr ? a.dk_split : 1, parts = dk_parts(a);
   const int bg = bgp / parts;
