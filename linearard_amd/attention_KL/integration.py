@@ -60,7 +60,7 @@ def kernel_path(d, ss: float, st: float):
 
 def _warn_slow_path(d, ss: float, st: float) -> str:
     """The path's name, with one RuntimeWarning per condition that moves a call
-    off the throughput kernels (the stage composition is about 4x slower at d=128)."""
+    off the throughput kernels."""
     name, why = kernel_path(d, ss, st)
     if name != "throughput" and why not in _WARNED:
         _WARNED.add(why)
