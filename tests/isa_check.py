@@ -1,16 +1,19 @@
-"""Static checks on the gfx950 assembly of the throughput kernels (CPU only).
+"""Static checks on the gfx950 assembly of the kernels (CPU only).
 
 Three properties of the device code, checked on its assembly:
 
 * No writes through the scalar data cache anywhere (every kernel of every
-  source): device code writes memory through vector stores only.
+  source): device code writes memory through vector stores only.  Checked by
+  what is allowed: a scalar instruction is a load, works on registers, or
+  controls the wave.
 
 Two hazards the compiler cannot police for code it did not write itself:
 
-* M0.  The HBM->LDS copies (``lds_async16``, inline asm) write M0, which the
+* M0.  The HBM->LDS copies (``lds_async16``, ``lds_async16_at``,
+  ``lds_async4_at``, inline asm) write M0, which the
   compiler reserves.  The kernels are correct only while nothing else in them
   uses M0: every instruction that names ``m0`` must be that copy sequence
-  (``s_mov_b32 m0, ...`` / ``s_nop 0`` / ``global_load_lds_dwordx4``), and no
+  (``s_mov_b32 m0, ...`` / ``s_nop 0`` / ``global_load_lds_dword[x4]``), and no
   instruction that reads M0 implicitly (movrel, gpr_idx, sendmsg, GWS,
   ``*_addtid``, interpolation) may appear at all.
 
@@ -32,10 +35,10 @@ from __future__ import annotations
 
 import os
 import re
+import shlex
 import subprocess
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 # gfx950, 8-pass XDL (v_mfma_f32_32x32x16_*): result -> VALU / memory read or
 # write needs 11 + 1 wait states and 16-pass ones 19; checking 19 covers both.
@@ -43,20 +46,28 @@ RESULT_WAIT = 19
 # VALU write of a VGPR -> MFMA reads it: 2 wait states.
 OPERAND_WAIT = 2
 
-# Writes through the scalar data cache (scalar stores and atomics, the
-# cache's write-back and discard): none may appear in any kernel.
-SCALAR_WRITE = re.compile(r"^(s_store|s_buffer_store|s_scratch_store|s_atomic|s_buffer_atomic|s_dcache_wb"
-                          r"|s_dcache_discard)")
+# Scalar instructions that write no memory: those on registers (their names end
+# in the operands' type), the loads, and the wave's control flow and waits.
+SCALAR_OK = re.compile(r"^s_(\w+_[iub](8|16|32|64)|(buffer_)?load_dword(x\d+)?|barrier|branch|cbranch_\w+|endpgm|nop"
+                       r"|setprio|sleep|waitcnt|memtime|memrealtime)$")
+
+COPIES = ("global_load_lds_dwordx4", "global_load_lds_dword")
 
 IMPLICIT_M0 = re.compile(r"^(v_movrel|s_movrel|s_set_gpr_idx|s_sendmsg|ds_gws|v_interp|ds_\w*addtid|s_ttracedata)")
 
 
 def device_asm(src: str, out_dir: str) -> str:
-    """gfx950 assembly of one HIP source (compiled like the Makefile does)."""
+    """gfx950 assembly of one HIP source, with the Makefile's command line for it."""
     os.makedirs(out_dir, exist_ok=True)
-    out = os.path.join(out_dir, os.path.basename(src) + ".s")
-    cmd = [HIPCC, *FLAGS, "--cuda-device-only", "-S", src, "-o", out]
-    subprocess.run(cmd, check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+    base, name = os.path.split(src)
+    out = os.path.join(os.path.abspath(out_dir), name + ".s")
+    made = subprocess.run(["make", "-n", "-B", "-s", "-C", base, f"HIPCC={HIPCC}", f"_build/{name[:-4]}.o"], check=True,
+                          capture_output=True, text=True).stdout
+    cmd, = [shlex.split(ln) for ln in made.splitlines() if ln.startswith(HIPCC)]
+    cut = cmd.index("-c")
+    assert cmd[cut + 1] == name and cmd[cut + 2] == "-o", cmd
+    cmd[cut:] = ["--cuda-device-only", "-S", name, "-o", out]
+    subprocess.run(cmd, check=True, cwd=base, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
     with open(out, "r", encoding="utf-8") as f:
         return f.read()
 
@@ -131,15 +142,15 @@ def check_m0(name: str, body) -> list:
             errs.append(f"{name}: {t!r} reads M0 implicitly")
         if any(o == "m0" for o in ops):
             ok = (op == "s_mov_b32" and ops[0] == "m0" and i + 2 < len(insts) and insts[i + 1] == "s_nop 0"
-                  and insts[i + 2].startswith("global_load_lds_dwordx4"))
+                  and _operands(insts[i + 2])[0] in COPIES)
             if not ok:
                 errs.append(f"{name}: {t!r} uses M0 outside the HBM->LDS copy sequence")
     return errs
 
 
 def check_no_scalar_writes(name: str, body) -> list:
-    return [f"{name}: {t!r} writes through the scalar data cache" for k, t in body
-            if k == "inst" and SCALAR_WRITE.match(_operands(t)[0])]
+    return [f"{name}: {t!r} may write through the scalar data cache" for k, t in body
+            if k == "inst" and t.startswith("s_") and not SCALAR_OK.match(_operands(t)[0])]
 
 
 def _successors(body, pos):
