@@ -161,7 +161,10 @@ __device__ __forceinline__ double exp_d(double x, bool valid, const double* tab)
   return __builtin_ldexp(__builtin_fma(t, p * r, t), k >> 6);
 }
 
-// Online log-sum-exp of this lane's quarter of a row, in double.
+// Online log-sum-exp of this lane's quarter of a row, in double.  A NaN score
+// makes the row's sum NaN and its LSE -inf, whichever lane and tile it falls
+// in (the row then leaves the loss and the gradients): before a lane's first
+// finite score r holds it, and no factor below clears it.
 struct OnlineLse {
   double m = kNegInfD, r = 0.0;
   // Raises the maximum to the tile's; returns the factor of earlier terms.
@@ -172,8 +175,12 @@ struct OnlineLse {
     double f = 1.0;
     if (mb > m) {
       f = exp_d(m - mb, m != kNegInfD, tab);
-      r = m == kNegInfD ? 0.0 : r * f;
+      r *= f;
       m = mb;
+    }
+    if (m == kNegInfD) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) r = valid[q] && x[q >> 2][q & 3] != x[q >> 2][q & 3] ? x[q >> 2][q & 3] : r;
     }
     return f;
   }
@@ -191,7 +198,7 @@ struct OnlineLse {
     o = xor_lanes(mm, 32);
     mm = o > mm ? o : mm;
     const double f = exp_d(m - mm, m != kNegInfD, tab);
-    r = m == kNegInfD ? 0.0 : r * f;
+    r *= f;
     r += xor_lanes(r, 16);
     r += xor_lanes(r, 32);
     m = mm;

@@ -205,3 +205,33 @@ def test_f32_needs_f32_on_both_sides(gpu_available):
     y = torch.zeros((1, 2, 8, 16), device="cuda", dtype=torch.bfloat16)
     with pytest.raises(AssertionError, match="float32 on both sides"):
         attn_kl_align(x, x, y, y)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("pad,bad", [(0, 0), (0, 2), (0, 5), (37, 38), (37, 40), (0, 33)])
+def test_a_nan_score_takes_its_rows_out(gpu_available, causal, pad, bad):
+    """A NaN key makes the LSE of every row that sees it -inf, also where it is
+    the first or only score of a lane (lanes hold every fourth key); such rows
+    leave the loss, and the others are those of the tokens before it."""
+    from linearard_amd.attention_KL import attn_kl_align, lse_stats
+
+    rng = np.random.default_rng(bad)
+    B, H, T, D = 1, 2, 70, 64
+    qs, ks, qt, kt, _ = _inputs(rng, B, H, H, H, T, D, D, None)
+    mask = np.ones((B, T), np.int32)
+    mask[:, :pad] = 0
+    a = 1 / math.sqrt(D)
+    seen = bad if causal else 0  # rows before `seen` do not see the key
+    ref = O.lse_stats(qs[:, :, :seen], ks[:, :, :seen], mask[:, :seen], causal, a) if seen > pad else None
+    for side in (0, 1):
+        x = [to_dev(v, "f32") for v in (qs, ks, qt, kt)]
+        x[2 * side + 1][:, :, bad] = float("nan")
+        m = mask_to_dev(mask)
+        lse = lse_stats(x[2 * side], x[2 * side + 1], m, causal, a).cpu().numpy()
+        assert (lse[:, :, max(seen, pad):] == -np.inf).all()
+        assert (lse[:, :, :pad] == 0).all()
+        if side == 0 and ref is not None:
+            np.testing.assert_allclose(lse[:, :, pad:seen], ref[:, :, pad:], rtol=1e-6, atol=1e-5)
+        want = (float(attn_kl_align(*(v[:, :, :seen].contiguous() for v in x), attn_mask=m[:, :seen].contiguous(),
+                                    causal=causal)) if seen > pad else 0.0)
+        assert float(attn_kl_align(*x, attn_mask=m, causal=causal)) == pytest.approx(want, rel=1e-6, abs=0)
