@@ -147,9 +147,15 @@ constexpr double kNegInfD = -__builtin_inf();
 // overlap the double matrix products here (they take the sum of their times),
 // so its length counts: 12 double instructions against 25 for the series over
 // |r| <= ln(2) / 2 and more for the library's exp.
+// ABOVE: x may lie above 0, as a score against a given LSE may (against a
+// running maximum it does not).  n is then held at 2^20, where the result is
+// inf whatever r is: unbounded, x = inf has r = inf - inf, and a large x
+// leaves the int's range.
+template <bool ABOVE>
 __device__ __forceinline__ double exp_d(double x, bool valid, const double* tab) {
   x = valid && !(x < -800.0) ? x : -800.0;  // 2^-1154 is 0; keeps r finite for -inf
-  const double n = __builtin_rint(x * (64.0 * 1.4426950408889634));
+  double n = __builtin_rint(x * (64.0 * 1.4426950408889634));
+  if constexpr (ABOVE) n = fmin(n, 0x1p20);  // NaN: r stays NaN
   double r = __builtin_fma(n, -0x1.62e42fefa39efp-7, x);
   r = __builtin_fma(n, -0x1.abc9e3b39803fp-62, r);
   const int k = (int)n;
@@ -174,7 +180,7 @@ struct OnlineLse {
     for (int q = 0; q < 8; ++q) mb = valid[q] && x[q >> 2][q & 3] > mb ? x[q >> 2][q & 3] : mb;
     double f = 1.0;
     if (mb > m) {
-      f = exp_d(m - mb, m != kNegInfD, tab);
+      f = exp_d<false>(m - mb, m != kNegInfD, tab);
       r *= f;
       m = mb;
     }
@@ -188,7 +194,7 @@ struct OnlineLse {
     (void)raise(x, valid, tab);
     if (m == kNegInfD) return;  // no finite score yet
 #pragma unroll
-    for (int q = 0; q < 8; ++q) r += exp_d(x[q >> 2][q & 3] - m, valid[q], tab);
+    for (int q = 0; q < 8; ++q) r += exp_d<false>(x[q >> 2][q & 3] - m, valid[q], tab);
   }
   // Merges the row's four lanes; returns the factor of this lane's terms.
   __device__ __forceinline__ double merge(const double* tab) {
@@ -197,7 +203,7 @@ struct OnlineLse {
     mm = o > mm ? o : mm;
     o = xor_lanes(mm, 32);
     mm = o > mm ? o : mm;
-    const double f = exp_d(m - mm, m != kNegInfD, tab);
+    const double f = exp_d<false>(m - mm, m != kNegInfD, tab);
     r *= f;
     r += xor_lanes(r, 16);
     r += xor_lanes(r, 32);
@@ -384,7 +390,7 @@ __global__ __launch_bounds__(kF32Threads, MAXD <= 128 ? 2 : 1) void f32_kernel(c
         if (on_t.m != kNegInfD) {
 #pragma unroll
           for (int q = 0; q < 8; ++q) {
-            const double p = exp_d(st[q >> 2][q & 3] - on_t.m, valid[q], tab);
+            const double p = exp_d<false>(st[q >> 2][q & 3] - on_t.m, valid[q], tab);
             on_t.r += p;
             kl += valid[q] ? p * (st[q >> 2][q & 3] - ss[q >> 2][q & 3]) : 0.0;
           }
@@ -394,7 +400,7 @@ __global__ __launch_bounds__(kF32Threads, MAXD <= 128 ? 2 : 1) void f32_kernel(c
         for (int q = 0; q < 8; ++q) {
           const double lps = ss[q >> 2][q & 3] - lse_s;
           const double lpt = st[q >> 2][q & 3] - lse_t;
-          const double term = exp_d(lpt, valid[q], tab) * (lpt - lps);
+          const double term = exp_d<true>(lpt, valid[q], tab) * (lpt - lps);
           kl += valid[q] ? term : 0.0;
         }
       } else {  // D, then grad^T[d][owned] += sum_r tile[r][d] D[r][owned]
@@ -402,8 +408,8 @@ __global__ __launch_bounds__(kF32Threads, MAXD <= 128 ? 2 : 1) void f32_kernel(c
         for (int q = 0; q < 8; ++q) {
           const int r = 16 * (q >> 2) + 4 * (q & 3) + g;
           const double ls = kDk ? sh.lse_s[r] : lse_s, lt = kDk ? sh.lse_t[r] : lse_t;
-          const double ps = exp_d(ss[q >> 2][q & 3] - ls, valid[q], tab);
-          const double pt = exp_d(st[q >> 2][q & 3] - lt, valid[q], tab);
+          const double ps = exp_d<true>(ss[q >> 2][q & 3] - ls, valid[q], tab);
+          const double pt = exp_d<true>(st[q >> 2][q & 3] - lt, valid[q], tab);
           // four exponentials in flight at a time (the empty asm also keeps the
           // vectoriser from joining all sixteen): the gradient modes would spill
           double d = ps - pt;

@@ -235,3 +235,22 @@ def test_a_nan_score_takes_its_rows_out(gpu_available, causal, pad, bad):
         want = (float(attn_kl_align(*(v[:, :, :seen].contiguous() for v in x), attn_mask=m[:, :seen].contiguous(),
                                     causal=causal)) if seen > pad else 0.0)
         assert float(attn_kl_align(*x, attn_mask=m, causal=causal)) == pytest.approx(want, rel=1e-6, abs=0)
+
+
+@pytest.mark.parametrize("value", [float("inf"), 1e30, 1e5])
+def test_a_score_far_above_its_lse_overflows_to_infinity(gpu_available, value):
+    """exp(S - lse) of a caller's LSE that does not cover S: inf, as in the
+    oracle's formula, not NaN, in the row KL and in D."""
+    from linearard_amd.attention_KL import kl_backward, kl_forward
+
+    B, H, T, D, key = 1, 2, 40, 32, 9
+    rng = np.random.default_rng(5)
+    qs, ks, qt, kt = (to_dev(np.abs(rng.standard_normal((B, H, T, D))) + 0.1, "f32") for _ in range(4))
+    kt[:, :, key, 0] = value
+    lse = torch.zeros((B, H, T), device="cuda")
+    # the row KL exceeds float32 (and double, for inf): p_t (l_t - l_s) = inf
+    assert float(kl_forward(qs, ks, lse, qt, kt, lse, None, True, 1.0, 1.0)) == math.inf
+    dq, dk = kl_backward(qs, ks, lse, qt, kt, lse, None, True, 1.0, 1.0)
+    # D = p_s - p_t is -inf at this key for the rows that see it, finite elsewhere
+    assert bool((dq[:, :, key:] == -math.inf).all()) and bool(torch.isfinite(dq[:, :, :key]).all())
+    assert bool((dk[:, :, key] == -math.inf).all()) and bool(torch.isfinite(dk[:, :, key + 1:]).all())
