@@ -144,7 +144,9 @@ __global__ __launch_bounds__(kPrepThreads) void keys_f16_fixup_kernel(const KeyB
 KeySide key_side(const SideArgs& s, int B, int Hq, unsigned* maxima, float* scale, u16* k16) {
   KeySide k{};
   k.k = s.k;
-  k.q = s.q != s.k ? s.q : nullptr;
+  // q is k: the same heads, not only the same address (k = q[:, :hkv])
+  const bool same = s.q == s.k && Hq == s.hkv && s.q_sb == s.k_sb && s.q_sh == s.k_sh && s.q_st == s.k_st;
+  k.q = same ? nullptr : s.q;
   k.k_sb = s.k_sb, k.k_sh = s.k_sh, k.k_st = s.k_st;
   k.q_sb = s.q_sb, k.q_sh = s.q_sh, k.q_st = s.q_st;
   k.hkv = s.hkv, k.hq = Hq, k.k_heads = B * s.hkv;

@@ -443,6 +443,29 @@ def test_keys_beyond_the_float16_range_take_a_scale(gpu_available, self_rel):
         check_grad(tks.grad.float().cpu().numpy(), rdk, cid, "dk")
 
 
+@pytest.mark.parametrize("side", ["student", "teacher"])
+def test_large_queries_whose_keys_are_their_first_heads(gpu_available, side):
+    """bf16, ks = qs[:, :2]: the keys share the queries' address, and the only
+    value beyond the float16 range is in a query head past them; it still sets
+    the scale of the float16 operands.  Against the float64 oracle."""
+    from linearard_amd.attention_KL import attn_kl_align
+
+    rng = np.random.default_rng(31)
+    B, Hq, Hkv, T, D, a = 1, 4, 2, 130, 64, 2.0 ** -19
+    qs, qt = (O.round_to(rng.standard_normal((B, Hq, T, D)).astype(np.float32) * 256, "bf16") for _ in range(2))
+    (qs if side == "student" else qt)[0, 3, 60, 5] = 7.0e4
+    qs, qt = O.round_to(qs, "bf16"), O.round_to(qt, "bf16")
+    x, y = to_dev(qs, "bf16", requires_grad=True), to_dev(qt, "bf16")
+    ks, kt = x.detach()[:, :Hkv], y[:, :Hkv]
+    assert ks.data_ptr() == x.data_ptr() and ks.is_contiguous()
+    loss = attn_kl_align(x, ks, y, kt, causal=True, sm_scale_s=a, sm_scale_t=a)
+    dq, = torch.autograd.grad(loss, [x])
+    rl, rdq, _, _, _ = O.attn_kl_align(qs, qs[:, :Hkv], qt, qt[:, :Hkv], None, True, a, a)
+    case = f"f16-key-scale-views-{side}"
+    check_loss(loss.item(), rl, case)
+    check_grad(dq.float().cpu().numpy(), rdq, case, "dq")
+
+
 @pytest.mark.parametrize("case", ["self", "gqa", "batched"])
 def test_second_backward_through_the_same_graph(gpu_available, case):
     """retain_graph: the first backward adds the column side to the row side
