@@ -122,7 +122,9 @@ int lard_kl_backward(const lard_tensor4* qs, const lard_tensor4* ks, const float
  * cut into parts (query heads, ranges of query tiles) that run as workgroups
  * of their own and are added up in a fixed order.  workspace: 16-byte aligned,
  * lard_kl_backward_workspace_bytes(...) bytes (0 where nothing is cut; a
- * smaller or NULL workspace is accepted and runs uncut). */
+ * smaller or NULL workspace is accepted and runs uncut).  The parts take at most
+ * 512 * 128 * head_dim floats; from seq_len 4096 (8192) twice (four times) that,
+ * and then no more than dq_out. */
 size_t lard_kl_backward_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t seq_len,
                                         int64_t head_dim);
 int lard_kl_backward_ws(const lard_tensor4* qs, const lard_tensor4* ks, const float* lse_s,

@@ -371,27 +371,47 @@ struct BwdWs {
   float* dk_part;  // null unless the dk sums are cut (dk_cut)
 };
 
-// How a grouped-query dk sum is cut (RelArgs::dk_part): `split` ranges of
-// query tiles times the group's heads, 0 for one workgroup per key block.
-// rows: key rows per workgroup.  One workgroup per key block sums its whole
-// group (4 heads of 24 tiles on 48 of 256 CUs: 149 us of a 239 us fwd+bwd at
-// B=2, Hq=16, Hkv=4, n=1531, d=64), so a grid below one workgroup per CU is
-// cut by heads, and by query tiles (of 64, at least 4 each) until there are
-// two per CU.  Larger grids keep the sum in registers: the parts cost a write
-// and a read of group * split float32 copies of dk (at most 256 * 8 key blocks
-// of them, 256 MB at d = 128).
-int dk_cut(int64_t B, int64_t Hq, int64_t Hkv, int64_t T, int64_t rows) {
-  if (Hkv <= 0 || Hq <= Hkv || T <= 0) return 0;
-  const int64_t wgs = (T + rows - 1) / rows * B * Hkv;
-  if (wgs >= 256) return 0;
-  int64_t split = 512 / (wgs * (Hq / Hkv));
-  const int64_t most = (T + 255) / 256;
-  if (split > most) split = most;
-  return (int)(split < 1 ? 1 : split > 8 ? 8 : split);
+// How a grouped-query dk sum is cut (RelArgs::dk_part): parts of `heads` heads
+// of the group, each over one of `split` ranges of query tiles; parts = 0: one
+// workgroup per key block.  rows: key rows per workgroup.
+struct DkCut {
+  int heads, split, parts;
+};
+
+// One workgroup per key block sums its whole group (4 heads of 24 tiles on 48
+// of 256 CUs: 149 us of a 239 us fwd+bwd at B=2, Hq=16, Hkv=4, n=1531, d=64),
+// so a grid below one workgroup per CU is cut: by heads, up to 512 workgroups,
+// and, each head apart, by query tiles (of 64, at least 4 each).
+// The parts cost a write and a read of a float32 copy of dk each, which short
+// sequences feel (252 key blocks of 255 tokens, group 4: 188 us of column side
+// in 4 parts, 139 in 2, 164 uncut) and long causal ones do not: theirs take up
+// to 1024 (2048 from T = 8192), whose longest block ends earlier (stage dq + dk of
+// 64 heads on 1, T 4096: 1167 us with 512, 949 with 1024; of 14 on 2, T 8192,
+// D 64: 860 and 677).
+// So the parts take at most 512 / 1024 / 2048 * rows * dim floats (64 / 128 /
+// 256 MB for the 128-wide throughput kernels, whose rows are 256, and the
+// 256-wide stage kernels, 128) and, cut by heads alone, no more than dq's.
+DkCut dk_cut(int64_t B, int64_t Hq, int64_t Hkv, int64_t T, int64_t rows) {
+  if (Hkv <= 0 || Hq <= Hkv || T <= 0) return {0, 0, 0};
+  const int64_t wgs = (T + rows - 1) / rows * B * Hkv, group = Hq / Hkv;
+  if (wgs >= 256) return {0, 0, 0};
+  const int64_t most = (T >= 8192 ? 2048 : T >= 4096 ? 1024 : 512) / wgs;  // parts by heads, at least 2
+  const int64_t heads = most < group ? (group + most - 1) / most : 1;
+  const int64_t split = std::max<int64_t>(1, std::min<int64_t>({512 / (wgs * group), (T + 255) / 256, 8}));
+  return {(int)heads, (int)split, (int)((group + heads - 1) / heads * split)};
 }
 
 int64_t dk_part_floats(int64_t B, int64_t Hq, int64_t Hkv, int64_t T, int64_t D, int64_t rows) {
-  return (int64_t)dk_cut(B, Hq, Hkv, T, rows) * B * Hq * T * D;
+  return (int64_t)dk_cut(B, Hq, Hkv, T, rows).parts * B * Hkv * T * D;
+}
+
+// The parts of a call: in `part` (null: not cut).
+void set_dk_cut(lard::RelArgs& a, float* part, int64_t rows) {
+  if (part == nullptr) return;
+  const DkCut c = dk_cut(a.B, a.Hq, a.s.hkv, a.T, rows);
+  a.dk_part = part;
+  a.dk_heads = c.heads;
+  a.dk_split = c.split;
 }
 
 BwdWs bwd_layout(void* base, int64_t B, int64_t Hq, int64_t T, size_t* bytes, int64_t part_floats = 0) {
@@ -414,8 +434,7 @@ void cut_stage_dk(lard::RelArgs& a, void* workspace, size_t workspace_bytes) {
   if (floats == 0 || workspace == nullptr || workspace_bytes < (size_t)floats * 4 ||
       reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
     return;
-  a.dk_part = static_cast<float*>(workspace);
-  a.dk_split = dk_cut(a.B, a.Hq, a.s.hkv, a.T, lard::kStageRows);
+  set_dk_cut(a, static_cast<float*>(workspace), lard::kStageRows);
 }
 
 // Opt-in launch timing (lard_timing_*): event pairs recorded around the
@@ -1065,8 +1084,7 @@ int attn_kl_backward_impl(const lard_tensor4* qs, const lard_tensor4* ks, const 
     f.r.dk_out = dk_out;
     f.r.dk_add = self_relation ? dk_out : nullptr;
     f.r.dscale = dloss;
-    f.r.dk_part = w.dk_part;
-    f.r.dk_split = dk_cut(B, Hq, ks->size[1], T, lard::kRows);
+    set_dk_cut(f.r, w.dk_part, lard::kRows);
     if ((rc = hip_status(timed(LARD_KERNEL_COL_GRAD, st, [&] { return lard::launch_hot_bwd(f, padded_dim(ds), bf, st); }),
                          "attn_kl_backward dk launch")) != LARD_OK)
       return rc;
@@ -1234,11 +1252,10 @@ int backward_colgrad_impl(const lard_tensor4* qs, const lard_tensor4* ks, const 
   const int Tp = (int)padded_len(T);
   const BwdWs w = bwd_layout(workspace, B, Hq, T, nullptr, dk_part_floats(B, Hq, ks->size[1], T, ds, lard::kRows));
   lard::HotArgs f{};
-  f.r.dk_part = w.dk_part;
-  f.r.dk_split = dk_cut(B, Hq, ks->size[1], T, lard::kRows);
   fill_side(f.r.s, qs, ks, Hq, sm_scale_s);
   fill_side(f.r.t, qt, kt, Hq, sm_scale_t);
   fill_common(f.r, B, Hq, T, mask, causal);
+  set_dk_cut(f.r, w.dk_part, lard::kRows);
   f.r.lse_s_in = lse_s;
   f.r.lse_t_in = lse_t;
   lard::RowPrepBatch rp = lard::row_prep_batch(f.r, Tp);

@@ -786,6 +786,7 @@ __device__ __forceinline__ void hot_bwd_body(const HotArgs& f, int item) {
   const int bg = bgp / parts;
   const int part = bgp - bg * parts;
   const int part_h = part / split, part_s = part - part_h * split;
+  const int heads = a.dk_part != nullptr ? a.dk_heads : a.s.group;
   const int b = bg / a.s.hkv;
   const int g = bg - b * a.s.hkv;
   const int j0w = cb * kRows + w * 32;
@@ -831,8 +832,8 @@ __device__ __forceinline__ void hot_bwd_body(const HotArgs& f, int item) {
   tro.init(lane);
   int loaded_ht = -1;
 
-  const int hh_end = a.dk_part != nullptr ? part_h + 1 : a.s.group;
-  for (int hh = part_h; hh < hh_end; ++hh) {
+  const int hh_end = min((part_h + 1) * heads, a.s.group);
+  for (int hh = part_h * heads; hh < hh_end; ++hh) {
     const int h = g * a.s.group + hh;
     const int ht = h / a.t.group;
     if (ht != loaded_ht) {

@@ -72,11 +72,13 @@ struct RelArgs {
   const float* dk_add;  // [B, Hkv_s, T, Ds] or null (self relation: the row-side term dq)
   const float* dscale;  // device scalar or null (autograd's dloss)
   // dk kernels, grouped queries on a grid too small for the chip: each key
-  // block's sum over its group's heads and dk_split ranges of query tiles is
-  // cut into group * dk_split parts, one workgroup each, written (scaled by
-  // scale_s only) to dk_part [B * Hkv_s][group * dk_split][T, Ds]; the finish
-  // kernel adds them up (null: one workgroup sums everything into dk_out).
+  // block's sum over its group's heads and query tiles is cut into parts, one
+  // workgroup each, of dk_heads heads (the last of a group fewer) over one of
+  // dk_split ranges of query tiles.  A part goes, scaled by scale_s only, to
+  // dk_part [B * Hkv_s][dk_parts][T, Ds]; the finish kernel adds them up (null:
+  // one workgroup sums everything into dk_out).
   float* dk_part;
+  int dk_heads;
   int dk_split;
   // Throughput kernels: dk rounded to the input type here instead of dk_out
   // (null: float32 to dk_out).

@@ -74,6 +74,38 @@ def test_abi_rejects_bad_arguments_without_a_gpu():
     assert L.lard_attn_kl_backward_workspace_bytes(0, H, H, T, D, 0) == 0
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_the_scratch_of_cut_dk_sums_is_bounded(D):
+    """The parts of the dk sums fit 512 workgroups' rows (1024 from T = 4096,
+    2048 from T = 8192), and beyond 512 workgroups no more than dq itself,
+    however large the group; full grids take none."""
+    L = _lib.lib()
+    cut = 0
+    for B in (1, 2, 7, 31, 63):
+        for Hkv in (1, 2, 3, 8):
+            for group in (2, 3, 4, 7, 8, 32, 128):
+                for T in (1, 255, 256, 257, 1000, 4095, 4096, 8191, 8192, 32512, 32513, 65024):
+                    Hq = Hkv * group
+                    least = L.lard_attn_kl_backward_workspace_bytes(B, Hq, Hq, T, D, 0)
+                    full = L.lard_attn_kl_backward_workspace_bytes(B, Hq, Hkv, T, D, 0)
+                    stage = L.lard_kl_backward_workspace_bytes(B, Hq, Hkv, T, D)
+                    for rows, parts in ((128, stage), (256, full - least)):
+                        wgs = (T + rows - 1) // rows * B * Hkv
+                        most = 2048 if T >= 8192 else 1024 if T >= 4096 else 512
+                        cap = most * rows * D * 4 if wgs < 256 else 0
+                        if cap > 512 * rows * D * 4:
+                            cap = min(cap, max(512 * rows * D * 4, B * Hq * T * D * 4))
+                        if rows == 256:  # the call's size also covers the stage kernels' parts
+                            cap = max(cap, stage)
+                        assert parts <= cap, (B, Hq, Hkv, T, rows, parts, cap)
+                        cut += parts > 0
+    assert cut > 100
+    # 127 key blocks, 32 heads on one: 532 MB when each head was a part
+    assert L.lard_kl_backward_workspace_bytes(1, 32, 1, 32512, 128) <= 256 << 20
+    assert L.lard_attn_kl_backward_workspace_bytes(1, 128, 1, 65024, 128, 0) <= (256 << 20) + L.lard_attn_kl_backward_workspace_bytes(
+        1, 128, 128, 65024, 128, 0)
+
+
 def test_noalloc_forward_rejects_sizes_beyond_its_scratch_without_a_gpu():
     """The library's own workspace holds LARD_NOALLOC_SCRATCH_BYTES (16 MiB) per
     GPU: a forward needing more is refused before anything is launched."""

@@ -1,7 +1,7 @@
 """dk sums cut into parts (grouped queries on a grid below one workgroup per
 CU): the autograd pair, the general backward and the stage entry point against
-the float64 oracle, around the sizes where the cut changes, and the stage entry
-point without a workspace (uncut) against the cut one."""
+the float64 oracle, at ragged sizes and around every limit of the cut, and the
+stage entry point without a workspace (uncut) against the cut one."""
 
 import ctypes
 import math
@@ -62,6 +62,43 @@ def test_cut_dk_matches_the_oracle(gpu_available, dtype, B, hq, hkv, T, D, causa
     assert rc == 0, L.lard_last_error()
     assert torch.equal(dq, dq0)
     assert float((dk - dk0).abs().max()) <= 1e-5 * float(dk0.abs().max())
+
+
+# around each limit of the cut; parts: of one key block's sum
+@pytest.mark.parametrize("B,hq,hkv,T,D,causal,parts,stage_parts", [
+    (1, 2, 1, 2100, 16, True, 16, 16),   # 9 / 17 blocks of one group of 2: ranges of tiles, at their cap of 8
+    (32, 8, 2, 250, 32, True, 4, 4),     # 64 / 128 blocks of a group of 4: one range (T < 256; 512 workgroups)
+    (33, 8, 2, 250, 32, False, 4, 2),    # 66 / 132 blocks: the stage kernels take two heads a part
+    (66, 8, 2, 60, 32, True, 2, 2),      # 132 blocks: two heads a part in both
+    (33, 16, 2, 63, 64, True, 4, 4),     # 66 blocks of a group of 8
+    (85, 9, 3, 30, 16, False, 2, 2),     # 255 blocks of a group of 3: parts of two heads and of one
+    (64, 8, 4, 40, 16, True, 0, 0),      # 256 blocks: not cut
+    (85, 6, 3, 129, 16, True, 2, 0),     # 255 / 510
+])
+def test_cut_dk_at_its_limits(gpu_available, B, hq, hkv, T, D, causal, parts, stage_parts):
+    from linearard_amd.attention_KL import attn_kl_align, kl_backward, lse_stats
+
+    qs, ks, qt, kt, mask = _problem(B + T, "f16", B, hq, hkv, T, D, 0.2)
+    L = _lib.lib()
+    part = B * hkv * T * D * 4
+    assert L.lard_kl_backward_workspace_bytes(B, hq, hkv, T, D) == stage_parts * part
+    base = L.lard_attn_kl_backward_workspace_bytes(B, hq, hq, T, D, 0)
+    full = L.lard_attn_kl_backward_workspace_bytes(B, hq, hkv, T, D, 0)
+    Tp = (T + 63) // 64 * 64
+    layout = sum((n + 255) // 256 * 256 for n in (B * Tp, 8 * B, 4 * B * hq * Tp, 4 * B * hq * Tp, parts * part))
+    assert full == max(base, layout, (stage_parts * part + 255) // 256 * 256)
+    a = 1 / math.sqrt(D)
+    d = [to_dev(x, "f16", requires_grad=i < 2) for i, x in enumerate((qs, ks, qt, kt))]
+    m = mask_to_dev(mask)
+    case = f"dklimits-{B}-{hq}-{hkv}-{T}-{D}-c{int(causal)}"
+    _, rq, rk, _, _ = O.attn_kl_align(qs, ks, qt, kt, mask, causal, a, a)
+    dq, dk = torch.autograd.grad(attn_kl_align(*d, attn_mask=m, causal=causal), d[:2])
+    check_grad(dq.float().cpu().numpy(), rq, case, "dq")
+    check_grad(dk.float().cpu().numpy(), rk, case, "dk")
+    x = [t.detach() for t in d]
+    ls, lt = lse_stats(x[0], x[1], m, causal, a), lse_stats(x[2], x[3], m, causal, a)
+    _, dk = kl_backward(x[0], x[1], ls, x[2], x[3], lt, m, causal, a, a)
+    check_grad(dk.cpu().numpy(), rk, case + "-stage", "dk")
 
 
 def _general_backward(L, x, lse, mask, causal, a, dloss, self_rel):
