@@ -59,6 +59,17 @@ inline int stage_types(const RelArgs& a, bool two_sided) {
   return a.s.bf16 ? kTypesBf16 : kTypesF16;
 }
 
+// Workgroups per CU (waves per SIMD) that an instance's registers are held to.
+// Two hide each other's waits, also where a few registers spill for it (the
+// general gradients of a 128-wide student with a teacher up to 128: one per CU
+// took up to 1.7 times as long); 256-wide students have no room for two, and
+// beside a 256-wide teacher the 128-wide general gradients spilled up to 161
+// registers in the tile loop (dq + dk at B=1, H=16, n=2048, causal: 414 us
+// with two, 245 with one).
+constexpr int stage_waves(int dps, int dpt, int types, bool grad) {
+  return grad && (dps > 128 || (dps == 128 && dpt > 128 && types == kTypesAny)) ? 1 : 2;
+}
+
 // This workgroup's block (of gridDim.x) and head (of gridDim.y), numbered so
 // that each XCD works on a contiguous range of heads: its L2 then holds the
 // head's tiles that all its workgroups walk.  (With heads dealt round robin
@@ -232,7 +243,7 @@ __device__ __forceinline__ void pin_agprs(f32x16* acc) {
 }
 
 template <int MODE, int DPS, int DPT, int DT = kTypesAny>
-__global__ __launch_bounds__(kStageThreads, DPS <= 128 || MODE != MODE_DQ ? 2 : 1) void row_kernel(const RelArgs a) {
+__global__ __launch_bounds__(kStageThreads, stage_waves(DPS, DPT, DT, MODE == MODE_DQ)) void row_kernel(const RelArgs a) {
   constexpr int BN = kStageTile;
   constexpr bool HAS_T = MODE != MODE_LSE;
   constexpr bool HAS_DQ = MODE == MODE_DQ;
@@ -466,7 +477,7 @@ __global__ __launch_bounds__(kStageThreads, DPS <= 128 || MODE != MODE_DQ ? 2 : 
 }
 
 template <int DPS, int DPT, int DT = kTypesAny>
-__global__ __launch_bounds__(kStageThreads, DPS <= 128 ? 2 : 1) void col_kernel(const RelArgs a) {
+__global__ __launch_bounds__(kStageThreads, stage_waves(DPS, DPT, DT, true)) void col_kernel(const RelArgs a) {
   constexpr int BM = kStageTile;
   constexpr int kBufs = stage_bufs(DPS, DPT, true);
   constexpr int KS = DPS / 16;

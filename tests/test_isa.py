@@ -8,6 +8,8 @@
   asm; on every control-flow path of every instantiation, MFMA results are
   left alone for the gfx950 wait states and no VALU write of an MFMA operand
   comes within 2 wait states before it (tests/isa_check.py).
+* The general gradient kernels of a 128-wide student and a 256-wide teacher
+  use no scratch memory.
 * The checker itself catches planted violations.
 """
 
@@ -67,6 +69,16 @@ def test_the_other_sources_leave_m0_alone(asm_dir):
     for src in ("abi.hip", "logits_kl.hip", "reduce.hip", "rope.hip", "stage_f32.hip"):
         for name, body in _kernels(src, asm_dir).items():
             assert not C.check_m0(name, body) and not any("load_lds" in t for _, t in body), (src, name)
+
+
+@needs_hipcc
+@pytest.mark.parametrize("src,kernel", [("stage_dq.hip", "10row_kernelILi2ELi128ELi256ELi2E"),
+                                        ("stage_dk.hip", "10col_kernelILi128ELi256ELi2E")])
+def test_wide_teacher_gradients_keep_their_registers(asm_dir, src, kernel):
+    """128-wide student, 256-wide teacher: spilled in the tile loop, these
+    instances took 1.7 times as long."""
+    body, = [b for n, b in _kernels(src, asm_dir).items() if kernel in n]
+    assert not [t for k, t in body if k == "inst" and t.startswith("scratch_")]
 
 
 @needs_hipcc
