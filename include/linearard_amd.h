@@ -196,7 +196,8 @@ int lard_attn_kl_forward_noalloc(const lard_tensor4* qs, const lard_tensor4* ks,
 /* Workspace needed by lard_attn_kl_backward (bytes): one validity byte per
  * token and two log2-domain row normalisers per query row, and with kv_heads
  * < heads on a small grid the parts of the dk sums (as
- * lard_kl_backward_ws).  self_relation does not change the size; it is kept so
+ * lard_kl_backward_ws).  The size for kv_heads == heads is enough too: the dk
+ * sums then run uncut.  self_relation does not change the size; it is kept so
  * the call describes the whole problem. */
 size_t lard_attn_kl_backward_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t seq_len,
                                              int64_t head_dim, int self_relation);

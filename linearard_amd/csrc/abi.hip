@@ -427,6 +427,25 @@ BwdWs bwd_layout(void* base, int64_t B, int64_t Hq, int64_t T, size_t* bytes, in
   return w;
 }
 
+// The least a backward runs with (the size for kv_heads == heads): without the
+// parts of cut dk sums, which it then sums uncut.  float32 inputs: both sides'
+// LSEs in double (the refine pass).
+size_t bwd_least_bytes(int64_t B, int64_t Hq, int64_t T) {
+  size_t bytes = 0;
+  bwd_layout(nullptr, B, Hq, T, &bytes);
+  return std::max(bytes, align256((size_t)(2 * B * Hq * T) * sizeof(double)));
+}
+
+// The throughput backward's regions in a workspace of at least bwd_least_bytes,
+// with the parts if they fit (16-byte aligned).
+BwdWs bwd_regions(void* workspace, size_t workspace_bytes, int64_t B, int64_t Hq, int64_t Hkv, int64_t T, int64_t D) {
+  int64_t floats = dk_part_floats(B, Hq, Hkv, T, D, lard::kRows);
+  size_t bytes = 0;
+  bwd_layout(nullptr, B, Hq, T, &bytes, floats);
+  if (bytes > workspace_bytes || reinterpret_cast<uintptr_t>(workspace) % 16 != 0) floats = 0;
+  return bwd_layout(workspace, B, Hq, T, nullptr, floats);
+}
+
 // The stage kernels' dk sums in parts, when they are cut and `workspace` (16-byte
 // aligned) holds them.
 void cut_stage_dk(lard::RelArgs& a, void* workspace, size_t workspace_bytes) {
@@ -1014,9 +1033,7 @@ size_t lard_attn_kl_backward_workspace_bytes(int64_t batch, int64_t heads, int64
   bwd_layout(nullptr, batch, heads, seq_len, &bytes,
              dk_part_floats(batch, heads, kv_heads, seq_len, head_dim, lard::kRows));
   const size_t stage = align256((size_t)dk_part_floats(batch, heads, kv_heads, seq_len, head_dim, lard::kStageRows) * 4);
-  // float32 inputs: both sides' LSEs in double (the refine pass)
-  const size_t f64 = align256((size_t)(2 * batch * heads * seq_len) * sizeof(double));
-  return std::max(bytes, std::max(stage, f64));
+  return std::max({bytes, stage, bwd_least_bytes(batch, heads, seq_len)});
 }
 
 }  // extern "C"
@@ -1054,13 +1071,12 @@ int attn_kl_backward_impl(const lard_tensor4* qs, const lard_tensor4* ks, const 
   const int ds = (int)qs->size[3], dt = (int)qt->size[3];
   std::string why;
   if (attn_kl_path(qs, ks, qt, kt, sm_scale_s, sm_scale_t, &why) == LARD_PATH_THROUGHPUT) {
-    const size_t need = lard_attn_kl_backward_workspace_bytes(B, Hq, ks->size[1], T, ds, self_relation);
+    const size_t need = bwd_least_bytes(B, Hq, T);
     if (workspace == nullptr || workspace_bytes < need)
       return fail(LARD_ERR_INVALID_ARGUMENT, "workspace too small: need %zu bytes", need);
     if ((rc = check_blocks(B, Hq, T)) != LARD_OK) return rc;
     const int Tp = (int)padded_len(T);
-    const int64_t parts = dk_part_floats(B, Hq, ks->size[1], T, ds, lard::kRows);
-    const BwdWs w = bwd_layout(workspace, B, Hq, T, nullptr, parts);
+    const BwdWs w = bwd_regions(workspace, workspace_bytes, B, Hq, ks->size[1], T, ds);
     if ((rc = hip_status(lard::launch_token_prep(lard::token_prep(a, Tp, w.tok_ok, w.first2, nullptr), (int)B, st),
                          "attn_kl_backward token prep launch")) != LARD_OK)
       return rc;
@@ -1096,7 +1112,7 @@ int attn_kl_backward_impl(const lard_tensor4* qs, const lard_tensor4* ks, const 
   } else if (qs->dtype == LARD_DTYPE_F32) {
     // float32: refine both LSEs in double first (the stored ones are float32
     // roundings, too coarse for D = P_s - P_t of a near-identical pair)
-    const size_t need = lard_attn_kl_backward_workspace_bytes(B, Hq, ks->size[1], T, ds, self_relation);
+    const size_t need = bwd_least_bytes(B, Hq, T);
     if (workspace == nullptr || workspace_bytes < need)
       return fail(LARD_ERR_INVALID_ARGUMENT, "workspace too small: need %zu bytes", need);
     if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
@@ -1244,13 +1260,13 @@ int backward_colgrad_impl(const lard_tensor4* qs, const lard_tensor4* ks, const 
     return fail(LARD_ERR_UNSUPPORTED, "the column-gradient backward runs on the throughput kernels only (%s)",
                 why.c_str());
   const int ds = (int)qs->size[3];
-  const size_t need = lard_attn_kl_backward_workspace_bytes(B, Hq, ks->size[1], T, ds, self_relation);
+  const size_t need = bwd_least_bytes(B, Hq, T);
   if (workspace == nullptr || workspace_bytes < need)
     return fail(LARD_ERR_INVALID_ARGUMENT, "workspace too small: need %zu bytes", need);
   if ((rc = check_blocks(B, Hq, T)) != LARD_OK) return rc;
   const hipStream_t st = static_cast<hipStream_t>(stream);
   const int Tp = (int)padded_len(T);
-  const BwdWs w = bwd_layout(workspace, B, Hq, T, nullptr, dk_part_floats(B, Hq, ks->size[1], T, ds, lard::kRows));
+  const BwdWs w = bwd_regions(workspace, workspace_bytes, B, Hq, ks->size[1], T, ds);
   lard::HotArgs f{};
   fill_side(f.r.s, qs, ks, Hq, sm_scale_s);
   fill_side(f.r.t, qt, kt, Hq, sm_scale_t);

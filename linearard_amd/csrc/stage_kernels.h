@@ -61,8 +61,8 @@ inline int stage_types(const RelArgs& a, bool two_sided) {
 
 // Workgroups per CU (waves per SIMD) that an instance's registers are held to.
 // Two hide each other's waits, also where a few registers spill for it (the
-// general gradients of a 128-wide student with a teacher up to 128: one per CU
-// took up to 1.7 times as long); 256-wide students have no room for two, and
+// general gradients of a 128-wide student: with a teacher up to 64 one per CU
+// took 1.04 to 1.7 times as long, with a 128-wide one 0.8 to 1.3); 256-wide students have no room for two, and
 // beside a 256-wide teacher the 128-wide general gradients spilled up to 161
 // registers in the tile loop (dq + dk at B=1, H=16, n=2048, causal: 414 us
 // with two, 245 with one).

@@ -118,6 +118,47 @@ def _general_backward(L, x, lse, mask, causal, a, dloss, self_rel):
     return dq, dk
 
 
+def test_backwards_accept_a_workspace_without_the_parts(gpu_available):
+    """A workspace of the size for kv_heads == heads: the dk sums run uncut, equal
+    to the cut ones up to the order of their float32 terms."""
+    B, hq, hkv, T, D, causal = 1, 4, 2, 500, 64, True
+    qs, ks, qt, kt, _ = _problem(11, "bf16", B, hq, hkv, T, D, None)
+    a = 1 / math.sqrt(D)
+    x = [to_dev(v, "bf16") for v in (qs, ks, qt, kt)]
+    L = _lib.lib()
+    p = [ctypes.byref(_lib.tensor4(t)) for t in x]
+    md, st = ctypes.byref(_lib.mask_desc(None)), _lib.stream_of(x[0])
+    lse = [torch.empty((B, hq, T), device="cuda") for _ in range(2)]
+    out, dloss = torch.empty((), device="cuda"), torch.ones((), device="cuda")
+    row = torch.empty((B, hq, T, D), device="cuda")
+    ws = torch.empty((L.lard_attn_kl_forward_rowgrad_workspace_bytes(B, hq, hkv, hkv, T, D),), device="cuda",
+                     dtype=torch.uint8)
+    assert L.lard_attn_kl_forward_rowgrad(*p, md, int(causal), a, a, lse[0].data_ptr(), lse[1].data_ptr(),
+                                          out.data_ptr(), row.data_ptr(), ws.data_ptr(), ws.numel(), st) == 0
+    full = L.lard_attn_kl_backward_workspace_bytes(B, hq, hkv, T, D, 0)
+    least = L.lard_attn_kl_backward_workspace_bytes(B, hq, hq, T, D, 0)
+    assert least < full
+    got = {}
+    for size in (full, least):
+        ws = torch.empty((size,), device="cuda", dtype=torch.uint8)
+        head = (p[0], p[1], lse[0].data_ptr(), p[2], p[3], lse[1].data_ptr(), md, int(causal), a, a, dloss.data_ptr(), 0)
+        tail = (ws.data_ptr(), size, st)
+        q, k = torch.empty_like(row), torch.empty((B, hkv, T, D), device="cuda")
+        q16, k16 = torch.empty_like(x[0]), torch.empty_like(x[1])
+        r = row.clone()
+        k2 = torch.empty_like(k)
+        assert L.lard_attn_kl_backward(*head, q.data_ptr(), k.data_ptr(), *tail) == 0, L.lard_last_error()
+        assert L.lard_attn_kl_backward_colgrad16(*head, row.data_ptr(), q16.data_ptr(), k16.data_ptr(),
+                                                 *tail) == 0, L.lard_last_error()
+        assert L.lard_attn_kl_backward_colgrad(*head, r.data_ptr(), k2.data_ptr(), *tail) == 0, L.lard_last_error()
+        got[size] = q, k, k2, k16.float()
+        assert L.lard_attn_kl_backward(*head, q.data_ptr(), k.data_ptr(), ws.data_ptr(), least - 1, st) == -1
+    cut, uncut = got.values()
+    assert torch.equal(cut[0], uncut[0])
+    for c, u, bound in zip(cut[1:], uncut[1:], (1e-5, 1e-5, 2.0 ** -8)):  # float32 sums; one bfloat16 rounding
+        assert float((c - u).abs().max()) <= bound * float(u.abs().max())
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("self_rel,hkv,T,D", [(True, 4, 333, 128), (True, 4, 65, 8), (False, 2, 900, 64), (False, 4, 130, 32)])
 def test_gradients_in_the_input_dtype(gpu_available, dtype, self_rel, hkv, T, D):
