@@ -8,6 +8,7 @@
   asm; on every control-flow path of every instantiation, MFMA results are
   left alone for the gfx950 wait states and no VALU write of an MFMA operand
   comes within 2 wait states before it (tests/isa_check.py).
+* The loss sum's ticket is a release and an acquire.
 * The general gradient kernels of a 128-wide student and a 256-wide teacher
   use no scratch memory.
 * The checker itself catches planted violations.
@@ -69,6 +70,22 @@ def test_the_other_sources_leave_m0_alone(asm_dir):
     for src in ("abi.hip", "logits_kl.hip", "reduce.hip", "rope.hip", "stage_f32.hip"):
         for name, body in _kernels(src, asm_dir).items():
             assert not C.check_m0(name, body) and not any("load_lds" in t for _, t in body), (src, name)
+
+
+@needs_hipcc
+def test_loss_sum_ticket_orders_the_partials(asm_dir):
+    """The ticket of the loss sum releases the workgroup's partial and acquires
+    the others' at agent scope: the L2's lines written back, with a wait,
+    before the atomic, and stale ones dropped after it."""
+    body, = [b for n, b in _kernels("reduce.hip", asm_dir).items() if "reduce_sum_kernel" in n]
+    ops = [t for k, t in body if k == "inst"]
+    at, = [i for i, t in enumerate(ops) if t.startswith("global_atomic_add")]
+    back = max(i for i, t in enumerate(ops[:at]) if t.startswith("buffer_wbl2 sc1"))
+    stores = [i for i, t in enumerate(ops[:at]) if t.startswith("global_store_dwordx2")]
+    assert stores and stores[-1] < back
+    assert any(t.startswith("s_waitcnt") and "vmcnt(0)" in t for t in ops[back:at])
+    load = min(i for i, t in enumerate(ops) if i > at and t.startswith("global_load_dwordx2"))
+    assert sum(t.startswith("buffer_inv sc1") for t in ops[at:load]) >= 2  # the ticket's wave, and every wave
 
 
 @needs_hipcc
