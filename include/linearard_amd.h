@@ -9,7 +9,8 @@
  * Conventions
  *   - Every tensor argument is a device pointer the caller owns.  The
  *     library never allocates or frees device memory; scratch space is
- *     passed in by the caller, sized by the matching *_workspace_bytes().
+ *     passed in by the caller, sized by the matching *_workspace_bytes() and
+ *     16-byte aligned (lard_kl_forward: 8).
  *   - q/k tensors are [B, H, T, D] with element strides; stride[3] must be 1,
  *     the data pointer 16-byte aligned and strides[0..2] multiples of 8
  *     elements (4 for float32; every contiguous tensor with D in

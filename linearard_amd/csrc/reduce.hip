@@ -9,6 +9,8 @@
 namespace lard {
 
 constexpr int kReduceThreads = 256;
+// x is the start of the caller's workspace: any 4-byte alignment
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ __forceinline__ double block_sum(double s, double* part) {
   __syncthreads();  // part may hold an earlier sum
@@ -37,8 +39,8 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_sum_kernel(const float*
   double s = 0.0;
   int64_t i = lo + 4 * threadIdx.x;
 #pragma unroll 4
-  for (; i + 4 <= hi; i += 4 * kReduceThreads) {  // x is 256-byte aligned and lo a multiple of 1024
-    const f32x4 v = *reinterpret_cast<const f32x4*>(x + i);
+  for (; i + 4 <= hi; i += 4 * kReduceThreads) {
+    const f32x4_any v = *reinterpret_cast<const f32x4_any*>(x + i);
     s += ((double)v[0] + (double)v[1]) + ((double)v[2] + (double)v[3]);
   }
   for (; i < hi; ++i) s += (double)x[i];  // the slice's last 1-3 values, one thread

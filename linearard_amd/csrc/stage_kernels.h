@@ -672,7 +672,7 @@ hipError_t launch_row_dq(const RelArgs& a, int dps, int dpt, hipStream_t stream)
 hipError_t launch_col_dk(const RelArgs& a, int dps, int dpt, hipStream_t stream);
 // Loss reduction: out = sum(x[0..n)) through at most kReduceBlocks double
 // partials; *counter must be 0 when the launch starts (the forward kernels
-// clear it: RelArgs::counter), x 16-byte aligned.
+// clear it: RelArgs::counter).
 constexpr int kReduceBlocks = 64;
 hipError_t launch_reduce_sum(const float* x, int64_t n, double* partial, unsigned* counter, float* out,
                              hipStream_t stream);

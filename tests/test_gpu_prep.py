@@ -45,6 +45,25 @@ def test_loss_is_the_sum_of_the_rows_at_slice_edges(gpu_available, n):
         assert abs(loss.double() - rows.sum()) <= 2.0 ** -24 * abs(rows.sum()) + 1e-12 * rows.abs().sum()
 
 
+@pytest.mark.parametrize("n", [3, 1025, 5000])
+def test_loss_sum_in_a_workspace_at_8_bytes(gpu_available, n):
+    """lard_kl_forward takes a workspace that a caller cut out of another at any
+    multiple of 8 bytes: the same loss."""
+    L = _lib.lib()
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, y = (torch.randn((1, 2, n, 8), device="cuda", generator=g).to(torch.float16) for _ in range(2))
+    lse = torch.randn((1, 2, n), device="cuda", generator=g)
+    size = L.lard_kl_forward_workspace_bytes(1, 2, n)
+    ws = torch.empty((size + 16,), device="cuda", dtype=torch.uint8)
+    d = [ctypes.byref(_lib.tensor4(t)) for t in (x, x, y, y)]
+    loss = torch.empty((2,), device="cuda")
+    for i, shift in enumerate((0, 8)):
+        rc = L.lard_kl_forward(d[0], d[1], lse.data_ptr(), d[2], d[3], lse.data_ptr(), ctypes.byref(_lib.mask_desc(None)),
+                               1, 0.3, 0.3, loss[i:].data_ptr(), ws.data_ptr() + shift, size, _lib.stream_of(x))
+        assert rc == 0, L.lard_last_error()
+    assert torch.equal(loss[0], loss[1])
+
+
 @pytest.mark.parametrize("D,T", [(8, 1023), (8, 1025), (64, 127), (64, 129), (128, 63), (128, 64), (128, 65)])
 @pytest.mark.parametrize("masked", [False, True])
 def test_nine_relations_equal_single_calls(gpu_available, D, T, masked):
