@@ -85,8 +85,10 @@ __device__ __forceinline__ void stage_item(int& blk, int& head, int causal, int 
 
 // One side's tile copies: rows [row0, row0 + 32) x [0, DP) of one head into a
 // swizzled tile.  Addresses are 64-bit per lane: these kernels also serve
-// heads of 2^31 bytes and more.  Rows >= T copy row T - 1 and chunks >= dim
-// chunk 0 (their contributions are masked, or meet zero operands).
+// heads of 2^31 bytes and more.  Rows >= T copy row T - 1 (their contributions
+// are masked).  Chunks >= dim (the second one of D = 8; the other dims fill
+// their tiles) are not copied: clear_padding sets them to zero once, so that
+// they add nothing also where a row holds infinities.
 template <int DP>
 struct StageCopier {
   using TC = TileCopies<DP, kStageWaves, kStageTile>;
@@ -98,6 +100,7 @@ struct StageCopier {
   int64_t lane_row;    // this lane's row of the wave's first copy, elements
   int r0;
   unsigned c[NITER];   // this lane's chunk of each copy, bytes
+  bool padding;        // DP = 16: this lane's chunk is one
 
   __device__ __forceinline__ void init(const u16* head, int64_t row_stride, int dim, int wave, int lane) {
     src = head;
@@ -107,7 +110,15 @@ struct StageCopier {
 #pragma unroll
     for (int i = 0; i < NITER; ++i) {
       const int ch = ((64 * wave + lane) % CPR) ^ swz<DP>(r0 + i * RPI);
-      c[i] = ch * 8 < dim ? 16u * ch : 0u;
+      c[i] = 16u * ch;
+      padding = DP == 16 && ch * 8 >= dim;  // one copy per tile there
+    }
+  }
+  // tiles: `bufs` tiles; a barrier must follow before they are read.
+  __device__ __forceinline__ static void clear_padding(u16* tiles, int bufs, int dim) {
+    if constexpr (DP == 16) {
+      for (int i = (int)threadIdx.x; i < bufs * kStageTile * CPR; i += kStageThreads)
+        if (((i % CPR) ^ swz<DP>(i / CPR)) * 8 >= dim) *reinterpret_cast<u16x8*>(tiles + 8 * i) = (u16x8)(0);
     }
   }
   __device__ __forceinline__ void issue(unsigned tile, int row0, int T, int wave) const {
@@ -121,7 +132,11 @@ struct StageCopier {
         const int over = row0 + i * RPI + r0 - (T - 1);
         if (over > 0) p -= (int64_t)over * stride;
       }
-      lds_async16_at(reinterpret_cast<const char*>(p) + c[i], tile + 1024u * n);
+      if constexpr (DP == 16) {
+        if (!padding) lds_async16_at(reinterpret_cast<const char*>(p) + c[i], tile + 1024u * n);
+      } else {
+        lds_async16_at(reinterpret_cast<const char*>(p) + c[i], tile + 1024u * n);
+      }
     }
   }
 };
@@ -336,7 +351,11 @@ __global__ __launch_bounds__(kStageThreads, stage_waves(DPS, DPT, DT, MODE == MO
   StageCopier<DPS> cps;
   StageCopier<HAS_T ? DPT : 16> cpt;
   cps.init(ks_base, a.s.k_st, a.s.dim, w, lane);
-  if constexpr (HAS_T) cpt.init(kt_base, a.t.k_st, a.t.dim, w, lane);
+  StageCopier<DPS>::clear_padding(lks[0], kBufs, a.s.dim);
+  if constexpr (HAS_T) {
+    cpt.init(kt_base, a.t.k_st, a.t.dim, w, lane);
+    StageCopier<DPT>::clear_padding(lkt[0], kBufs, a.t.dim);
+  }
   constexpr bool kUniform = StageCopier<DPS>::TC::kUniform && (!HAS_T || StageCopier<HAS_T ? DPT : 16>::TC::kUniform);
   constexpr int kPerWave =
       StageCopier<DPS>::TC::kRowPerWave + (HAS_T ? StageCopier<HAS_T ? DPT : 16>::TC::kRowPerWave : 0);
@@ -542,6 +561,9 @@ __global__ __launch_bounds__(kStageThreads, stage_waves(DPS, DPT, DT, true)) voi
   int loaded_ht = -1;
   const unsigned gs = row_chunk_xor<DPS>(l32, half), gt = row_chunk_xor<DPT>(l32, half);
   const TokenBits tok = {lbits, &a, (int64_t)b * a.mask_sb};
+
+  StageCopier<DPS>::clear_padding(lqs[0], kBufs, a.s.dim);
+  StageCopier<DPT>::clear_padding(lqt[0], kBufs, a.t.dim);
 
   const int hh_end = min((part_h + 1) * heads, a.s.group);
   for (int hh = part_h * heads; hh < hh_end; ++hh) {

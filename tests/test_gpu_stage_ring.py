@@ -54,14 +54,16 @@ def test_mixed_types(gpu_available, dts, dtt, ds, dt):
     _check(7, 1, 4, 2, 4, 130, ds, dt, dts, dtt, True, 0.2)
 
 
-def test_validity_bits_of_a_second_window(gpu_available):
+@pytest.mark.parametrize("D", [16, 64])
+def test_validity_bits_of_a_second_window(gpu_available, D):
     """One masked head of 32768 + 200 tokens, almost all of them masked: the
     stages on the whole sequence equal the stages on the kept tokens alone
     (masked tokens take no part), bitwise in dq and dk rows up to the order of
-    the sums: 1e-3 of the largest."""
+    the sums: 1e-3 of the largest.  D = 64 refills the bits with tiles in
+    flight, D = 16 with none."""
     from linearard_amd.attention_KL import kl_backward, kl_forward, lse_stats
 
-    T, D, n = 32768 + 200, 16, 300
+    T, n = 32768 + 200, 300
     g = torch.Generator(device="cuda").manual_seed(3)
     keep = torch.cat([torch.randperm(32768, generator=g, device="cuda")[: n - 60],
                       32768 + torch.randperm(200, generator=g, device="cuda")[:60]]).sort().values
@@ -84,3 +86,55 @@ def test_validity_bits_of_a_second_window(gpu_available):
         for i in (3, 4):
             assert float((a[i][:, :, keep] - b[i]).abs().max()) <= 1e-3 * float(b[i].abs().max())
             assert float(a[i][:, :, ~mask[0]].abs().max()) == 0.0
+
+
+def test_validity_bits_of_a_second_window_256_wide(gpu_available):
+    """The same for the 256-wide autograd pair (its forward refills the bits of
+    its own ring): loss and gradient of the kept tokens, to the bars."""
+    from linearard_amd.attention_KL import attn_kl_align
+
+    T, D, n = 32768 + 200, 256, 300
+    g = torch.Generator(device="cuda").manual_seed(4)
+    keep = torch.cat([torch.randperm(32768, generator=g, device="cuda")[: n - 60],
+                      32768 + torch.randperm(200, generator=g, device="cuda")[:60]]).sort().values
+    mask = torch.zeros((1, T), dtype=torch.bool, device="cuda")
+    mask[0, keep] = True
+    y = torch.randn((1, 1, T, D), generator=g, device="cuda").to(torch.float16)
+    x = (y.float() + 0.3 * torch.randn(y.shape, generator=g, device="cuda")).to(torch.float16)
+    for causal in (True, False):
+        out = []
+        for s, t, m in ((x, y, mask), (x[:, :, keep].contiguous(), y[:, :, keep].contiguous(), None)):
+            s = s.clone().requires_grad_(True)
+            loss = attn_kl_align(s, s, t, t, attn_mask=m, causal=causal, sm_scale_s=0.02, sm_scale_t=0.02)
+            out.append((float(loss.detach()), *torch.autograd.grad(loss, [s])))
+        case = f"window-256-c{int(causal)}"
+        check_loss(out[0][0], out[1][0], case)
+        check_grad(out[0][1][:, :, keep].float().cpu().numpy(), out[1][1].float().cpu().numpy(), case)
+        assert float(out[0][1][:, :, ~mask[0]].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("ds,dt", [(8, 8), (8, 64), (64, 8)])
+def test_an_infinite_key_element_does_not_reach_the_padding(gpu_available, dtype, ds, dt):
+    """D = 8 runs in tiles of 16 dims: an infinite key element against queries
+    of the other sign scores -inf (its weight is 0 in the LSE, and the KL with a
+    student's is +inf), not NaN from the padding's zeros."""
+    from linearard_amd.attention_KL import kl_forward, lse_stats
+
+    rng = np.random.default_rng(ds + dt)
+    B, H, T, key = 1, 2, 70, 40
+    x = [randn(rng, (B, H, T, d), dtype) for d in (ds, ds, dt, dt)]
+    m = np.ones((B, T), np.int32)
+    m[:, key] = 0  # the oracle: without that key (and its row)
+    rows = np.arange(T) != key
+    for side, d in ((0, ds), (1, dt)):
+        q, k = x[2 * side].copy(), x[2 * side + 1].copy()
+        q[..., 0] = -1.0
+        ref = O.lse_stats(q, k, m, False, 0.3)
+        k[:, :, key, 0] = np.inf
+        got = lse_stats(to_dev(q, dtype), to_dev(k, dtype), None, False, 0.3).cpu().numpy()
+        np.testing.assert_allclose(got[:, :, rows], ref[:, :, rows], rtol=1e-6, atol=1e-5)
+        if side == 0:
+            y = [to_dev(v, dtype) for v in (q, k, x[2], x[3])]
+            ls, lt = (lse_stats(y[2 * i], y[2 * i + 1], None, False, 0.3) for i in (0, 1))
+            assert float(kl_forward(y[0], y[1], ls, y[2], y[3], lt, None, False, 0.3, 0.3)) == math.inf
