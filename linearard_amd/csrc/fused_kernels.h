@@ -84,8 +84,6 @@ __global__ __launch_bounds__(kStageThreads, 2) void fused_fwd_kernel(const Fused
   StageCopier<DPT> cpt;
   cps.init(ks_base, a.s.k_st, a.s.dim, w, lane);
   cpt.init(kt_base, a.t.k_st, a.t.dim, w, lane);
-  StageCopier<DPS>::clear_padding(lks[0], kBufs, a.s.dim);
-  StageCopier<DPT>::clear_padding(lkt[0], kBufs, a.t.dim);
   constexpr bool kUniform = StageCopier<DPS>::TC::kUniform && StageCopier<DPT>::TC::kUniform;
   constexpr int kPerWave = StageCopier<DPS>::TC::kRowPerWave + StageCopier<DPT>::TC::kRowPerWave;
   auto issue_tile = [&](int kb, int buf) {

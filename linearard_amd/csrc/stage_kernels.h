@@ -87,8 +87,10 @@ __device__ __forceinline__ void stage_item(int& blk, int& head, int causal, int 
 // swizzled tile.  Addresses are 64-bit per lane: these kernels also serve
 // heads of 2^31 bytes and more.  Rows >= T copy row T - 1 (their contributions
 // are masked).  Chunks >= dim (the second one of D = 8; the other dims fill
-// their tiles) are not copied: clear_padding sets them to zero once, so that
-// they add nothing also where a row holds infinities.
+// their tiles) copy zeros, so that they add nothing also where a row holds
+// infinities.
+__device__ __attribute__((aligned(16))) const u16 kZeroChunk[8] = {};
+
 template <int DP>
 struct StageCopier {
   using TC = TileCopies<DP, kStageWaves, kStageTile>;
@@ -100,7 +102,8 @@ struct StageCopier {
   int64_t lane_row;    // this lane's row of the wave's first copy, elements
   int r0;
   unsigned c[NITER];   // this lane's chunk of each copy, bytes
-  bool padding;        // DP = 16: this lane's chunk is one
+  const u16* lane_src; // DP = 16 (one copy per tile): this lane's chunk of row r0, or zeros,
+  int64_t lane_stride; // and the elements to its next row
 
   __device__ __forceinline__ void init(const u16* head, int64_t row_stride, int dim, int wave, int lane) {
     src = head;
@@ -110,19 +113,19 @@ struct StageCopier {
 #pragma unroll
     for (int i = 0; i < NITER; ++i) {
       const int ch = ((64 * wave + lane) % CPR) ^ swz<DP>(r0 + i * RPI);
-      c[i] = 16u * ch;
-      padding = DP == 16 && ch * 8 >= dim;  // one copy per tile there
-    }
-  }
-  // tiles: `bufs` tiles; a barrier must follow before they are read.
-  __device__ __forceinline__ static void clear_padding(u16* tiles, int bufs, int dim) {
-    if constexpr (DP == 16) {
-      for (int i = (int)threadIdx.x; i < bufs * kStageTile * CPR; i += kStageThreads)
-        if (((i % CPR) ^ swz<DP>(i / CPR)) * 8 >= dim) *reinterpret_cast<u16x8*>(tiles + 8 * i) = (u16x8)(0);
+      c[i] = ch * 8 < dim ? 16u * ch : 0u;
+      if constexpr (DP == 16) {
+        lane_src = ch * 8 < dim ? head + lane_row + 8 * ch : kZeroChunk;
+        lane_stride = ch * 8 < dim ? row_stride : 0;
+      }
     }
   }
   __device__ __forceinline__ void issue(unsigned tile, int row0, int T, int wave) const {
     const bool full = row0 + kStageTile <= T;
+    if constexpr (DP == 16) {
+      if (wave == 0) lds_async16_at(lane_src + (row0 + min(0, T - 1 - (row0 + r0))) * lane_stride, tile);
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < NITER; ++i) {
       const int n = wave + kStageWaves * i;
@@ -132,11 +135,7 @@ struct StageCopier {
         const int over = row0 + i * RPI + r0 - (T - 1);
         if (over > 0) p -= (int64_t)over * stride;
       }
-      if constexpr (DP == 16) {
-        if (!padding) lds_async16_at(reinterpret_cast<const char*>(p) + c[i], tile + 1024u * n);
-      } else {
-        lds_async16_at(reinterpret_cast<const char*>(p) + c[i], tile + 1024u * n);
-      }
+      lds_async16_at(reinterpret_cast<const char*>(p) + c[i], tile + 1024u * n);
     }
   }
 };
@@ -351,11 +350,7 @@ __global__ __launch_bounds__(kStageThreads, stage_waves(DPS, DPT, DT, MODE == MO
   StageCopier<DPS> cps;
   StageCopier<HAS_T ? DPT : 16> cpt;
   cps.init(ks_base, a.s.k_st, a.s.dim, w, lane);
-  StageCopier<DPS>::clear_padding(lks[0], kBufs, a.s.dim);
-  if constexpr (HAS_T) {
-    cpt.init(kt_base, a.t.k_st, a.t.dim, w, lane);
-    StageCopier<DPT>::clear_padding(lkt[0], kBufs, a.t.dim);
-  }
+  if constexpr (HAS_T) cpt.init(kt_base, a.t.k_st, a.t.dim, w, lane);
   constexpr bool kUniform = StageCopier<DPS>::TC::kUniform && (!HAS_T || StageCopier<HAS_T ? DPT : 16>::TC::kUniform);
   constexpr int kPerWave =
       StageCopier<DPS>::TC::kRowPerWave + (HAS_T ? StageCopier<HAS_T ? DPT : 16>::TC::kRowPerWave : 0);
@@ -561,9 +556,6 @@ __global__ __launch_bounds__(kStageThreads, stage_waves(DPS, DPT, DT, true)) voi
   int loaded_ht = -1;
   const unsigned gs = row_chunk_xor<DPS>(l32, half), gt = row_chunk_xor<DPT>(l32, half);
   const TokenBits tok = {lbits, &a, (int64_t)b * a.mask_sb};
-
-  StageCopier<DPS>::clear_padding(lqs[0], kBufs, a.s.dim);
-  StageCopier<DPT>::clear_padding(lqt[0], kBufs, a.t.dim);
 
   const int hh_end = min((part_h + 1) * heads, a.s.group);
   for (int hh = part_h * heads; hh < hh_end; ++hh) {
