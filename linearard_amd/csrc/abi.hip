@@ -410,8 +410,9 @@ void set_dk_cut(lard::RelArgs& a, float* part, int64_t rows) {
   if (part == nullptr) return;
   const DkCut c = dk_cut(a.B, a.Hq, a.s.hkv, a.T, rows);
   a.dk_part = part;
-  a.dk_heads = c.heads;
-  a.dk_split = c.split;
+  a.dk_count = c.parts;
+  a.dk_heads = (lard::u16)c.heads;
+  a.dk_split = (lard::u16)c.split;
 }
 
 BwdWs bwd_layout(void* base, int64_t B, int64_t Hq, int64_t T, size_t* bytes, int64_t part_floats = 0) {

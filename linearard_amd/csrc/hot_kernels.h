@@ -786,7 +786,6 @@ __device__ __forceinline__ void hot_bwd_body(const HotArgs& f, int item) {
   const int bg = bgp / parts;
   const int part = bgp - bg * parts;
   const int part_h = part / split, part_s = part - part_h * split;
-  const int heads = a.dk_part != nullptr ? a.dk_heads : a.s.group;
   const int b = bg / a.s.hkv;
   const int g = bg - b * a.s.hkv;
   const int j0w = cb * kRows + w * 32;
@@ -832,9 +831,10 @@ __device__ __forceinline__ void hot_bwd_body(const HotArgs& f, int item) {
   tro.init(lane);
   int loaded_ht = -1;
 
-  const int hh_end = min((part_h + 1) * heads, a.s.group);
-  for (int hh = part_h * heads; hh < hh_end; ++hh) {
-    const int h = g * a.s.group + hh;
+  // this part's heads, or the group's (part_h is 0 then)
+  const int h_end = a.dk_part != nullptr ? min(g * a.s.group + (part_h + 1) * a.dk_heads, (g + 1) * a.s.group)
+                                         : (g + 1) * a.s.group;
+  for (int h = g * a.s.group + part_h * a.dk_heads; h < h_end; ++h) {
     const int ht = h / a.t.group;
     if (ht != loaded_ht) {
       const u16* p = a.t.k + (int64_t)b * a.t.k_sb + (int64_t)ht * a.t.k_sh + (int64_t)my_j * a.t.k_st;

@@ -75,11 +75,12 @@ struct RelArgs {
   // block's sum over its group's heads and query tiles is cut into parts, one
   // workgroup each, of dk_heads heads (the last of a group fewer) over one of
   // dk_split ranges of query tiles.  A part goes, scaled by scale_s only, to
-  // dk_part [B * Hkv_s][dk_parts][T, Ds]; the finish kernel adds them up (null:
+  // dk_part [B * Hkv_s][dk_count][T, Ds]; the finish kernel adds them up (null:
   // one workgroup sums everything into dk_out).
   float* dk_part;
-  int dk_heads;
-  int dk_split;
+  int dk_count;
+  u16 dk_heads;  // at most 32768: half of the largest group
+  u16 dk_split;
   // Throughput kernels: dk rounded to the input type here instead of dk_out
   // (null: float32 to dk_out).
   u16* dk16;

@@ -241,9 +241,7 @@ __device__ __forceinline__ void stage_grad(const TrXor<DP>& tr, unsigned tile, c
 }
 
 // Parts of a key block's dk sum (RelArgs::dk_part).
-__host__ __device__ inline int dk_parts(const RelArgs& a) {
-  return a.dk_part != nullptr ? (a.s.group + a.dk_heads - 1) / a.dk_heads * a.dk_split : 1;
-}
+__host__ __device__ inline int dk_parts(const RelArgs& a) { return a.dk_part != nullptr ? a.dk_count : 1; }
 
 // 256-wide gradients: the accumulators (128 registers) stay in AGPRs around the
 // loop.  Left alone, the compiler keeps them in VGPRs between tiles and copies
@@ -517,7 +515,6 @@ __global__ __launch_bounds__(kStageThreads, stage_waves(DPS, DPT, DT, true)) voi
   const int bg = bgp / parts;
   const int part = bgp - bg * parts;
   const int part_h = part / split, part_s = part - part_h * split;
-  const int heads = a.dk_part != nullptr ? a.dk_heads : a.s.group;
   const int b = bg / a.s.hkv;
   const int g = bg - b * a.s.hkv;
   const int j0w = cb * kStageRows + w * 32;
@@ -557,9 +554,10 @@ __global__ __launch_bounds__(kStageThreads, stage_waves(DPS, DPT, DT, true)) voi
   const unsigned gs = row_chunk_xor<DPS>(l32, half), gt = row_chunk_xor<DPT>(l32, half);
   const TokenBits tok = {lbits, &a, (int64_t)b * a.mask_sb};
 
-  const int hh_end = min((part_h + 1) * heads, a.s.group);
-  for (int hh = part_h * heads; hh < hh_end; ++hh) {
-    const int h = g * a.s.group + hh;
+  // this part's heads, or the group's (part_h is 0 then)
+  const int h_end = a.dk_part != nullptr ? min(g * a.s.group + (part_h + 1) * a.dk_heads, (g + 1) * a.s.group)
+                                         : (g + 1) * a.s.group;
+  for (int h = g * a.s.group + part_h * a.dk_heads; h < h_end; ++h) {
     const int ht = h / a.t.group;
     if (ht != loaded_ht) {
       const u16* p = a.t.k + (int64_t)b * a.t.k_sb + (int64_t)ht * a.t.k_sh + (int64_t)my_j * a.t.k_st;
