@@ -9,7 +9,7 @@ divides by the number of layers (train.py:410).  That is 3 L calls and
 
 ``attn_kl_align_batched(xs, xt, weights)`` computes
 ``sum_r weights[r] * attn_kl_align(xs[r], xs[r], xt[r], xt[r])`` with one
-launch per 8 relations (``lard_attn_kl_batched_forward`` / ``_backward``):
+launch per 8 relations (``lard_attn_kl_batched_forward``):
 the relations' row blocks share one grid even when their head counts differ
 (Q/Q 32 heads next to K/K 8).  When the students need gradients the forward
 is ``lard_attn_kl_batched_forward_rowgrad``, which also leaves the row side
@@ -102,12 +102,13 @@ class AttnKLBatchedFn(torch.autograd.Function):
         ctx.n = n
         ctx.causal = bool(causal)
         ctx.ss, ctx.st = ss, st
-        ctx.batched = batched
         return loss
 
     @staticmethod
     def backward(ctx, dloss):
         n = ctx.n
+        if not any(ctx.needs_input_grad[6:6 + n]):  # weights or teachers alone: no gradient
+            return (None,) * (6 + 2 * n)
         saved = ctx.saved_tensors
         weights, attn_mask, lse = saved[:3]
         xs, xt = saved[3:3 + n], saved[3 + n:3 + 2 * n]
@@ -129,27 +130,19 @@ class AttnKLBatchedFn(torch.autograd.Function):
                                                            ws.data_ptr(), ws_bytes, stream)
             _lib.check(rc, "lard_attn_kl_batched_backward_colgrad16")
             return (None, None, None, None, None, None, *dxs, *([None] * n))
+        # relation by relation, as the forward
         dxs = [torch.empty(x.shape, device=dev, dtype=torch.float32) for x in xs]
-        if ctx.batched:
-            rels = _lib.relations(xs, xt, lse_s, lse_t, [x.data_ptr() for x in dxs])
-            ws_bytes = L.lard_attn_kl_batched_workspace_bytes(rels, n)
+        scaled = (dloss * weights).contiguous()  # dloss * w_r, one device scalar per relation
+        for r in range(n):
+            B_, H_, T_, D_ = xs[r].shape
+            ws_bytes = L.lard_attn_kl_backward_workspace_bytes(B_, H_, H_, T_, D_, 1)
             ws = _workspace(ws_bytes, dev)
-            rc = L.lard_attn_kl_batched_backward(rels, n, ctypes.byref(md), int(ctx.causal), ctx.ss[0], ctx.st[0],
-                                                 weights.data_ptr(), dloss.data_ptr(), ws.data_ptr(), ws_bytes,
-                                                 stream)
-            _lib.check(rc, "lard_attn_kl_batched_backward")
-        else:
-            scaled = (dloss * weights).contiguous()  # dloss * w_r, one device scalar per relation
-            for r in range(n):
-                B_, H_, T_, D_ = xs[r].shape
-                ws_bytes = L.lard_attn_kl_backward_workspace_bytes(B_, H_, H_, T_, D_, 1)
-                ws = _workspace(ws_bytes, dev)
-                d = [_lib.tensor4(x) for x in (xs[r], xt[r])]
-                rc = L.lard_attn_kl_backward(
-                    ctypes.byref(d[0]), ctypes.byref(d[0]), lse_s[r], ctypes.byref(d[1]),
-                    ctypes.byref(d[1]), lse_t[r], ctypes.byref(md), int(ctx.causal), ctx.ss[r], ctx.st[r],
-                    scaled[r:r + 1].data_ptr(), 1, None, dxs[r].data_ptr(), ws.data_ptr(), ws_bytes, stream)
-                _lib.check(rc, "lard_attn_kl_backward")
+            d = [_lib.tensor4(x) for x in (xs[r], xt[r])]
+            rc = L.lard_attn_kl_backward(
+                ctypes.byref(d[0]), ctypes.byref(d[0]), lse_s[r], ctypes.byref(d[1]),
+                ctypes.byref(d[1]), lse_t[r], ctypes.byref(md), int(ctx.causal), ctx.ss[r], ctx.st[r],
+                scaled[r:r + 1].data_ptr(), 1, None, dxs[r].data_ptr(), ws.data_ptr(), ws_bytes, stream)
+            _lib.check(rc, "lard_attn_kl_backward")
         return (None, None, None, None, None, None, *dxs, *([None] * n))
 
 

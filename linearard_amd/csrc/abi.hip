@@ -251,6 +251,8 @@ struct LossWs {
   unsigned* counter;  // ticket of the reduction
 };
 
+// Partials in the workspaces' layout; the reduction uses kReduceBlocks of them
+// (the sizes that *_workspace_bytes return are the interface's and stay).
 constexpr int kLossPartials = 512;
 
 LossWs loss_layout(void* base, int64_t n, size_t* bytes) {
@@ -1280,8 +1282,6 @@ int backward_colgrad_impl(const lard_tensor4* qs, const lard_tensor4* ks, const 
   if ((rc = hip_status(lard::launch_row_prep(rp, (int)B, st), "attn_kl_backward_colgrad row prep launch")) != LARD_OK)
     return rc;
   f.Tp = Tp;
-  f.tok_ok = w.tok_ok;
-  f.first2 = w.first2;
   f.nl_s = w.nl_s;
   f.nl_t = w.nl_t;
   f.r.dk_out = dk_out;
@@ -1578,7 +1578,7 @@ int batched_colgrad_impl(const lard_relation* rels, int nrel, const lard_mask* m
   int64_t nl_off = 0;
   for (int r = 0; r < nrel; ++r) {
     lard::HotArgs& f = fs[(size_t)r];
-    f = relation_args(rels[r], mask, causal, sm_scale_s, sm_scale_t, Tp, w.tok_ok, w.first2);
+    f = relation_args(rels[r], mask, causal, sm_scale_s, sm_scale_t, Tp, nullptr, nullptr);
     f.r.lse_s_in = rels[r].lse_s;
     f.r.lse_t_in = rels[r].lse_t;
     float* nl_s = w.nl_s + nl_off;

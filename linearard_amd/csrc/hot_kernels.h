@@ -47,7 +47,7 @@ constexpr int kRows = kWaves * 32;
 struct HotArgs {
   RelArgs r;
   int Tp;                        // T rounded up to kTile
-  const unsigned char* tok_ok;   // [B][Tp] token validity
+  const unsigned char* tok_ok;   // [B][Tp] token validity (null with first2 in a backward of the column side alone)
   const int* first2;             // [B][2] first and second valid token of each sequence (T if none)
   const float* nl_s;             // backward: [B*Hq][Tp] -lse_s*log2(e), -inf for excluded rows
   const float* nl_t;

@@ -183,43 +183,4 @@ __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_lo
 
 __device__ __forceinline__ float xor32(float v) { return __shfl_xor(v, 32, 64); }
 
-// Rows [row0, row0+NROWS) x [0, DP) of a [T, D]-strided 16-bit matrix,
-// staged into LDS (row stride lds_stride elements) through registers in two
-// steps, so that one tile's global loads are in flight while the previous
-// tile is consumed: load() issues the loads (a chunk outside the matrix --
-// row >= T or column >= dim -- loads row 0, column 0 instead, which exists
-// whenever T > 0, and is remembered as invalid), store() writes the
-// registers to LDS later, zeros for the invalid chunks, so the MFMA sees
-// exact zero padding.
-template <int NROWS, int DP, int NTHREADS>
-struct TileRegs {
-  static constexpr int CPR = DP / 8;  // 16-byte chunks per row
-  static constexpr int NCH = NROWS * CPR;
-  static constexpr int N = (NCH + NTHREADS - 1) / NTHREADS;
-  u16x8 v[N];
-  bool ok[N];
-
-  __device__ __forceinline__ void load(const u16* g, int64_t row_stride, int row0, int T, int dim, int tid) {
-#pragma unroll
-    for (int n = 0; n < N; ++n) {
-      const int c = tid + n * NTHREADS;
-      if (NCH % NTHREADS == 0 || c < NCH) {
-        const int row = row0 + c / CPR;
-        const int dc = (c % CPR) * 8;
-        ok[n] = row < T && dc < dim;
-        v[n] = *reinterpret_cast<const u16x8*>(g + (ok[n] ? (int64_t)row * row_stride + dc : 0));
-      }
-    }
-  }
-
-  __device__ __forceinline__ void store(u16* lds, int lds_stride, int tid) const {
-#pragma unroll
-    for (int n = 0; n < N; ++n) {
-      const int c = tid + n * NTHREADS;
-      if (NCH % NTHREADS == 0 || c < NCH)
-        *reinterpret_cast<u16x8*>(lds + (c / CPR) * lds_stride + (c % CPR) * 8) = ok[n] ? v[n] : (u16x8)(0);
-    }
-  }
-};
-
 }  // namespace lard

@@ -179,3 +179,27 @@ def test_batched_takes_the_hooks_strided_views(gpu_available):
     assert l1.item() == l2.item()
     for a, b in zip(views, copies):
         assert torch.equal(a.grad, b.grad)
+
+
+@pytest.mark.parametrize("which", ["weights", "teachers"])
+@pytest.mark.parametrize("D", [64, 256])
+def test_no_gradient_to_weights_or_teachers(gpu_available, which, D):
+    """Weights or teachers that ask for a gradient get none, alone or beside the
+    students' (which is the same), on the batched and the per-relation path."""
+    from linearard_amd.attention_KL import attn_kl_align_batched
+
+    rng = np.random.default_rng(D)
+    xs = [to_dev(randn(rng, (1, h, 65, D), "bf16"), "bf16") for h in (2, 1)]
+    xt = [to_dev(randn(rng, (1, h, 65, D), "bf16"), "bf16") for h in (2, 1)]
+    w = torch.tensor([0.5, 2.0], device="cuda")
+    asked = [w] if which == "weights" else xt
+    for x in xs:
+        x.requires_grad_(True)
+    ref = torch.autograd.grad(attn_kl_align_batched(xs, xt, w), xs)
+    for x in asked:
+        x.requires_grad_(True)
+    loss = attn_kl_align_batched(xs, xt, w)
+    got = torch.autograd.grad(loss, [*xs, *asked], allow_unused=True)
+    assert all(torch.equal(a, b) for a, b in zip(got, ref)) and all(g is None for g in got[2:])
+    loss = attn_kl_align_batched([x.detach() for x in xs], xt, w)
+    assert all(g is None for g in torch.autograd.grad(loss, asked, allow_unused=True))
