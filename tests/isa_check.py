@@ -95,7 +95,7 @@ def kernels(asm: str) -> dict:
             out[cur].append(("label", lm.group(1)))
         elif not t.startswith("."):
             out[cur].append(("inst", t))
-    return out
+    return {name: body for name, body in out.items() if body}  # a constant's label has none
 
 
 def _regs(tok: str):
