@@ -65,7 +65,7 @@ def _warn_slow_path(d, ss: float, st: float) -> str:
     if name != "throughput" and why not in _WARNED:
         _WARNED.add(why)
         warnings.warn(f"attn_kl_align: {why}: these inputs run the {name} kernels, not the throughput "
-                      f"kernels (several times slower)", RuntimeWarning, stacklevel=3)
+                      f"kernels (slower)", RuntimeWarning, stacklevel=3)
     return name
 
 

@@ -39,9 +39,10 @@
 // Bound by the double units: a 16x16x4 product takes 64 cycles of a SIMD (77
 // TFLOP/s in a loop of nothing else), and the double VALU work (a score's
 // exponentials, the conversions of the operands) adds to it rather than
-// overlapping.  At B=1, H=32, n=1024, d=128, causal, a fwd+bwd takes 821 us
-// (forward 238, dq 301, dk 330; the LSE refine of a backward without the
-// forward's double LSEs 235 more) against 4630 us with VALU FMAs (two
+// overlapping.  At B=1, H=32, n=1024, d=128, causal, a fwd+bwd takes 825 us
+// in a loop of calls (single launches at a colder clock: forward 238, dq 302,
+// dk 333; the LSE refine of a backward without the forward's double LSEs about
+// the forward's time more) against 4630 us with VALU FMAs (two
 // conversions and 1.25 LDS reads per four of them) and a refine pass.
 
 #include "stage_f32.h"
@@ -145,7 +146,7 @@ constexpr double kNegInfD = -__builtin_inf();
 // Taylor series to r^5 (the first dropped term, r^6 / 720, is below 4e-17).
 // Underflows to 0, overflows to inf, NaN stays NaN.  Double VALU work does not
 // overlap the double matrix products here (they take the sum of their times),
-// so its length counts: 12 double instructions against 25 for the series over
+// so its length counts: 12 double instructions (ABOVE: 13) against 25 for the series over
 // |r| <= ln(2) / 2 and more for the library's exp.
 // ABOVE: x may lie above 0, as a score against a given LSE may (against a
 // running maximum it does not).  n is then held at 2^20, where the result is
