@@ -130,6 +130,8 @@ class AttnKLAlignFn(torch.autograd.Function):
     def backward(ctx, dloss):
         """integration.py:48-67: stage C and the chain rule with dloss."""
         qs, ks, qt, kt, lse, attn_mask, extra = ctx.saved_tensors
+        if ctx.self_relation:  # saved-tensor hooks hand out a tensor for each
+            ks = qs
         dloss = _lib.loss_grad(dloss)
         B, Hq, T, Ds = qs.shape
         Hkv = ks.shape[1]

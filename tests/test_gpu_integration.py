@@ -443,6 +443,26 @@ def test_keys_beyond_the_float16_range_take_a_scale(gpu_available, self_rel):
         check_grad(tks.grad.float().cpu().numpy(), rdk, cid, "dk")
 
 
+@pytest.mark.parametrize("dtype,D", [("bf16", 64), ("bf16", 256), ("f32", 64)])
+@pytest.mark.parametrize("self_rel", [True, False])
+def test_saved_tensor_hooks(gpu_available, dtype, D, self_rel):
+    """save_on_cpu between forward and backward (every saved tensor comes back
+    as a tensor of its own, also a self relation's query and key): the same
+    gradients."""
+    from linearard_amd.attention_KL import attn_kl_align
+
+    rng = np.random.default_rng(D)
+    x, k, y, z = (to_dev(randn(rng, (1, 2, 130, D), dtype), dtype) for _ in range(4))
+    x.requires_grad_(True)
+    k, z = (x, y) if self_rel else (k.requires_grad_(True), z)
+    wrt = [x] if self_rel else [x, k]
+    ref = torch.autograd.grad(attn_kl_align(x, k, y, z), wrt)
+    with torch.autograd.graph.save_on_cpu():
+        loss = attn_kl_align(x, k, y, z)
+    got = torch.autograd.grad(loss, wrt)
+    assert all(torch.equal(a, b) for a, b in zip(got, ref))
+
+
 @pytest.mark.parametrize("side", ["student", "teacher"])
 def test_large_queries_whose_keys_are_their_first_heads(gpu_available, side):
     """bf16, ks = qs[:, :2]: the keys share the queries' address, and the only
